@@ -40,7 +40,6 @@ using namespace sbdg;
 
 namespace {
 constexpr int MAXSUB = 48;
-constexpr size_t LDS_BUDGET = 160 * 1024;  // alpha-beta kernel: all of a CU's LDS, one 1024-thread workgroup
 
 // Scratch of sbdg_sigma_device, the sigma entry point that allocates nothing: one array
 // per device, held from the library's load until the process ends.  On the host the
@@ -92,7 +91,7 @@ struct sbdg_ctx {
   std::vector<uint64_t> a, b;
   std::vector<double> user_vec;
   DBuf<double> d_h1, d_eri, d_hii;
-  DBuf<float> d_eri32, d_hii32;
+  DBuf<float> d_hii32;
   DBuf<uint64_t> d_a, d_b;
   Table Sa, Da, Sb, Db;
   SpmmTable Ma, Mb;
@@ -101,6 +100,8 @@ struct sbdg_ctx {
   bool use_ca = false, use_cb = false;
   DBuf<double> Ja, Jb;    // occupation tables of the alpha / beta strings
   DBuf<float> Ja32, Jb32;
+  DBuf<double> Vt;        // alpha-beta integral slices by orbital pair
+  DBuf<float> Vt32;
   DBuf<double> Wp;        // antisymmetrised pair integrals
   DBuf<float> Wp32;
   DBuf<double> Zbuf;      // core-product workspace
@@ -108,6 +109,7 @@ struct sbdg_ctx {
   EllTable ell;      // beta singles, ELL (alpha-beta sigma, FP64; FP32 too when the geometries agree)
   EllTable ell32;    // the FP32 ELL when its launch geometry differs (wide rows)
   bool own_ell32 = false;
+  AbSegments seg;    // bra-row segments of the alpha-beta kernel
   // solver state
   DBuf<double> V, HV, W, R, T, HX, scr64, small;
   DBuf<float> HV32, c32, s32, scr32;
@@ -147,14 +149,6 @@ double now() {
   return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
 
-// column chunk of the alpha-beta kernel: ket-row chunks and the integral slices of 16-byte
-// row vectors (2 FP64 or 4 FP32 rows) in LDS
-int64_t choose_chunk(int64_t nb, int L) {
-  const int64_t budget = (int64_t)(LDS_BUDGET / 16) - ab_slice_span(L) - 1;
-  int64_t ch = std::max<int64_t>(256, budget);
-  return std::min<int64_t>(std::max<int64_t>(nb, 1), ch);
-}
-
 SigmaPlan plan(sbdg_ctx* c, bool fp32) {
   SigmaPlan P;
   P.na = (int64_t)c->a.size();
@@ -166,8 +160,9 @@ SigmaPlan plan(sbdg_ctx* c, bool fp32) {
   P.mb = &c->Mb;
   P.sa = &c->Sa;
   P.ell = (fp32 && c->own_ell32) ? &c->ell32 : &c->ell;
-  P.eri = c->d_eri.p;
-  P.eri32 = c->d_eri32.p;
+  P.seg = &c->seg;
+  P.Vt = c->Vt.p;
+  P.Vt32 = c->Vt32.p;
   P.hii = c->d_hii.p;
   P.hii32 = c->d_hii32.p;
   P.Ja = c->Ja.p;
@@ -196,10 +191,8 @@ void build(sbdg_ctx* c) {
   const int64_t L4 = (int64_t)L * L * L * L;
   c->d_h1.alloc(L * L);
   c->d_eri.alloc(L4);
-  c->d_eri32.alloc(L4);
   SBDG_CHECK(hipMemcpyAsync(c->d_h1.p, c->h1.data(), sizeof(double) * L * L, hipMemcpyHostToDevice, c->st));
   SBDG_CHECK(hipMemcpyAsync(c->d_eri.p, c->eri.data(), sizeof(double) * L4, hipMemcpyHostToDevice, c->st));
-  cast_d2f(c->d_eri.p, c->d_eri32.p, L4, c->st);
   c->d_a.alloc(std::max<int64_t>(na, 1));
   c->d_b.alloc(std::max<int64_t>(nb, 1));
   SBDG_CHECK(hipMemcpyAsync(c->d_a.p, c->a.data(), sizeof(uint64_t) * na, hipMemcpyHostToDevice, c->st));
@@ -252,16 +245,21 @@ void build(sbdg_ctx* c) {
   } else {
     c->Zbuf.free();
   }
-  build_ab(c->Sb, L, rdm_chunk(nb, L), c->ab64, c->st);
-  build_ell(c->Sb, L, choose_chunk(nb, L), 8, c->ell, c->st);
   {
-    int nt64, m64, nt32, m32;
-    ab_geometry(nb, 8, nt64, m64);
-    ab_geometry(nb, 4, nt32, m32);
-    c->own_ell32 = nt64 != nt32 || m64 != m32;
-    if (c->own_ell32) build_ell(c->Sb, L, choose_chunk(nb, L), 4, c->ell32, c->st);
+    const size_t npair = (size_t)L * (L - 1) / 2;
+    c->Vt.alloc(std::max<size_t>(npair * npair, 1));
+    c->Vt32.alloc(std::max<size_t>(npair * npair, 1));
+    build_pair_slices(c->d_eri.p, L, c->Vt.p, c->Vt32.p, c->st);
+  }
+  build_ab(c->Sb, L, rdm_chunk(nb, L), c->ab64, c->st);
+  build_ell(c->Sb, L, 8, c->ell, c->st);
+  {
+    const AbGeometry g64 = ab_geometry(nb, L, 8), g32 = ab_geometry(nb, L, 4);
+    c->own_ell32 = g64.nt != g32.nt || g64.m != g32.m || g64.s != g32.s || g64.chunk != g32.chunk;
+    if (c->own_ell32) build_ell(c->Sb, L, 4, c->ell32, c->st);
     else c->ell32.release();
   }
+  build_segments(c->Sa, nb, c->ell.ntiles, c->seg, c->st);
   c->d_hii.alloc(std::max<int64_t>(N, 1));
   c->d_hii32.alloc(std::max<int64_t>(N, 1));
   compute_hii(c->d_a.p, na, c->d_b.p, nb, L, c->core, c->d_h1.p, c->d_eri.p, c->d_hii.p, c->st);
@@ -327,7 +325,8 @@ int64_t davidson_bytes(const sbdg_options& o, int64_t N) {
 int64_t build_bytes(const sbdg_options& o, int L, int64_t na, int64_t nb, const int64_t* nnz, const int64_t* mem,
                     const int64_t* dir) {
   const int64_t L2 = (int64_t)L * L, L4 = L2 * L2, N = na * nb, npair = (int64_t)L * (L - 1) / 2;
-  int64_t b = 8 * L2 + 12 * L4 + 8 * (na + nb) + 12 * N;  // h1, eri FP64+FP32, strings, hii FP64+FP32
+  int64_t b = 8 * L2 + 8 * L4 + 8 * (na + nb) + 12 * N;  // h1, eri, strings, hii FP64+FP32
+  b += 12 * std::max<int64_t>(npair * npair, 1);           // alpha-beta slices
   bool any_core = false;
   int64_t zwant = 0;
   const int64_t ns[2] = {na, nb}, nc[2] = {nb, na};
@@ -349,13 +348,16 @@ int64_t build_bytes(const sbdg_options& o, int L, int64_t na, int64_t nb, const 
   const int64_t Sb = nnz[2];
   const int64_t ach = rdm_chunk(nb, L);
   b += 4 * Sb + 4 * (nb * ((nb + ach - 1) / ach + 1) + 1);
-  const int64_t nch = (nb + choose_chunk(nb, L) - 1) / choose_chunk(nb, L);
-  const int64_t groups = (nb + 63) / 64 + 1024;  // tiles round the lane positions up
-  int nt64, m64, nt32, m32;
-  ab_geometry(nb, 8, nt64, m64);
-  ab_geometry(nb, 4, nt32, m32);
-  const int nell = (nt64 != nt32 || m64 != m32) ? 2 : 1;  // an FP32 ELL of its own (wide rows)
-  b += nell * (4 * (64 * Sb + 192 * groups * nch) + 4 * nch * groups * 64 + 16 * groups * nch);
+  const AbGeometry g64 = ab_geometry(nb, L, 8), g32 = ab_geometry(nb, L, 4);
+  const bool two = g64.nt != g32.nt || g64.m != g32.m || g64.s != g32.s || g64.chunk != g32.chunk;
+  for (const AbGeometry& g : {g64, g32}) {
+    const int64_t nch = std::max<int64_t>(1, (nb + g.chunk - 1) / g.chunk);
+    const int64_t tw = (int64_t)g.nt * g.m, groups = (nb + tw - 1) / tw * (tw / 64);
+    b += 4 * (64 * Sb + 64 * AB_BATCH * groups * nch) + 4 * nch * groups * 64 + 16 * groups * nch;
+    if (!two) break;  // one table for both precisions
+  }
+  // bra-row segments: at most every single its own, and their partial rows
+  b += 16 * (na + nnz[0]) + std::min<int64_t>(AB_PART_BYTES, 8 * nnz[0] * nb);
   return b;
 }
 

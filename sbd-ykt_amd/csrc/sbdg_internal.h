@@ -122,7 +122,7 @@ struct AbTable {
 };
 
 // Beta singles in an ELL layout for the alpha-beta sigma kernel.  Columns are cut into
-// tiles of nt*m lane positions (one workgroup each); in ket chunk k, colperm[k*npos + pos]
+// contiguous tiles of nt*m lane positions (one workgroup each); in ket chunk k, colperm[k*npos + pos]
 // is the column at lane position pos (-1: none).  Per chunk, a tile's columns are sorted by
 // their entry count in that chunk and cut into 64-lane groups (lists of similar length);
 // wave w of tile t walks the groups at slots g = t*W*m + w + j*W, j < m (W = nt/64), and
@@ -136,9 +136,10 @@ struct AbTable {
 // the chunk); offset `chunk` is a zero vector: padding), bits 18-29 the slice vector of
 // orbital pair (b, j) (ab_pair(b, j)), bit 31 sign.  Within a lane the entries are ordered
 // so that lanes read distinct LDS slots where possible.
+constexpr int AB_BATCH = 4;  // ELL rows per batch of the alpha-beta kernel
 struct EllTable {
   int nch = 0;
-  int nt = 0, m = 0;        // alpha-beta launch: threads per workgroup, columns per thread
+  int nt = 0, m = 0, s = 1;  // alpha-beta launch: threads per workgroup, columns per thread, groups staged at once
   int64_t chunk = 0, groups = 0, ntiles = 0;
   int64_t kbase = 0;        // first ket vector (16-byte units): after the slice vectors
   DBuf<int64_t> soff;       // ntiles*(nt/64)*nch + 1: start of each wave's entry stream per chunk
@@ -152,6 +153,20 @@ struct EllTable {
     colperm.free();
     nch = nt = m = 0;
   }
+};
+
+// Bra rows of the alpha-beta kernel cut into segments of their alpha singles (longest
+// first): one workgroup per segment and column tile.  A row's first segment writes sigma's
+// row, the others rows of `part`, which k_ab_join adds in order.
+constexpr int64_t AB_PART_BYTES = (int64_t)256 << 20;  // at most this much in partial rows
+struct AbSegments {
+  int64_t nseg = 0, npart = 0, njoin = 0;
+  DBuf<int32_t> row;   // nseg
+  DBuf<int64_t> q;     // 2*nseg: first and past-the-end alpha single
+  DBuf<int32_t> dst;   // nseg: -1 or the row of part
+  DBuf<int32_t> jrow;  // njoin rows with partial rows
+  DBuf<int32_t> jptr;  // njoin + 1
+  DBuf<double> part;   // npart rows of nb
 };
 
 // Double excitations of one spin grouped by their (n-2)-electron core: a double pair
@@ -199,10 +214,19 @@ void build_occ_table(const uint64_t* d_str, int64_t n, int L, const double* d_er
                      hipStream_t st);
 // W[P*npair + Q] (FP64 and FP32), npair = L(L-1)/2
 void build_pair_integrals(const double* d_eri, int L, double* W, float* W32, hipStream_t st);
+// Vt[ab_pair(a,i)*npair + ab_pair(b,j)] = (ai|bj): one alpha single's slice is contiguous
+void build_pair_slices(const double* d_eri, int L, double* Vt, float* Vt32, hipStream_t st);
 void build_ab(const Table& sb, int L, int64_t chunk, AbTable& ab, hipStream_t st);
 // prec_bytes: 8 (FP64) or 4 (FP32) -- the launch geometry depends on the accumulator size
-void build_ell(const Table& sb, int L, int64_t chunk, int prec_bytes, EllTable& e, hipStream_t st);
-void ab_geometry(int64_t nb, int prec_bytes, int& nt, int& m);
+void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t st);
+// Launch geometry of the alpha-beta kernel: threads, columns per thread, ket-row groups staged
+// at once, ket columns per chunk.
+struct AbGeometry {
+  int nt, m, s;
+  int64_t chunk;
+};
+AbGeometry ab_geometry(int64_t nb, int L, int prec_bytes);
+void build_segments(const Table& sa, int64_t nb, int64_t ntiles, AbSegments& g, hipStream_t st);
 void compute_hii(const uint64_t* d_a, int64_t na, const uint64_t* d_b, int64_t nb, int L, double core,
                  const double* d_h1, const double* d_eri, double* d_hii, hipStream_t st);
 
@@ -216,8 +240,9 @@ struct SigmaPlan {
   const SpmmTable* mb = nullptr;  // beta merged
   const Table* sa = nullptr;      // alpha singles (exc, col)
   const EllTable* ell = nullptr;
-  const double* eri = nullptr;
-  const float* eri32 = nullptr;
+  const AbSegments* seg = nullptr;
+  const double* Vt = nullptr;  // (ai|bj) over orbital pairs a > i, b > j (alpha-beta slices)
+  const float* Vt32 = nullptr;
   const double* hii = nullptr;
   const float* hii32 = nullptr;
   const double* Jb = nullptr;  // beta-occupation table (columns of c), alpha singles
@@ -256,7 +281,7 @@ size_t ab_lds_bytes(int64_t kbase, int64_t chunk);
 inline int64_t ab_pairs(int L) {
   return std::max<int64_t>(1, (int64_t)L * (L - 1) / 2);
 }
-inline uint32_t ab_pair(uint32_t b, uint32_t j) {
+__host__ __device__ inline uint32_t ab_pair(uint32_t b, uint32_t j) {
   const uint32_t h = b > j ? b : j, l = b > j ? j : b;
   return h * (h - 1) / 2 + l;
 }

@@ -319,20 +319,17 @@ __global__ void __launch_bounds__(256) k_transpose(int64_t R, int64_t C, const T
   }
 }
 
-// alpha-beta and cross-spin single terms.  One workgroup per (bra row ia, tile of lane
-// positions); thread t owns positions col0 + t + m*blockDim.x, m < M (every wave owns
-// whole 64-lane groups of the ELL table), i.e. columns colperm[position].  The ket rows
-// ja in S(ia) are taken G at a time (G = 2 in FP64, 4 in FP32: 16 bytes either way):
-// the G (ai|..) slices and the G rows' current column chunk sit in LDS interleaved, so one
-// 16-byte LDS read serves all G rows, and every ELL entry read from the L2-resident table
-// serves them too.  LDS: [slice G-vectors of the pairs b > j] [chunk + 1 ket G-vectors
-// from kbase, the last one zero].
+// alpha-beta terms.  The ket rows ja in S(ia) are taken G at a time (G = 2 in FP64, 4 in
+// FP32: 16 bytes either way): the G (ai|..) slices and the G rows' current column chunk sit
+// in LDS interleaved, so one 16-byte LDS read serves all G rows, and every ELL entry read
+// from the L2-resident table serves them too.
 template <class T>
 struct AbRows {
   static constexpr int G = 16 / (int)sizeof(T);
   struct __align__(16) V {
     T v[G];
   };
+  typedef T P2 __attribute__((ext_vector_type(2), aligned(sizeof(T))));
   // x with its sign flipped where bit 31 of sbit is set
   __device__ static inline T flip(T x, uint32_t sbit) {
     if constexpr (sizeof(T) == 8)
@@ -355,159 +352,202 @@ __device__ inline V lds_at(uint32_t a) {
   return r;
 }
 
-// One batch of four stream rows of one lane: s[g] += sign_e * V[pair_e][g] * cb[jb_e][g] for
-// the G staged rows at once (all eight LDS reads issued before the products).
-template <class T>
-__device__ inline void ab_batch(const uint32_t (&p)[4], T (&s)[AbRows<T>::G]) {
+// One batch of stream rows of one lane: s[g] += sign_e * V[pair_e][g] * C[jb_e][g] for the G
+// rows staged at byte offset off (all LDS reads issued before the products; one sum per row:
+// a single chain of dependent FMAs was slower).
+template <class T, int B>
+__device__ inline void ab_batch(const uint32_t (&p)[B], uint32_t off, T (&s)[AbRows<T>::G]) {
   using R = AbRows<T>;
   using RV = typename R::V;
   constexpr int G = R::G;
-  RV v[4], x[4];
+  RV v[B], x[B];
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
-    v[u] = lds_at<RV>((p[u] >> 14) & 0xFFF0u);  // slice vector of pair (b, j)
-    x[u] = lds_at<RV>(p[u] & 0x3FFFFu);         // ket vector
+  for (int u = 0; u < B; ++u) {
+    v[u] = lds_at<RV>(((p[u] >> 14) & 0xFFF0u) + off);  // slice vector of pair (b, j)
+    x[u] = lds_at<RV>((p[u] & 0x3FFFFu) + off);         // ket vector
   }
 #pragma unroll
-  for (int u = 0; u < 4; ++u) {
+  for (int u = 0; u < B; ++u) {
 #pragma unroll
     for (int g = 0; g < G; ++g) s[g] += R::flip(v[u].v[g], p[u]) * x[u].v[g];
   }
 }
 
-// Alpha-beta terms of one bra row ia over one column tile:
-//   sigma[ia, ib] += sum_{ja in S(ia)} sa * sum_{entries (jb, b<-j) of ib} sb (ai|bj) c[ja, jb]
+// A table the kernel never writes, read at wave-uniform indices: through the constant address
+// space, so that the reads are scalar loads.  (As vector loads they share the counter of the
+// entry prefetch, and every group's start waited for the whole of it.)
+template <class I>
+__device__ inline I uniform_at(const I* p, int64_t i) {
+  return reinterpret_cast<const __attribute__((address_space(4))) I*>(reinterpret_cast<uintptr_t>(p))[i];
+}
+
+template <class T>
+struct AbArgs {
+  int64_t nb, ntiles, chunk, kbase, groups;
+  int L, nch, nseg, assign;
+  const int32_t* segrow;  // bra row of each segment
+  const int64_t* segq;    // its alpha singles [segq[2s], segq[2s+1])
+  const int32_t* segdst;  // -1: sigma's row; else the row of part
+  const int32_t* colSa;
+  const uint32_t* excSa;
+  const int64_t* soff;
+  const int32_t* nq;
+  const uint32_t* ent;
+  const int32_t* colperm;
+  const T* Vt;  // (ai|bj) by orbital pairs a > i, b > j
+  const T* c;
+  T* sigma;
+  T* part;
+};
+
+// Alpha-beta terms of one segment of a bra row's alpha singles over one column tile:
+//   out[ib] += sum_{ja in segment} sa * sum_{entries (jb, b<-j) of ib} sb (ai|bj) c[ja, jb]
 // (the other-spin occupation parts of the singles are in the row products).  Chunk by chunk of
-// ket columns: G ket rows of the chunk and their slices sit in LDS as interleaved
-// G-vectors, each lane walks its ELL entries for that chunk (the lane -> column map is per
-// chunk, so lanes of a group carry lists of similar length), and the chunk's sums are
-// added into sigma before the next chunk (one owner per element: a column belongs to one
-// tile; with one tile per row, through LDS in column order).  A wave's entries of a chunk are one stream (its groups one after another, four
-// rows per batch); the next batch is loaded while the current one is used, across group
-// boundaries, and after the last batch the stream's first batch is loaded again for the
-// next ket rows.
-// Workgroup w runs on XCD w % 8: consecutive workgroups of one XCD take the column tiles of
-// one bra row (rows wider than one tile), so the tiles' staged ket rows and slices meet in
-// that XCD's L2.  NTMAX bounds the workgroup (1024 threads; 768 for the widest FP64 rows,
-// whose accumulators need more than 128 VGPRs).
-template <class T, int M, int NTMAX>
-__global__ void __launch_bounds__(NTMAX) k_ab(int64_t na, int64_t nb, int L, int64_t ntiles,
-                                             const int64_t* __restrict__ rpSa,
-                                             const int32_t* __restrict__ colSa,
-                                             const uint32_t* __restrict__ excSa,
-                                             const int64_t* __restrict__ soff, const int32_t* __restrict__ nq,
-                                             const uint32_t* __restrict__ ent,
-                                             const int32_t* __restrict__ colperm, int nch, int64_t chunk,
-                                             int64_t kbase,
-                                             int64_t groups, const T* __restrict__ eri, const T* __restrict__ c,
-                                             T* __restrict__ sigma, int assign) {
+// ket columns: S groups of G ket rows of the chunk (signed) and their slices sit in LDS as
+// interleaved G-vectors, each lane walks its ELL entries for that chunk (the lane -> column
+// map is per chunk, so lanes of a group carry lists of similar length), and the chunk's sums
+// are added into the output row before the next chunk (through LDS in column order: scattered
+// 8-byte read-modify-writes fetch and write back whole cache lines once the rows in flight
+// outgrow the L2).  A wave's entries of a chunk are one stream, four rows per batch; the next
+// batch is loaded while the current one is used, across group boundaries, and after the last
+// batch the stream's first batch is loaded again for the next ket rows.
+//
+// Bound: the two 16-byte LDS gathers per entry (their bank conflicts above all); then the
+// staging, which the products of the same workgroup wait for.  What the staging costs is the
+// number of times a wave waits for memory in it, so no load of a round is under a condition
+// and the wave-uniform tables are scalar loads: with each ket value loaded and waited for in
+// its own exec region (as a condition on the row and the column compiles) k_ab<double> took
+// 83.9 ms at norb=36, 20,000^2 strings (FP32 45.0) and staging alone 29.6 of them; issued
+// together 69.5 (37.6), with two columns per load 68.1 (37.1); norb=26, 2,801 x 2,749: 1.56 ->
+// 0.93 ms, norb=58, 40,000^2: 318 -> 256 ms.  Rows of few columns take S groups per barrier
+// (239^2 at norb=18: 25 -> 21 us at S = 4).  Cutting rows into segments of their alpha
+// singles (build_segments) took norb=18, 239^2 from 132 to 26 us and norb=58, 200 x 40,000
+// from 6.7 to 1.0 ms: the Hartree-Fock row has ten times the singles of the average row.
+// Measured and not kept: batches of two rows (the shorter padding is no gain: the
+// padding reads one broadcast address), two batches in flight, two column tiles per row with
+// two workgroups on a CU at norb=36, 20,000^2 (91.8 ms: the ket rows are staged twice).
+template <class T, int M, int NT, int S>
+__global__ void __launch_bounds__(NT, NT == 768 ? 3 : 4) k_ab(const AbArgs<T> A) {
   using R = AbRows<T>;
   using RV = typename R::V;
   constexpr int G = R::G;
+  constexpr int B = AB_BATCH;
   // 16-byte vectors per thread per staging round: SR ket vectors (4*SR VGPRs beside the
-  // accumulators; eight only where they fit without spills) and SV slice vectors (at most
-  // 2,016 pairs: one round at 1,024 threads)
-  constexpr int SR = (sizeof(T) == 8 && M <= 20) ? 8 : 4;
+  // accumulators) and SV slice vectors
+  constexpr int SR = (int)sizeof(T) * M <= 160 ? 8 : 4;
   constexpr int SV = 2;
   extern __shared__ __align__(16) unsigned char smem[];
-  RV* Vv = reinterpret_cast<RV*>(smem);  // slice G-vectors of the pairs b > j
-  RV* cbv = Vv + kbase;                   // chunk + 1 G-vectors (the last one stays zero: padding)
-  const int64_t LL = (int64_t)L * L;
+  const int64_t nb = A.nb, chunk = A.chunk, kbase = A.kbase;
+  const int L = A.L;
   const int NP = L * (L - 1) / 2, NPS = max(NP, 1);  // slice vectors: pairs b > j (at least one)
-  const int NT = blockDim.x;
-  const int64_t npos = groups * 64;
+  const int64_t npos = A.groups * 64;
+  const int gvec = (int)(kbase + chunk + 1);  // LDS vectors of one staged group
   const int64_t xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const int64_t tile = slot % ntiles;
-  const int64_t ia = (slot / ntiles) * 8 + xcd;
-  if (ia >= na) return;  // the grid rounds the rows up to a multiple of 8 (whole workgroup)
-  const int64_t col0 = tile * (int64_t)NT * M;
+  const int64_t tile = slot % A.ntiles;
+  const int64_t seg = (slot / A.ntiles) * 8 + xcd;
+  if (seg >= A.nseg) return;  // the grid rounds the segments up to a multiple of 8 (whole workgroup)
+  const int64_t c0 = tile * (int64_t)NT * M, c1 = min(nb, c0 + (int64_t)NT * M);  // the tile's columns
+  const int64_t ia = uniform_at(A.segrow, seg);
+  const int64_t q0 = uniform_at(A.segq, 2 * seg), q1 = uniform_at(A.segq, 2 * seg + 1);
+  const int dst = uniform_at(A.segdst, seg);
+  T* out = dst < 0 ? A.sigma + ia * nb : A.part + (int64_t)dst * nb;
+  const bool assign = dst >= 0 || A.assign;
   const int lane = threadIdx.x & 63;
-  const int64_t s0 = (tile * (NT >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * nch;  // wave-uniform
-  if (threadIdx.x == 0)
-    for (int g = 0; g < G; ++g) cbv[chunk].v[g] = T(0);
-  const int64_t q0 = rpSa[ia], q1 = rpSa[ia + 1];
-  for (int k = 0; k < nch; ++k) {
+  const int64_t s0 = (tile * (NT >> 6) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * A.nch;  // wave-uniform
+  if (threadIdx.x < S) {
+    RV* z = reinterpret_cast<RV*>(smem) + (int64_t)threadIdx.x * gvec + kbase + chunk;
+    for (int g = 0; g < G; ++g) z->v[g] = T(0);
+  }
+  for (int k = 0; k < A.nch; ++k) {
     const int64_t j0 = (int64_t)k * chunk;
     const int nj = (int)(min(nb, j0 + chunk) - j0);
-    // this wave's entry stream of chunk k: `rows` rows (a multiple of four); pn holds the
+    // this wave's entry stream of chunk k: `rows` rows (a multiple of B); pn holds the
     // next batch, pf the row after it (wrapping to the start)
-    const int64_t so = soff[s0 + k];
-    const int rows = (int)((soff[s0 + k + 1] - so) >> 6);
-    const uint32_t* sp = ent + so;  // wave-uniform; lanes add their index
-    uint32_t pn[4];
+    const int64_t so = uniform_at(A.soff, s0 + k);
+    const int rows = (int)((uniform_at(A.soff, s0 + k + 1) - so) >> 6);
+    const uint32_t* sp = A.ent + so;  // wave-uniform; lanes add their index
+    uint32_t pn[B];
     int pf = 0;
 #pragma unroll
-    for (int u = 0; u < 4; ++u) pn[u] = (uint32_t)chunk;
+    for (int u = 0; u < B; ++u) pn[u] = (uint32_t)chunk;
     if (rows > 0) {
 #pragma unroll
-      for (int u = 0; u < 4; ++u) pn[u] = sp[u * 64 + lane];
-      pf = rows > 4 ? 4 : 0;
+      for (int u = 0; u < B; ++u) pn[u] = sp[u * 64 + lane];
+      pf = rows > B ? B : 0;
     }
     T acc[M];
 #pragma unroll
     for (int m = 0; m < M; ++m) acc[m] = T(0);
-    for (int64_t t = q0; t < q1; t += G) {
-      // rows t..t+G-1; rows at or past q1 are absent (zero)
-      T coef[G];
-      const T* crow[G];
-      const T* srow[G];
-      bool has[G];
+    for (int64_t t = q0; t < q1; t += S * G) {
       __syncthreads();  // previous rows done with LDS (and the previous chunk's sums are stored)
-#pragma unroll
-      for (int g = 0; g < G; ++g) {
-        const int64_t q = t + g;
-        has[g] = q < q1;
-        coef[g] = T(0);
-        crow[g] = c + ia * nb + j0;
-        srow[g] = eri;
-        if (has[g]) {
-          const uint32_t e = excSa[q];
-          coef[g] = ((e >> 24) & 1u) ? T(-1) : T(1);
-          crow[g] = c + (int64_t)colSa[q] * nb + j0;
-          srow[g] = eri + (int64_t)((int)((e >> 6) & 63u) * L + (int)(e & 63u)) * LL;  // (ai|..), a*L + i
-        }
-      }
-      // the G slices and the G ket rows' chunk into LDS: in rounds of SR ket and SV slice
-      // vectors per thread, every global load of a round issued before its LDS stores (the loads do not depend on
-      // each other), so a round costs one memory latency.  The thread index is opaque here so
-      // that the addresses are formed per step rather than held in registers through the
-      // products.
+      // The thread index is opaque here so that the addresses are formed per step rather
+      // than held in registers through the products.
       int xt = (int)threadIdx.x;
       asm volatile("" : "+v"(xt));
-      for (int x0 = xt, y0 = xt; x0 < nj || y0 < NPS; x0 += SR * NT, y0 += SV * NT) {
-        RV sv[SV], kv[SR];
 #pragma unroll
-        for (int u = 0; u < SV; ++u) {
-          // slice vector y is orbital pair (b, j), b > j, y = b(b-1)/2 + j: element b*L + j
-          // of the slice (the float root is exact to within one, corrected below)
-          const int y = y0 + u * NT;
-          const bool sl = y < NP;
-          int src = 0;
-          if (sl) {
-            int b = (int)((1.0f + __builtin_sqrtf(8.0f * (float)y + 1.0f)) * 0.5f);
-            if (b * (b - 1) / 2 > y) --b;
-            else if (b * (b + 1) / 2 <= y) ++b;
-            src = b * L + (y - b * (b - 1) / 2);
+      for (int sg = 0; sg < S; ++sg) {
+        RV* Vv = reinterpret_cast<RV*>(smem) + sg * gvec;  // slice G-vectors of the pairs b > j
+        RV* cbv = Vv + kbase;                               // ket G-vectors
+        // rows t..t+G-1 of the group; rows at or past q1 are absent: their ket values are set
+        // to zero (their slice is any finite one)
+        uint32_t neg[G];
+        const T* crow[G];
+        const T* srow[G];
+        bool has[G];
+#pragma unroll
+        for (int g = 0; g < G; ++g) {
+          const int64_t q = min(t + sg * G + g, q1 - 1);
+          has[g] = t + sg * G + g < q1;
+          const uint32_t e = uniform_at(A.excSa, q);
+          neg[g] = ((e >> 24) & 1u) << 31;
+          crow[g] = A.c + (int64_t)uniform_at(A.colSa, q) * nb + j0;
+          srow[g] = A.Vt + (int64_t)ab_pair((e >> 6) & 63u, e & 63u) * NP;  // (ai|..)
+        }
+        // the G slices and the G rows' chunk (signed by the alpha single) into LDS: in rounds
+        // of SR ket and SV slice vectors per thread.  Every global load of a round is issued,
+        // at an index held inside the row, before its first use: a round costs one memory
+        // latency (a load under a condition is waited for by itself).
+        const int xl = max(nj - 2, 0);   // the last pair of columns starts at xl
+        if (nj < 2 && xt == 0) {  // a single column
+#pragma unroll
+          for (int g = 0; g < G; ++g) cbv[0].v[g] = has[g] ? R::flip(crow[g][0], neg[g]) : T(0);
+        }
+        for (int x0 = nj < 2 ? 2 : 2 * xt, y0 = xt; x0 < nj || y0 < NPS; x0 += SR * NT, y0 += SV * NT) {
+          RV sv[SV], kv[SR];
+#pragma unroll
+          for (int u = 0; u < SV; ++u) {
+            const int y = min(y0 + u * NT, NPS - 1);
+#pragma unroll
+            for (int g = 0; g < G; ++g) sv[u].v[g] = srow[g][y];
           }
 #pragma unroll
-          for (int g = 0; g < G; ++g) sv[u].v[g] = (has[g] && sl) ? srow[g][src] : T(0);
-        }
+          for (int u = 0; u < SR; u += 2) {
+            const int x = min(x0 + u * NT, xl);
 #pragma unroll
-        for (int u = 0; u < SR; ++u) {
-          const int x = x0 + u * NT;
+            for (int g = 0; g < G; ++g) {
+              const typename R::P2 w = __builtin_nontemporal_load(reinterpret_cast<const typename R::P2*>(crow[g] + x));
+              kv[u].v[g] = w.x;
+              kv[u + 1].v[g] = w.y;
+            }
+          }
 #pragma unroll
-          for (int g = 0; g < G; ++g)
-            kv[u].v[g] = (has[g] && x < nj) ? __builtin_nontemporal_load(crow[g] + x) : T(0);
-        }
+          for (int u = 0; u < SV; ++u) {
+            const int y = y0 + u * NT;
+            if (y < NPS) Vv[y] = sv[u];
+          }
 #pragma unroll
-        for (int u = 0; u < SV; ++u) {
-          const int y = y0 + u * NT;
-          if (y < NPS) Vv[y] = sv[u];
-        }
+          for (int u = 0; u < SR; u += 2) {
 #pragma unroll
-        for (int u = 0; u < SR; ++u) {
-          const int x = x0 + u * NT;
-          if (x < nj) cbv[x] = kv[u];
+            for (int g = 0; g < G; ++g) {
+              kv[u].v[g] = has[g] ? R::flip(kv[u].v[g], neg[g]) : T(0);
+              kv[u + 1].v[g] = has[g] ? R::flip(kv[u + 1].v[g], neg[g]) : T(0);
+            }
+            const int xx = x0 + u * NT, x = min(xx, xl);
+            if (xx < nj) {
+              cbv[x] = kv[u];
+              cbv[x + 1] = kv[u + 1];
+            }
+          }
         }
       }
       __syncthreads();
@@ -517,24 +557,25 @@ __global__ void __launch_bounds__(NTMAX) k_ab(int64_t na, int64_t nb, int L, int
       asm volatile("" : "+s"(qi));
 #pragma unroll
       for (int m = 0; m < M; ++m) {
-        const int nb4 = nq[qi + m];  // batches of this wave's m-th group
-        T sg[G];
+        const int nbt = uniform_at(A.nq, qi + m);  // batches of this wave's m-th group
+        T s[G];
 #pragma unroll
-        for (int r = 0; r < G; ++r) sg[r] = T(0);
-        for (int b = 0; b < nb4; ++b) {
-          uint32_t p[4];
+        for (int g = 0; g < G; ++g) s[g] = T(0);
+        for (int b = 0; b < nbt; ++b) {
+          uint32_t p[B];
           const uint32_t* rp = sp + pf * 64;
 #pragma unroll
-          for (int u = 0; u < 4; ++u) {
+          for (int u = 0; u < B; ++u) {
             p[u] = pn[u];
             pn[u] = rp[u * 64 + lane];
           }
-          pf = pf + 4 == rows ? 0 : pf + 4;
-          ab_batch<T>(p, sg);
+          pf = pf + B == rows ? 0 : pf + B;
+#pragma unroll
+          for (int sg = 0; sg < S; ++sg) ab_batch<T, B>(p, (uint32_t)(sg * gvec) * 16u, s);
         }
         T a = acc[m];
 #pragma unroll
-        for (int r = 0; r < G; ++r) a += coef[r] * sg[r];
+        for (int g = 0; g < G; ++g) a += s[g];
         asm volatile("" : "+v"(a));  // formed here, so the group's partial sums die here
         acc[m] = a;
       }
@@ -543,56 +584,43 @@ __global__ void __launch_bounds__(NTMAX) k_ab(int64_t na, int64_t nb, int L, int
     int ft = (int)threadIdx.x;
     asm volatile("" : "+v"(ft));
     const bool first = assign && k == 0;  // every column has a position in chunk 0
-    if (ntiles == 1) {
-      // One tile holds the whole row, each column at exactly one position of this chunk: the
-      // sums go through LDS (the slices and ket vectors, idle now and staged again for the
-      // next rows; the zero slot after them stays untouched) one block of columns at a time,
-      // then into sigma with coalesced
-      // read-modify-writes.  Scattered 8-byte ones fetch and write back whole cache lines
-      // once the rows in flight outgrow the L2 (at 40,000 columns they moved 4.7x the
-      // kernel's algorithmic bytes).  Each element is read and written by the same thread in
-      // every chunk.
-      T* rowbuf = reinterpret_cast<T*>(Vv);
-      const int64_t cap = (kbase + chunk) * G;
-      T* out = sigma + ia * nb;
-      for (int64_t b0 = 0; b0 < nb; b0 += cap) {
-        const int64_t b1 = min(nb, b0 + cap);
-        __syncthreads();  // the products, or the previous block's readers, are done with LDS
-        int fb = ft;  // opaque per block: the column map is read per block, not held in M registers
-        asm volatile("" : "+v"(fb));
-#pragma unroll
-        for (int m = 0; m < M; ++m) {
-          const int64_t pos = (int64_t)m * NT + fb;
-          if ((pos >> 6) < groups) {
-            const int32_t ib = colperm[(int64_t)k * npos + pos];
-            if (ib >= b0 && ib < b1) rowbuf[ib - b0] = acc[m];
-          }
-        }
-        __syncthreads();
-        for (int64_t x = threadIdx.x; x < b1 - b0; x += NT) {
-          if (first) out[b0 + x] = rowbuf[x];
-          else out[b0 + x] += rowbuf[x];
-        }
-      }
-    } else {
+    // Each column of the tile sits at exactly one position of this chunk: the sums go through
+    // LDS (the slices and ket vectors of the first group, idle now; the zero slot after them
+    // stays untouched) one block of columns at a time, then into the output row with coalesced
+    // read-modify-writes.  Each element is read and written by the same thread in every chunk.
+    T* rowbuf = reinterpret_cast<T*>(smem);
+    const int64_t cap = (kbase + chunk) * G;
+    for (int64_t b0 = c0; b0 < c1; b0 += cap) {
+      const int64_t b1 = min(c1, b0 + cap);
+      __syncthreads();  // the products, or the previous block's readers, are done with LDS
+      int fb = ft;  // opaque per block: the column map is read per block, not held in M registers
+      asm volatile("" : "+v"(fb));
 #pragma unroll
       for (int m = 0; m < M; ++m) {
-        const int64_t pos = col0 + (int64_t)m * NT + ft;
-        if ((pos >> 6) < groups) {
-          const int32_t ib = colperm[(int64_t)k * npos + pos];
-          if (ib >= 0) {
-            if (first) sigma[ia * nb + ib] = acc[m];
-            else sigma[ia * nb + ib] += acc[m];
-          }
-        }
+        const int64_t pos = c0 + (int64_t)m * NT + fb;
+        const int32_t ib = A.colperm[(int64_t)k * npos + pos];
+        if (ib >= b0 && ib < b1) rowbuf[ib - b0] = acc[m];
+      }
+      __syncthreads();
+      for (int64_t x = threadIdx.x; x < b1 - b0; x += NT) {
+        if (first) out[b0 + x] = rowbuf[x];
+        else out[b0 + x] += rowbuf[x];
       }
     }
-    // with several tiles a column's owner thread changes from chunk to chunk: the next
-    // chunk's read-modify-write of an element must see this chunk's store.  The barriers
-    // inside the row loop order them only when the bra row has alpha singles; this one also
-    // covers rows without (and the LDS reads of the last flush block).
-    if (nch > 1) __syncthreads();
   }
+}
+
+// out[row, :] += the partial rows of the row's further segments, in order
+template <class T>
+__global__ void __launch_bounds__(256) k_ab_join(int64_t nb, const int32_t* __restrict__ jrow,
+                                                 const int32_t* __restrict__ jptr, const T* __restrict__ part,
+                                                 T* __restrict__ out) {
+  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  if (c >= nb) return;
+  const int64_t r = jrow[blockIdx.y];
+  T v = out[r * nb + c];
+  for (int e = jptr[blockIdx.y]; e < jptr[blockIdx.y + 1]; ++e) v += part[(int64_t)e * nb + c];
+  out[r * nb + c] = v;
 }
 
 template <class T>
@@ -687,21 +715,42 @@ void launch_transpose(int64_t R, int64_t C, const T* in, T* out, hipStream_t st,
   hipLaunchKernelGGL((k_transpose<T, ADD>), g, dim3(256), 0, st, R, C, in, out, add);
 }
 
-template <class T, int M, int NTMAX = 1024>
+template <class T, int M, int NT, int S>
 void launch_ab_m(const SigmaPlan& P, size_t lds, const T* eri, const T* c, T* sigma, hipStream_t st, int assign) {
   const EllTable& E = *P.ell;
-  if (E.nt > NTMAX || E.nt % 64) throw Error(SBDG_ERR_STATE, "alpha-beta workgroup size");
-  const int64_t nblk = (P.na + 7) / 8 * 8 * E.ntiles;
+  const AbSegments& G = *P.seg;
+  const int64_t nblk = (G.nseg + 7) / 8 * 8 * E.ntiles;
   if (nblk > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
   static const bool lds_at_zero = [] {  // entries hold absolute LDS byte addresses
     hipFuncAttributes fa;
-    return hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&k_ab<T, M, NTMAX>)) == hipSuccess &&
+    return hipFuncGetAttributes(&fa, reinterpret_cast<const void*>(&k_ab<T, M, NT, S>)) == hipSuccess &&
            fa.sharedSizeBytes == 0;
   }();
   if (!lds_at_zero) throw Error(SBDG_ERR_STATE, "alpha-beta kernel has static LDS: entry addresses invalid");
-  hipLaunchKernelGGL((k_ab<T, M, NTMAX>), dim3((unsigned)nblk), dim3(E.nt), lds, st, P.na, P.nb, P.L, E.ntiles,
-                     P.sa->rowptr.p, P.sa->col.p, P.sa->exc.p, E.soff.p, E.nq.p, E.ent.p, E.colperm.p, E.nch, E.chunk,
-                     E.kbase, E.groups, eri, c, sigma, assign);
+  AbArgs<T> A;
+  A.nb = P.nb;
+  A.ntiles = E.ntiles;
+  A.chunk = E.chunk;
+  A.kbase = E.kbase;
+  A.groups = E.groups;
+  A.L = P.L;
+  A.nch = E.nch;
+  A.nseg = (int)G.nseg;
+  A.assign = assign;
+  A.segrow = G.row.p;
+  A.segq = G.q.p;
+  A.segdst = G.dst.p;
+  A.colSa = P.sa->col.p;
+  A.excSa = P.sa->exc.p;
+  A.soff = E.soff.p;
+  A.nq = E.nq.p;
+  A.ent = E.ent.p;
+  A.colperm = E.colperm.p;
+  A.Vt = eri;
+  A.c = c;
+  A.sigma = sigma;
+  A.part = reinterpret_cast<T*>(G.part.p);
+  hipLaunchKernelGGL((k_ab<T, M, NT, S>), dim3((unsigned)nblk), dim3(NT), lds, st, A);
 }
 
 template <class T>
@@ -709,32 +758,44 @@ void launch_ab(const SigmaPlan& P, const T* eri, const T* c, T* sigma, hipStream
   if (P.na == 0 || P.nb == 0) return;
   const EllTable& E = *P.ell;
   if ((int64_t)E.nt * E.m * E.ntiles != E.groups * 64) throw Error(SBDG_ERR_STATE, "alpha-beta table geometry");
-  const size_t lds = ab_lds_bytes(E.kbase, E.chunk);
-  switch (E.m) {  // columns per thread, fixed when the table was built
-    case 1: launch_ab_m<T, 1>(P, lds, eri, c, sigma, st, assign); break;
-    case 2: launch_ab_m<T, 2>(P, lds, eri, c, sigma, st, assign); break;
-    case 4: launch_ab_m<T, 4>(P, lds, eri, c, sigma, st, assign); break;
-    case 8: launch_ab_m<T, 8>(P, lds, eri, c, sigma, st, assign); break;
-    case 12: launch_ab_m<T, 12>(P, lds, eri, c, sigma, st, assign); break;
-    case 16: launch_ab_m<T, 16>(P, lds, eri, c, sigma, st, assign); break;
-    case 20: launch_ab_m<T, 20>(P, lds, eri, c, sigma, st, assign); break;
-    case 24: launch_ab_m<T, 24>(P, lds, eri, c, sigma, st, assign); break;
-    default:
-      if constexpr (sizeof(T) == 8) {  // 768 threads (ab_geometry)
-        switch (E.m) {
-          case 32: launch_ab_m<T, 32, 768>(P, lds, eri, c, sigma, st, assign); return;
-          case 40: launch_ab_m<T, 40, 768>(P, lds, eri, c, sigma, st, assign); return;
-          case 48: launch_ab_m<T, 48, 768>(P, lds, eri, c, sigma, st, assign); return;
-          case 53: launch_ab_m<T, 53, 768>(P, lds, eri, c, sigma, st, assign); return;
-        }
-      } else {
-        switch (E.m) {
-          case 40: launch_ab_m<T, 40>(P, lds, eri, c, sigma, st, assign); return;
-          case 48: launch_ab_m<T, 48>(P, lds, eri, c, sigma, st, assign); return;
-        }
-      }
-      throw Error(SBDG_ERR_STATE, "alpha-beta columns per thread");
+  const size_t lds = ab_lds_bytes(E.kbase, E.chunk) * E.s;
+  bool done = false;  // the shapes ab_geometry picks
+#define SBDG_AB(NT, M, S)                                        \
+  if (!done && E.nt == NT && E.m == M && E.s == S) {             \
+    launch_ab_m<T, M, NT, S>(P, lds, eri, c, sigma, st, assign); \
+    done = true;                                                 \
   }
+  SBDG_AB(256, 1, 4)
+  SBDG_AB(256, 1, 2)
+  SBDG_AB(256, 2, 4)
+  SBDG_AB(256, 2, 2)
+  SBDG_AB(256, 4, 2)
+  SBDG_AB(256, 4, 1)
+  SBDG_AB(512, 4, 1)
+  SBDG_AB(512, 6, 1)
+  SBDG_AB(512, 8, 1)
+  SBDG_AB(512, 10, 1)
+  SBDG_AB(512, 12, 1)
+  SBDG_AB(1024, 8, 1)
+  SBDG_AB(1024, 12, 1)
+  SBDG_AB(1024, 16, 1)
+  SBDG_AB(1024, 20, 1)
+  SBDG_AB(1024, 24, 1)
+  if constexpr (sizeof(T) == 8) {
+    SBDG_AB(768, 32, 1)
+    SBDG_AB(768, 40, 1)
+    SBDG_AB(768, 48, 1)
+    SBDG_AB(768, 53, 1)
+  } else {
+    SBDG_AB(1024, 40, 1)
+    SBDG_AB(1024, 48, 1)
+  }
+#undef SBDG_AB
+  if (!done) throw Error(SBDG_ERR_STATE, "alpha-beta columns per thread");
+  const AbSegments& G = *P.seg;
+  if (G.njoin > 0)
+    hipLaunchKernelGGL(k_ab_join<T>, dim3((unsigned)((P.nb + 255) / 256), (unsigned)G.njoin), dim3(256), 0, st, P.nb,
+                       G.jrow.p, G.jptr.p, reinterpret_cast<const T*>(G.part.p), sigma);
 }
 
 }  // namespace
@@ -757,10 +818,10 @@ void sigma_apply(const SigmaPlan& P, const T* c, T* sigma, const SigmaScratch<T>
   const T* eri;
   if constexpr (sizeof(T) == 8) {
     hii = reinterpret_cast<const T*>(P.hii);
-    eri = reinterpret_cast<const T*>(P.eri);
+    eri = reinterpret_cast<const T*>(P.Vt);
   } else {
     hii = reinterpret_cast<const T*>(P.hii32);
-    eri = reinterpret_cast<const T*>(P.eri32);
+    eri = reinterpret_cast<const T*>(P.Vt32);
   }
   if (ev) SBDG_CHECK(hipEventRecord(ev[0], st));
   // the alpha-beta terms (LDS-bound) into their own buffer on the second stream, while the

@@ -324,6 +324,24 @@ __global__ void k_pair_int(const double* __restrict__ eri, int L, int64_t npair,
   W32[t] = (float)v;
 }
 
+__global__ void k_pair_slices(const double* __restrict__ eri, int L, int64_t npair, double* __restrict__ Vt,
+                              float* __restrict__ Vt32) {
+  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= npair * npair) return;
+  auto unpair = [](int64_t p, int& lo, int& hi) {
+    int b = 1;
+    while ((int64_t)(b + 1) * b / 2 <= p) ++b;
+    hi = b;
+    lo = (int)(p - (int64_t)b * (b - 1) / 2);
+  };
+  int a, i, b, j;
+  unpair(t / npair, i, a);
+  unpair(t % npair, j, b);
+  const double v = eri4(eri, L, a, i, b, j);
+  Vt[t] = v;
+  Vt32[t] = (float)v;
+}
+
 // per-string diagonal parts: E[s] = sum_{i in s} h_ii + sum_{i<j in s} [(ii|jj)-(ij|ji)]
 __global__ void k_strdiag(const uint64_t* __restrict__ s, int64_t n, int L,
                           const double* __restrict__ h1, const double* __restrict__ eri,
@@ -475,32 +493,103 @@ void build_ab(const Table& sb, int L, int64_t chunk, AbTable& ab, hipStream_t st
   SBDG_CHECK(hipGetLastError());
 }
 
-// Alpha-beta launch geometry: nt threads, m columns per thread, so that one workgroup
-// covers a whole row (the ket rows and integral slices are then staged once per bra row,
-// not once per column tile).  The FP64 accumulators bound m: 1024 threads (four waves per
-// SIMD, 128 VGPRs) hold up to 24 columns each; beyond 24,576 columns FP64 takes 768 threads
-// (three waves per SIMD, 168 VGPRs) with up to 53 columns each.  FP32 holds up to 48
-// columns at 1024 threads.  Wider rows take several column tiles at the largest m.
-void ab_geometry(int64_t nb, int elem, int& nt, int& m) {
-  nt = (int)std::min<int64_t>(1024, std::max<int64_t>(64, (nb + 63) / 64 * 64));
-  static const int m1024_64[] = {1, 2, 4, 8, 12, 16, 20, 24};
-  static const int m768_64[] = {32, 40, 48, 53};
-  static const int m1024_32[] = {1, 2, 4, 8, 12, 16, 20, 24, 40, 48};
-  const int* ms = elem == 4 ? m1024_32 : m1024_64;
-  int nms = elem == 4 ? 10 : 8;
-  int64_t need = (nb + nt - 1) / nt;
-  if (elem != 4 && need > 24) {
-    nt = 768;
-    need = (nb + nt - 1) / nt;
-    ms = m768_64;
-    nms = 4;
+// Alpha-beta launch geometry for rows of nb columns: nt threads, m columns per thread, so that
+// one workgroup covers a whole row where it can (a second column tile stages every ket row
+// again: norb=36, 4,000 x 24,000 9.2 ms with one tile, 11.7 with two), s groups of ket rows
+// staged per barrier, and the ket columns cut into equal chunks that fill the LDS share.
+//  * up to 1,024 columns: 256 threads and several groups per barrier while a few workgroups
+//    still fit a CU (norb=26, 2,000 x 1,000: 259 us with one group, 214 with two; norb=58,
+//    600 x 400: 115 / 104 / 249 us with one, two and four);
+//  * up to 6,000: 512 threads and half the LDS, so that two workgroups share a CU and one
+//    stages while the other computes (FP64, against 1,024 threads and all of it: norb=26,
+//    2,801 x 2,749 0.93 and 1.21 ms, norb=36, 5,001 x 4,999 1.65 and 1.97 ms, 1,000 x 7,000
+//    equal, 800 x 10,000 0.72 and 0.71, 500 x 15,000 1.01 and 0.82: more chunks, each with its
+//    slices and part-filled batches);
+//  * beyond: one workgroup per CU with all of its LDS.  FP64 accumulators bound the columns
+//    per thread: 1,024 threads (four waves per SIMD, 128 VGPRs) hold 24, 768 threads (three
+//    waves, 168 VGPRs) 53 (norb=58, 40,000^2 in one tile 256 ms, in two tiles of 1,024 threads
+//    316); FP32 holds 48 at 1,024 threads.  Wider rows take several tiles.
+AbGeometry ab_geometry(int64_t nb, int L, int elem) {
+  AbGeometry g;
+  const int64_t kb = ab_slice_span(L);
+  const bool half = nb <= 6000;
+  g.nt = nb <= 1024 ? 256 : half ? 512 : 1024;
+  g.s = 1;
+  if (nb <= 1024) {
+    const int64_t grp = 16 * (kb + nb + 1);
+    g.s = nb <= 512 && 4 * grp <= 48 * 1024 ? 4 : 2 * grp <= 80 * 1024 ? 2 : 1;
   }
-  m = ms[nms - 1];
-  for (int i = 0; i < nms; ++i)
-    if (need <= ms[i]) {
-      m = ms[i];
-      break;
+  if (elem == 8 && nb > 24 * 1024) g.nt = 768;
+  const int64_t maxchunk = (half ? 80 : 160) * 1024 / 16 / g.s - kb - 1;
+  const int64_t nch = std::max<int64_t>(1, (nb + maxchunk - 1) / maxchunk);
+  g.chunk = std::max<int64_t>(1, (nb + nch - 1) / nch);
+  static const int m256[] = {1, 2, 4, 0}, m512[] = {4, 6, 8, 10, 12, 0}, m1024d[] = {8, 12, 16, 20, 24, 0},
+                   m1024f[] = {8, 12, 16, 20, 24, 40, 48, 0}, m768[] = {32, 40, 48, 53, 0};
+  const int* ms = g.nt == 256 ? m256 : g.nt == 512 ? m512 : g.nt == 768 ? m768 : elem == 4 ? m1024f : m1024d;
+  g.m = 0;
+  for (int i = 0; ms[i]; ++i) {
+    g.m = ms[i];
+    if (nb <= (int64_t)ms[i] * g.nt) break;
+  }
+  return g;
+}
+
+// Segment length: an equal share of all alpha singles (times column tiles) over two workgroups
+// per CU, between 8 and 64 singles, in multiples of 8 (whole staging groups in both precisions);
+// longer where the partial rows would outgrow AB_PART_BYTES.  Longest first, so that the last
+// workgroups to start are short.  Lengths of 16, 32 and 64 measure alike at norb=26, 4,000^2
+// (2.63 / 2.63 / 2.61 ms); one segment per row 2.61 there, but 0.68 against 1.63 ms at norb=36,
+// 3,600 x 3,500 in FP32.
+void build_segments(const Table& sa, int64_t nb, int64_t ntiles, AbSegments& g, hipStream_t st) {
+  const int64_t na = sa.n;
+  std::vector<int64_t> rp(na + 1, 0);
+  SBDG_CHECK(hipMemcpyAsync(rp.data(), sa.rowptr.p, sizeof(int64_t) * (na + 1), hipMemcpyDeviceToHost, st));
+  SBDG_CHECK(hipStreamSynchronize(st));
+  int64_t len = std::min<int64_t>(64, std::max<int64_t>(8, (rp[na] * ntiles / 512 + 7) / 8 * 8));
+  auto extra = [&](int64_t l) {
+    int64_t e = 0;
+    for (int64_t r = 0; r < na; ++r) e += std::max<int64_t>(0, (rp[r + 1] - rp[r] - 1) / l);
+    return e;
+  };
+  while (extra(len) * nb * (int64_t)sizeof(double) > AB_PART_BYTES) len *= 2;
+  struct Seg {
+    int32_t row, dst;
+    int64_t q0, q1;
+  };
+  std::vector<Seg> segs;
+  std::vector<int32_t> jrow, jptr(1, 0);
+  int32_t np = 0;
+  for (int64_t r = 0; r < na; ++r) {
+    segs.push_back({(int32_t)r, -1, rp[r], std::min(rp[r + 1], rp[r] + len)});
+    if (rp[r] + len < rp[r + 1]) {
+      for (int64_t q = rp[r] + len; q < rp[r + 1]; q += len)
+        segs.push_back({(int32_t)r, np++, q, std::min(rp[r + 1], q + len)});
+      jrow.push_back((int32_t)r);
+      jptr.push_back(np);
     }
+  }
+  std::stable_sort(segs.begin(), segs.end(), [](const Seg& x, const Seg& y) { return x.q1 - x.q0 > y.q1 - y.q0; });
+  std::vector<int32_t> row, dst;
+  std::vector<int64_t> q;
+  for (const Seg& x : segs) {
+    row.push_back(x.row);
+    dst.push_back(x.dst);
+    q.push_back(x.q0);
+    q.push_back(x.q1);
+  }
+  g.nseg = (int64_t)segs.size();
+  g.npart = np;
+  g.njoin = (int64_t)jrow.size();
+  auto up = [&](auto& d, const auto& h) {
+    d.alloc(std::max<size_t>(h.size(), 1));
+    if (!h.empty()) SBDG_CHECK(hipMemcpy(d.p, h.data(), sizeof(h[0]) * h.size(), hipMemcpyHostToDevice));
+  };
+  up(g.row, row);
+  up(g.dst, dst);
+  up(g.q, q);
+  up(g.jrow, jrow);
+  up(g.jptr, jptr);
+  g.part.alloc(std::max<int64_t>((int64_t)np * nb, 1));
 }
 
 // Order of the entries of the lanes of one (group, chunk) block, step by step, so that the
@@ -571,14 +660,18 @@ static void schedule_block(std::vector<std::vector<uint32_t>>& lists, int K, int
   }
 }
 
-void build_ell(const Table& sb, int L, int64_t chunk, int prec_bytes, EllTable& e, hipStream_t st) {
+void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t st) {
   const int64_t nb = sb.n;
+  const AbGeometry geo = ab_geometry(nb, L, prec_bytes);
+  const int64_t chunk = geo.chunk;
   if (L > 64) throw Error(SBDG_ERR_LIMIT, "norb beyond 64");
   e.kbase = ab_slice_span(L);
   if (16 * (e.kbase + chunk + 1) > (1 << 18)) throw Error(SBDG_ERR_LIMIT, "alpha-beta LDS beyond 256 KiB");
   e.chunk = chunk;
   e.nch = (int)std::max<int64_t>(1, (nb + chunk - 1) / chunk);
-  ab_geometry(nb, prec_bytes, e.nt, e.m);
+  e.nt = geo.nt;
+  e.m = geo.m;
+  e.s = geo.s;
   const int64_t tw = (int64_t)e.nt * e.m;
   e.ntiles = std::max<int64_t>(1, (nb + tw - 1) / tw);
   const int64_t npos = e.ntiles * tw;
@@ -600,22 +693,17 @@ void build_ell(const Table& sb, int L, int64_t chunk, int prec_bytes, EllTable& 
   std::vector<int32_t> cnt((size_t)nb * nch, 0);
   for (int64_t ib = 0; ib < nb; ++ib)
     for (int64_t q = rp[ib]; q < rp[ib + 1]; ++q) ++cnt[(size_t)ib * nch + col[q] / chunk];
-  // column tiles: columns by decreasing total count, cut into tiles of tw lane positions;
-  // inside a tile, each chunk orders its columns by decreasing count in that chunk, so the
-  // 64 lanes of a group carry similar lists (little padding).  A column stays in its tile
-  // for every chunk: one workgroup owns it.
-  std::vector<int32_t> order(nb);
-  for (int64_t i = 0; i < nb; ++i) order[i] = (int32_t)i;
-  std::vector<int32_t> tot(nb, 0);
-  for (int64_t ib = 0; ib < nb; ++ib)
-    for (int k = 0; k < nch; ++k) tot[ib] += cnt[(size_t)ib * nch + k];
-  std::stable_sort(order.begin(), order.end(), [&](int32_t x, int32_t y) { return tot[x] > tot[y]; });
+  // column tiles: contiguous ranges of tw columns; inside a tile, each chunk orders its
+  // columns by decreasing count in that chunk, so the 64 lanes of a group carry similar
+  // lists (little padding).  A column stays in its tile for every chunk: one workgroup owns
+  // it, and the workgroup's output is a contiguous piece of the row.
   std::vector<int32_t> perm((size_t)std::max<int64_t>(npos * nch, 1), -1);
   for (int k = 0; k < nch; ++k) {
     for (int64_t t = 0; t < e.ntiles; ++t) {
       const int64_t lo = t * tw, hi = std::min<int64_t>(nb, lo + tw);
       if (lo >= hi) break;
-      std::vector<int32_t> cols(order.begin() + lo, order.begin() + hi);
+      std::vector<int32_t> cols(hi - lo);
+      for (int64_t i = lo; i < hi; ++i) cols[i - lo] = (int32_t)i;
       std::stable_sort(cols.begin(), cols.end(), [&](int32_t x, int32_t y) {
         return cnt[(size_t)x * nch + k] > cnt[(size_t)y * nch + k];
       });
@@ -631,12 +719,12 @@ void build_ell(const Table& sb, int L, int64_t chunk, int prec_bytes, EllTable& 
           if (used[w] < e.m && (best < 0 || load[w] < load[best])) best = w;
         const int64_t slot = (int64_t)best + (int64_t)used[best] * Wv;
         ++used[best];
-        load[best] += (mx + 3) & ~3;
+        load[best] += (mx + AB_BATCH - 1) / AB_BATCH * AB_BATCH;
         for (size_t l = 0; l < 64 && i0 + l < cols.size(); ++l) perm[(size_t)k * npos + lo + slot * 64 + l] = cols[i0 + l];
       }
     }
   }
-  // rows of each (group, chunk) block: the longest list of its lanes, rounded up to four
+  // rows of each (group, chunk) block: the longest list of its lanes, rounded up to whole batches
   std::vector<int32_t> K((size_t)std::max<int64_t>(ng, 1), 0);
   for (int64_t g = 0; g < e.groups; ++g)
     for (int k = 0; k < nch; ++k) {
@@ -645,7 +733,7 @@ void build_ell(const Table& sb, int L, int64_t chunk, int prec_bytes, EllTable& 
         const int32_t ib = perm[(size_t)k * npos + g * 64 + l];
         if (ib >= 0) mx = std::max(mx, cnt[(size_t)ib * nch + k]);
       }
-      K[g * nch + k] = (mx + 3) & ~3;
+      K[g * nch + k] = (mx + AB_BATCH - 1) / AB_BATCH * AB_BATCH;
     }
   // one stream per (tile, wave, chunk): the wave's groups j = 0..m-1 one after another
   const int W = e.nt / 64;
@@ -660,7 +748,7 @@ void build_ell(const Table& sb, int L, int64_t chunk, int prec_bytes, EllTable& 
         for (int j = 0; j < e.m; ++j) {
           const int64_t g = t * W * e.m + w + (int64_t)j * W;
           off[g * nch + k] = o;
-          nq[s * e.m + j] = K[g * nch + k] / 4;
+          nq[s * e.m + j] = K[g * nch + k] / AB_BATCH;
           o += (int64_t)K[g * nch + k] * 64;
         }
         soff[s + 1] = o;
@@ -872,6 +960,13 @@ void build_pair_integrals(const double* d_eri, int L, double* W, float* W32, hip
   hipLaunchKernelGGL(k_pair_int, dim3(blocks_for(npair * npair, 256)), dim3(256), 0, st, d_eri, L, npair, W, W32);
   SBDG_CHECK(hipGetLastError());
   SBDG_CHECK(hipStreamSynchronize(st));
+}
+
+void build_pair_slices(const double* d_eri, int L, double* Vt, float* Vt32, hipStream_t st) {
+  const int64_t npair = (int64_t)L * (L - 1) / 2;
+  if (npair == 0) return;
+  hipLaunchKernelGGL(k_pair_slices, dim3(blocks_for(npair * npair, 256)), dim3(256), 0, st, d_eri, L, npair, Vt, Vt32);
+  SBDG_CHECK(hipGetLastError());
 }
 
 void compute_hii(const uint64_t* d_a, int64_t na, const uint64_t* d_b, int64_t nb, int L, double core,
