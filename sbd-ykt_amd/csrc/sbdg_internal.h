@@ -192,7 +192,8 @@ struct CoreTable {
 };
 constexpr int CORE_XB = 16;     // output members per product block
 constexpr int CORE_COLS = 512;  // column granularity of the core-product passes
-constexpr int CORE_WORK = 256;  // member rows streamed per core-product workgroup (target)
+constexpr int CORE_WORK = 256;  // member rows streamed per core-product workgroup (at most, when several blocks share one)
+constexpr int CORE_WGS = 4096;  // workgroups a core pass should have before blocks are grouped
 // Smallest core taken through the workspace: a core of k members costs about 3k row
 // transfers there (member rows in, Z out, Z gathered) and at most k(k-1) read directly,
 // fewer where members' pairs overlap, and the direct reads of one core's member rows hit
@@ -206,8 +207,8 @@ void build_table(const uint64_t* d_str, int64_t n, int L, const double* d_h1, co
                  Table& t_single, Table& t_double, hipStream_t st);
 void build_spmm(const Table& s, const Table& d, SpmmTable& m, int L, hipStream_t st, bool with_doubles = true);
 // h_eri: the integrals on the host (full L^4), for the values of the direct pairs
-void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* h_eri, CoreTable& ct,
-                 Table& direct, hipStream_t st);
+void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* h_eri, int64_t ncols,
+                 CoreTable& ct, Table& direct, hipStream_t st);
 // J[(p+1)*n + r] = sum_{o in occ(s[r])} eri[p*L^2 + o*L + o] for p < L^2 (row 0 zero):
 // the occupation part of the other spin's singles, (ai|oo) summed over the string's orbitals
 void build_occ_table(const uint64_t* d_str, int64_t n, int L, const double* d_eri, double* J, float* J32,

@@ -24,16 +24,20 @@ template <class T>
 struct V16;
 template <>
 struct V16<double> {
-  using t = double2;
+  typedef double u __attribute__((ext_vector_type(2), aligned(8)));  // at element alignment
   static constexpr int n = 2;
 };
 template <>
 struct V16<float> {
-  using t = float4;
+  typedef float u __attribute__((ext_vector_type(4), aligned(4)));
   static constexpr int n = 4;
 };
 
 constexpr int TS = 256;  // threads of the row-streaming product
+// Row products of up to this many elements split each row's list over four waves (k_spmm):
+// norb=18, 239^2 strings 26 -> 9 us a product, norb=12, 495^2 19 -> 8; at norb=26, 1,400^2
+// (beyond) the plain form fills the chip.
+constexpr int64_t SPMM_KS_MAX = 1 << 20;
 constexpr int SPMM_U = 4;  // table entries gathered per step of the row product
 
 // rows per workgroup of the row product: FP64 one row of 512 columns, FP32 four rows (one
@@ -56,7 +60,16 @@ constexpr int spmm_rows() {
 // that XCD's L2.  Measured on one GPU against one 1,024-column row per FP32 workgroup, four
 // rows of 256 columns take 3-4 % less time per pass; for FP64 four rows of 128 columns take
 // 4-11 % more than one row of 512, and 2 or 8 rows, or 8 entries per step, were slower.
-template <class T, bool DIAG, bool VECTOR, bool ZG>
+//
+// A lane's VN columns are one 16-byte load at the element's own alignment (rows of an odd
+// length start anywhere); the lanes past the last whole vector take the row's last VN columns
+// again, with the same sums as their neighbour, so no lane leaves the vector path (ncols >= VN;
+// VECTOR is false below that).
+//
+// KS: with few rows and columns the chain of gathers of one row is the time (a row's list,
+// four entries per step, one memory latency each), so the four waves of a workgroup take one
+// row's columns together, a quarter of its list each, and their sums are added in order.
+template <class T, bool DIAG, bool VECTOR, bool ZG, bool KS>
 __global__ void __launch_bounds__(TS) k_spmm(int64_t nrows, int64_t ncols, int64_t cb, int64_t ce,
                                              const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
                                              const T* __restrict__ val, const int32_t* __restrict__ jai,
@@ -65,41 +78,47 @@ __global__ void __launch_bounds__(TS) k_spmm(int64_t nrows, int64_t ncols, int64
                                              const int32_t* __restrict__ zptr, const int32_t* __restrict__ zslot,
                                              const T* __restrict__ Z, int64_t zcols) {
   constexpr int VN = V16<T>::n;
-  using VT = typename V16<T>::t;
-  constexpr int RW = spmm_rows<T>();
-  constexpr int RT = TS / RW;  // threads per row
+  using VT = typename V16<T>::u;
+  constexpr int RW = KS ? 1 : spmm_rows<T>();
+  constexpr int RT = KS ? 64 : TS / RW;  // threads per row
   const int64_t ntl = (ce - cb + RT * VN - 1) / (RT * VN);
   const int64_t items = ntl * nrows;
   const int64_t per = ((items + RW - 1) / RW + 7) / 8;
   const int64_t bid = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;  // each XCD: a contiguous run of rows
   const int64_t item = bid * RW + (RW == 1 ? 0 : threadIdx.x / RT);
-  if (item >= items) return;  // no barrier in this kernel: a row group may leave alone
+  if (item >= items) return;  // RW > 1: no barrier in this kernel, a row group may leave alone
   const int64_t tile = item / nrows;
   const int64_t r = item - tile * nrows;
-  const int64_t c0 = cb + tile * (int64_t)(RT * VN) + (int64_t)(RW == 1 ? threadIdx.x : threadIdx.x % RT) * VN;
-  if (c0 >= ce) return;
+  const int wave = KS ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
+  int64_t c0 = cb + tile * (int64_t)(RT * VN) + (int64_t)(RT == TS ? threadIdx.x : threadIdx.x % RT) * VN;
+  const bool active = c0 < ce;
+  if (!KS && !active) return;
+  if (VECTOR) c0 = min(c0, ce - VN);
   T acc[VN];
-  const bool full = VECTOR && (c0 + VN <= ce);
-  if (DIAG) {
-    const T* h = hii + r * ncols + c0;
-    const T* x = X + r * ncols + c0;
-    if (full) {
+#pragma unroll
+  for (int k = 0; k < VN; ++k) acc[k] = T(0);
+  int64_t q = rowptr[r], q1 = rowptr[r + 1];
+  int32_t z = 0, z1 = 0;
+  if (ZG) {
+    z = zptr[r];
+    z1 = zptr[r + 1];
+  }
+  if (KS) {
+    const int64_t nq = (q1 - q + 3) / 4;
+    q = min(q1, q + wave * nq);
+    q1 = min(q1, q + nq);
+    const int32_t nz = (z1 - z + 3) / 4;
+    z = min(z1, z + wave * nz);
+    z1 = min(z1, z + nz);
+  }
+  if (VECTOR) {
+    if (DIAG && wave == 0) {
       T hv[VN], xv[VN];
-      *reinterpret_cast<VT*>(hv) = *reinterpret_cast<const VT*>(h);
-      *reinterpret_cast<VT*>(xv) = *reinterpret_cast<const VT*>(x);
+      *reinterpret_cast<VT*>(hv) = *reinterpret_cast<const VT*>(hii + r * ncols + c0);
+      *reinterpret_cast<VT*>(xv) = *reinterpret_cast<const VT*>(X + r * ncols + c0);
 #pragma unroll
       for (int k = 0; k < VN; ++k) acc[k] = hv[k] * xv[k];
-    } else {
-#pragma unroll
-      for (int k = 0; k < VN; ++k) acc[k] = (c0 + k < ce) ? h[k] * x[k] : T(0);
     }
-  } else {
-#pragma unroll
-    for (int k = 0; k < VN; ++k) acc[k] = T(0);
-  }
-  int64_t q = rowptr[r];
-  const int64_t q1 = rowptr[r + 1];
-  if (full) {
     for (; q + SPMM_U <= q1; q += SPMM_U) {
       int32_t j[SPMM_U];
       T v[SPMM_U], sg[SPMM_U], x[SPMM_U][VN], jv[SPMM_U][VN];
@@ -129,45 +148,46 @@ __global__ void __launch_bounds__(TS) k_spmm(int64_t nrows, int64_t ncols, int64
     }
     if (ZG) {
       const int64_t zc = c0 - cb;
-      int32_t s = zptr[r];
-      const int32_t s1 = zptr[r + 1];
-      for (; s + 2 <= s1; s += 2) {
-        T z0[VN], z1[VN];
-        *reinterpret_cast<VT*>(z0) = *reinterpret_cast<const VT*>(Z + (int64_t)zslot[s] * zcols + zc);
-        *reinterpret_cast<VT*>(z1) = *reinterpret_cast<const VT*>(Z + (int64_t)zslot[s + 1] * zcols + zc);
+      for (; z + 2 <= z1; z += 2) {
+        T za[VN], zb[VN];
+        *reinterpret_cast<VT*>(za) = *reinterpret_cast<const VT*>(Z + (int64_t)zslot[z] * zcols + zc);
+        *reinterpret_cast<VT*>(zb) = *reinterpret_cast<const VT*>(Z + (int64_t)zslot[z + 1] * zcols + zc);
 #pragma unroll
-        for (int k = 0; k < VN; ++k) acc[k] += z0[k] + z1[k];
+        for (int k = 0; k < VN; ++k) acc[k] += za[k] + zb[k];
       }
-      if (s < s1) {
-        T z0[VN];
-        *reinterpret_cast<VT*>(z0) = *reinterpret_cast<const VT*>(Z + (int64_t)zslot[s] * zcols + zc);
+      if (z < z1) {
+        T za[VN];
+        *reinterpret_cast<VT*>(za) = *reinterpret_cast<const VT*>(Z + (int64_t)zslot[z] * zcols + zc);
 #pragma unroll
-        for (int k = 0; k < VN; ++k) acc[k] += z0[k];
+        for (int k = 0; k < VN; ++k) acc[k] += za[k];
       }
+    }
+    if constexpr (KS) {
+      __shared__ T part[3][64][VN];
+      const int lane = threadIdx.x & 63;
+      if (wave > 0)
+#pragma unroll
+        for (int k = 0; k < VN; ++k) part[wave - 1][lane][k] = acc[k];
+      __syncthreads();
+      if (wave > 0 || !active) return;
+#pragma unroll
+      for (int w = 0; w < 3; ++w)
+#pragma unroll
+        for (int k = 0; k < VN; ++k) acc[k] += part[w][lane][k];
     }
     *reinterpret_cast<VT*>(out + r * ncols + c0) = *reinterpret_cast<VT*>(acc);
   } else {
-    for (; q < q1; ++q) {
-      const T v = val[q];
-      const int32_t p = jai[q];
-      const T sg = p < 0 ? T(-1) : T(1);
-      const T* x = X + (int64_t)col[q] * ncols + c0;
-      const T* jr = J + (int64_t)(p < 0 ? -p : p) * ncols + c0;
-#pragma unroll
-      for (int k = 0; k < VN; ++k)
-        if (c0 + k < ce) acc[k] += (v + sg * jr[k]) * x[k];
-    }
-    if (ZG) {
-      for (int32_t s = zptr[r]; s < zptr[r + 1]; ++s) {
-        const T* z = Z + (int64_t)zslot[s] * zcols + (c0 - cb);
-#pragma unroll
-        for (int k = 0; k < VN; ++k)
-          if (c0 + k < ce) acc[k] += z[k];
+    for (int k = 0; k < VN && c0 + k < ce; ++k) {
+      const int64_t c = c0 + k;
+      T a = DIAG ? hii[r * ncols + c] * X[r * ncols + c] : T(0);
+      for (int64_t e = q; e < q1; ++e) {
+        const int32_t p = jai[e];
+        a += (val[e] + (p < 0 ? T(-1) : T(1)) * J[(int64_t)(p < 0 ? -p : p) * ncols + c]) * X[(int64_t)col[e] * ncols + c];
       }
+      if (ZG)
+        for (int32_t e = z; e < z1; ++e) a += Z[(int64_t)zslot[e] * zcols + (c - cb)];
+      out[r * ncols + c] = a;
     }
-#pragma unroll
-    for (int k = 0; k < VN; ++k)
-      if (c0 + k < ce) out[r * ncols + c0 + k] = acc[k];
   }
 }
 
@@ -197,7 +217,7 @@ __global__ void __launch_bounds__(TS) k_core_prod(int64_t ncols, int64_t cb, int
                                                   T* __restrict__ Z, int64_t zcols) {
   constexpr int VN = V16<T>::n;
   constexpr int XB = CORE_XB;
-  using VT = typename V16<T>::t;
+  using VT = typename V16<T>::u;
   __shared__ __align__(16) T cf[CORE_YC][XB];  // signed coefficients of the staged members
   __shared__ int32_t rw[CORE_YC];              // their rows
   const int64_t ntiles = (ce - cb + TS * VN - 1) / (TS * VN);
@@ -207,9 +227,10 @@ __global__ void __launch_bounds__(TS) k_core_prod(int64_t ncols, int64_t cb, int
   if (w >= ntiles * ngrp) return;  // whole workgroup: no barrier is skipped by part of it
   const int64_t tile = w / ngrp;
   const int64_t g = w - tile * ngrp;
-  const int64_t c0 = cb + tile * (TS * VN) + (int64_t)threadIdx.x * VN;
+  int64_t c0 = cb + tile * (TS * VN) + (int64_t)threadIdx.x * VN;
   const bool active = c0 < ce;  // inactive lanes still take part in the barriers
-  const bool full = VECTOR && (c0 + VN <= ce);
+  if (VECTOR) c0 = min(c0, ce - VN);  // the last columns again rather than a part of a vector
+  constexpr bool full = VECTOR;
   const int64_t zc = c0 - cb;
   for (int b = grp[g]; b < grp[g + 1]; ++b) {
     const int core = blk[b];
@@ -298,23 +319,35 @@ __global__ void __launch_bounds__(TS) k_core_prod(int64_t ncols, int64_t cb, int
 
 constexpr int TT = 64;  // transpose tile
 
-// out[c][r] = in[r][c]   (ADD: out[c][r] += in[r][c])
-template <class T, bool ADD>
+// out[c][r] = in[r][c] (ADD 1: out[c][r] += in[r][c]; 2: and add[c][r]).  Every load of a tile is
+// issued, at an index held inside the matrix, before the first is used: loads under the edge
+// conditions are waited for one by one (16 latencies per tile: 239^2 took 12 us).
+template <class T, int ADD>
 __global__ void __launch_bounds__(256) k_transpose(int64_t R, int64_t C, const T* __restrict__ in,
                                                    T* __restrict__ out, const T* __restrict__ add) {
   __shared__ T tile[TT][TT + 1];
   const int64_t r0 = (int64_t)blockIdx.y * TT, c0 = (int64_t)blockIdx.x * TT;
   const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-  for (int k = ty; k < TT; k += 4) {
-    const int64_t r = r0 + k, c = c0 + tx;
-    if (r < R && c < C) tile[k][tx] = in[r * C + c];
+  T v[TT / 4], o[TT / 4], a[TT / 4];
+#pragma unroll
+  for (int u = 0; u < TT / 4; ++u) v[u] = in[min(r0 + ty + 4 * u, R - 1) * C + min(c0 + tx, C - 1)];
+  if constexpr (ADD > 0) {
+#pragma unroll
+    for (int u = 0; u < TT / 4; ++u) {
+      const int64_t x = min(c0 + ty + 4 * u, C - 1) * R + min(r0 + tx, R - 1);
+      o[u] = out[x];
+      a[u] = ADD == 2 ? add[x] : T(0);
+    }
   }
+#pragma unroll
+  for (int u = 0; u < TT / 4; ++u) tile[ty + 4 * u][tx] = v[u];
   __syncthreads();
-  for (int k = ty; k < TT; k += 4) {
-    const int64_t c = c0 + k, r = r0 + tx;
+#pragma unroll
+  for (int u = 0; u < TT / 4; ++u) {
+    const int64_t c = c0 + ty + 4 * u, r = r0 + tx;
     if (r < R && c < C) {
-      if (ADD) out[c * R + r] += tile[tx][k] + (add ? add[c * R + r] : T(0));
-      else out[c * R + r] = tile[tx][k];
+      if constexpr (ADD > 0) out[c * R + r] = o[u] + (tile[tx][ty + 4 * u] + a[u]);
+      else out[c * R + r] = tile[tx][ty + 4 * u];
     }
   }
 }
@@ -630,37 +663,35 @@ void launch_spmm(bool diag, int64_t nrows, int64_t ncols, const SpmmTable& tb, c
   if (ce < 0) ce = ncols;
   if (nrows == 0 || ce <= cb) return;
   constexpr int VN = V16<T>::n;
-  constexpr int RW = spmm_rows<T>();
-  const int64_t ntiles = (ce - cb + TS / RW * VN - 1) / (TS / RW * VN);
+  const bool ks = nrows * (ce - cb) <= SPMM_KS_MAX && ce - cb >= VN;
+  const int RW = ks ? 1 : spmm_rows<T>(), RT = ks ? 64 : TS / RW;
+  const int64_t ntiles = (ce - cb + RT * VN - 1) / (RT * VN);
   const int64_t nblk = ((ntiles * nrows + RW - 1) / RW + 7) / 8 * 8;
   if (nblk > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
   const T* val = nullptr;
   if constexpr (sizeof(T) == 8) val = reinterpret_cast<const T*>(tb.val.p);
   else val = reinterpret_cast<const T*>(tb.val32.p);
-  const bool vec = (ncols % VN) == 0 && (cb % VN) == 0;
+  const bool vec = ce - cb >= VN;
   const int32_t* zp = ct ? ct->slot_ptr.p : nullptr;
   const int32_t* zs = ct ? ct->slot.p : nullptr;
   dim3 g((unsigned)nblk), b(TS);
-#define SBDG_SPMM(D, V, ZG)                                                                                   \
-  hipLaunchKernelGGL((k_spmm<T, D, V, ZG>), g, b, 0, st, nrows, ncols, cb, ce, tb.rowptr.p, tb.col.p, val, \
+#define SBDG_SPMM(D, V, ZG, KS)                                                                                   \
+  hipLaunchKernelGGL((k_spmm<T, D, V, ZG, KS>), g, b, 0, st, nrows, ncols, cb, ce, tb.rowptr.p, tb.col.p, val, \
                      tb.jai.p, J, X, hii, out, zp, zs, Z, zcols)
+#define SBDG_SPMM_V(D, ZG)                    \
+  do {                                        \
+    if (ks) SBDG_SPMM(D, true, ZG, true);     \
+    else if (vec) SBDG_SPMM(D, true, ZG, false); \
+    else SBDG_SPMM(D, false, ZG, false);      \
+  } while (0)
   if (ct) {
-    if (diag) {
-      if (vec) SBDG_SPMM(true, true, true);
-      else SBDG_SPMM(true, false, true);
-    } else {
-      if (vec) SBDG_SPMM(false, true, true);
-      else SBDG_SPMM(false, false, true);
-    }
+    if (diag) SBDG_SPMM_V(true, true);
+    else SBDG_SPMM_V(false, true);
   } else {
-    if (diag) {
-      if (vec) SBDG_SPMM(true, true, false);
-      else SBDG_SPMM(true, false, false);
-    } else {
-      if (vec) SBDG_SPMM(false, true, false);
-      else SBDG_SPMM(false, false, false);
-    }
+    if (diag) SBDG_SPMM_V(true, false);
+    else SBDG_SPMM_V(false, false);
   }
+#undef SBDG_SPMM_V
 #undef SBDG_SPMM
 }
 
@@ -688,7 +719,6 @@ void launch_spin(bool diag, int64_t nrows, int64_t ncols, const SpmmTable& tb, c
   if (nrows == 0 || ncols == 0) return;
   constexpr int VN = V16<T>::n;
   const int64_t zcols = core_zcols<T>(P, *ct, ncols);
-  const bool vec = (ncols % VN) == 0;
   for (int64_t cb = 0; cb < ncols; cb += zcols) {
     const int64_t ce = std::min(ncols, cb + zcols);
     if (ct->ngrp > 0) {
@@ -697,7 +727,7 @@ void launch_spin(bool diag, int64_t nrows, int64_t ncols, const SpmmTable& tb, c
       const int64_t nwg = (items + 7) / 8 * 8;
       if (nwg > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
       dim3 g((unsigned)nwg), b(TS);
-      if (vec)
+      if (ce - cb >= VN)
         hipLaunchKernelGGL((k_core_prod<T, true>), g, b, 0, st, ncols, cb, ce, ct->start.p, ct->row.p, ct->pair.p,
                            ct->blk.p, ct->blk_x0.p, ct->grp.p, ct->ngrp, W, npair, X, Z, zcols);
       else
@@ -708,7 +738,7 @@ void launch_spin(bool diag, int64_t nrows, int64_t ncols, const SpmmTable& tb, c
   }
 }
 
-template <class T, bool ADD>
+template <class T, int ADD>
 void launch_transpose(int64_t R, int64_t C, const T* in, T* out, hipStream_t st, const T* add = nullptr) {
   if (R == 0 || C == 0) return;
   dim3 g((unsigned)((C + TT - 1) / TT), (unsigned)((R + TT - 1) / TT));
@@ -801,7 +831,7 @@ void launch_ab(const SigmaPlan& P, const T* eri, const T* c, T* sigma, hipStream
 }  // namespace
 
 void transpose_d(int64_t R, int64_t C, const double* in, double* out, hipStream_t st) {
-  launch_transpose<double, false>(R, C, in, out, st);
+  launch_transpose<double, 0>(R, C, in, out, st);
   SBDG_CHECK(hipGetLastError());
 }
 
@@ -825,15 +855,18 @@ void sigma_apply(const SigmaPlan& P, const T* c, T* sigma, const SigmaScratch<T>
   }
   if (ev) SBDG_CHECK(hipEventRecord(ev[0], st));
   // the alpha-beta terms (LDS-bound) into their own buffer on the second stream, while the
-  // spin phases (HBM-bound) run on this one; the transpose-add joins them
+  // spin phases (HBM-bound) run on this one; the transpose-add joins them.  Below 100,000
+  // determinants the fork and join cost more than the overlap gains (239^2 strings: 86 us
+  // with it, 69 in sequence; 275^2: 95 and 89; 500 x 321: 125 and 152).
   T* sab = scr.sab;
-  if (P.st2) {
+  const bool beside = P.st2 && P.na * P.nb >= 100000;
+  if (beside) {
     SBDG_CHECK(hipEventRecord(P.fork, st));
     SBDG_CHECK(hipStreamWaitEvent(P.st2, P.fork, 0));
     launch_ab<T>(P, eri, c, sab, P.st2, 1);
     SBDG_CHECK(hipEventRecord(P.join, P.st2));
   }
-  launch_transpose<T, false>(P.na, P.nb, c, cT, st);
+  launch_transpose<T, 0>(P.na, P.nb, c, cT, st);
   if (ev) SBDG_CHECK(hipEventRecord(ev[1], st));
   const T* W;
   if constexpr (sizeof(T) == 8) W = reinterpret_cast<const T*>(P.W);
@@ -851,13 +884,13 @@ void sigma_apply(const SigmaPlan& P, const T* c, T* sigma, const SigmaScratch<T>
   if (ev) SBDG_CHECK(hipEventRecord(ev[2], st));
   launch_spin<T>(true, P.na, P.nb, *P.ma, Jb, P.ca, W, P.npair, c, hii, sigma, Z, P, st);
   if (ev) SBDG_CHECK(hipEventRecord(ev[3], st));
-  if (P.st2) {
+  if (beside) {
     SBDG_CHECK(hipStreamWaitEvent(st, P.join, 0));
     if (ev) SBDG_CHECK(hipEventRecord(ev[4], st));
-    launch_transpose<T, true>(P.nb, P.na, sT, sigma, st, sab);
+    launch_transpose<T, 2>(P.nb, P.na, sT, sigma, st, sab);
     if (ev) SBDG_CHECK(hipEventRecord(ev[5], st));
   } else {
-    launch_transpose<T, true>(P.nb, P.na, sT, sigma, st);
+    launch_transpose<T, 1>(P.nb, P.na, sT, sigma, st);
     if (ev) SBDG_CHECK(hipEventRecord(ev[4], st));
     launch_ab<T>(P, eri, c, sigma, st, 0);
     if (ev) SBDG_CHECK(hipEventRecord(ev[5], st));

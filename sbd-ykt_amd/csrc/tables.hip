@@ -790,8 +790,8 @@ void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t 
   SBDG_CHECK(hipMemcpy(e.ent.p, ent.data(), sizeof(uint32_t) * ent.size(), hipMemcpyHostToDevice));
 }
 
-void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* h_eri, CoreTable& ct,
-                 Table& direct, hipStream_t st) {
+void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* h_eri, int64_t ncols,
+                 CoreTable& ct, Table& direct, hipStream_t st) {
   ct.ncore = ct.nmem = ct.nblk = 0;
   ct.maxm = 0;
   const int64_t npp = (int64_t)nel * (nel - 1) / 2;
@@ -882,12 +882,17 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
       }
       e = f;
     }
-    // workgroups: consecutive product blocks until about CORE_WORK member rows
+    // workgroups: consecutive product blocks until about CORE_WORK member rows, fewer where
+    // the pass would then have less than CORE_WGS workgroups (a small problem's blocks one
+    // after another in a few workgroups took 84-96 us at 239^2 and 495^2 strings)
     grp.push_back(0);
-    int64_t work = 0;
+    int64_t work = 0, total_work = 0;
+    for (int32_t c : blk) total_work += start[c + 1] - start[c];
+    const int64_t tiles = std::max<int64_t>(1, (ncols + CORE_COLS - 1) / CORE_COLS);
+    const int64_t target = std::min<int64_t>(CORE_WORK, total_work * tiles / CORE_WGS);
     for (size_t q = 0; q < blk.size(); ++q) {
       work += start[blk[q] + 1] - start[blk[q]];
-      if (work >= CORE_WORK || q + 1 == blk.size()) {
+      if (work >= target || q + 1 == blk.size()) {
         grp.push_back((int32_t)(q + 1));
         work = 0;
       }
