@@ -105,7 +105,7 @@ struct sbdg_ctx {
   DBuf<double> Wp;        // antisymmetrised pair integrals
   DBuf<float> Wp32;
   DBuf<double> Zbuf;      // core-product workspace
-  AbTable ab64;     // beta singles by chunk (RDMs)
+  AbPairs abp;      // beta pairs (RDMs; built by the first RDM of a string set)
   EllTable ell;      // beta singles, ELL (alpha-beta sigma, FP64; FP32 too when the geometries agree)
   EllTable ell32;    // the FP32 ELL when its launch geometry differs (wide rows)
   bool own_ell32 = false;
@@ -251,7 +251,6 @@ void build(sbdg_ctx* c) {
     c->Vt32.alloc(std::max<size_t>(npair * npair, 1));
     build_pair_slices(c->d_eri.p, L, c->Vt.p, c->Vt32.p, c->st);
   }
-  build_ab(c->Sb, L, rdm_chunk(nb, L), c->ab64, c->st);
   build_ell(c->Sb, L, 8, c->ell, c->st);
   {
     const AbGeometry g64 = ab_geometry(nb, L, 8), g32 = ab_geometry(nb, L, 4);
@@ -265,6 +264,7 @@ void build(sbdg_ctx* c) {
   compute_hii(c->d_a.p, na, c->d_b.p, nb, L, c->core, c->d_h1.p, c->d_eri.p, c->d_hii.p, c->st);
   cast_d2f(c->d_hii.p, c->d_hii32.p, N, c->st);
   SBDG_CHECK(hipStreamSynchronize(c->st));
+  c->abp.built = false;
   c->built = true;
   c->solved = c->have_rdm = c->have_dens = false;
   c->stats = sbdg_stats{};
@@ -343,11 +343,9 @@ int64_t build_bytes(const sbdg_options& o, int L, int64_t na, int64_t nb, const 
     }
   }
   if (any_core) b += 12 * npair * npair + std::min<int64_t>(zwant, (int64_t)(o.core_gib * 1073741824.0));
-  // alpha-beta tables: RDM pack and chunk pointers; ELL entries (a group pads to its longest
+  // alpha-beta tables: ELL entries (a group pads to its longest
   // list, at most the group's whole sum, plus three rows), lane maps, stream offsets
   const int64_t Sb = nnz[2];
-  const int64_t ach = rdm_chunk(nb, L);
-  b += 4 * Sb + 4 * (nb * ((nb + ach - 1) / ach + 1) + 1);
   const AbGeometry g64 = ab_geometry(nb, L, 8), g32 = ab_geometry(nb, L, 4);
   const bool two = g64.nt != g32.nt || g64.m != g32.m || g64.s != g32.s || g64.chunk != g32.chunk;
   for (const AbGeometry& g : {g64, g32}) {
@@ -363,16 +361,27 @@ int64_t build_bytes(const sbdg_options& o, int L, int64_t na, int64_t nb, const 
 
 // Transient bytes of the RDMs beyond the resident build and the vectors (which the RDMs
 // borrow): the largest of the per-table passes, plus the outputs 2 L^2 + 4 L^4 doubles.
-int64_t rdm_bytes(int L, const int64_t* nnz) {
+int64_t rdm_bytes(int L, int64_t na, int64_t nb, const int64_t* nnz) {
   const int64_t L2 = (int64_t)L * L, L4 = L2 * L2;
-  int64_t peak = 0;
+  int64_t peak = 8 * (na * 65 + nb + 128 * L2);  // diagonal: rows' occupation sums
+  int64_t sorted = 0;                            // both spins' sorted singles stay to the end
+  const int64_t nc[2] = {nb, na};
   for (int sp = 0; sp < 2; ++sp) {
     const int64_t S = nnz[2 * sp], D = nnz[2 * sp + 1];
-    peak = std::max(peak, 8 * S + 8 * S * L + 16 * S + 16 * S + 4 * (L2 + 1));  // gram, keys, sort
-    peak = std::max(peak, 8 * D + 32 * D + 16 * D);                            // gram, keys, scan, sort
+    sorted += 8 * S;
+    const int64_t tiles = nc[sp] / 1024 + 1, segs = S / 32 + L2;
+    const int64_t d = std::min(std::max(RDM_PART_BYTES, 8 * nc[sp] * (S / 512 + 1)), 8 * nc[sp] * segs);
+    peak = std::max(peak, std::max(8 * S + 16 * S + 4 * (L2 + 1), d + 8 * tiles * S + 512 * segs + 8 * segs));
+    peak = std::max(peak, 8 * D + 32 * D + 16 * D);  // gram, keys, scan, sort
   }
-  const int64_t Sa = nnz[0];
-  peak = std::max(peak, 8 * Sa + 16 * Sa + 16 * Sa + 8 * (Sa / 32 + L2 + 1) * L2);  // alpha-beta partials
+  peak = std::max(peak, 8 * (na + 65 * nb));  // density
+  // alpha-beta: the alpha pairs (keys, sort, rows), the tiles of beta pairs and the partial
+  // sums of one batch of keys (runs: at most one per beta pair and tile)
+  const int64_t Sa = nnz[0], pairs = nnz[2] / 2, nch = (nb + AB_PAIR_COLS / 2 - 1) / (AB_PAIR_COLS / 2);
+  const int64_t tiles = nch * (nch + 1) / 2 + pairs / 1024 + 1, runs = pairs + tiles;
+  const int64_t table = 32 * tiles + 6 * (pairs + 12288 * tiles) + 8 * runs + 4 * (L2 + runs);
+  const int64_t part = std::min(std::max(RDM_PART_BYTES, 16 * runs), 16 * runs * (Sa / 32 + L2));
+  peak = std::max(peak, part) + table + sorted;
   return peak + 8 * (2 * L2 + 4 * L4);
 }
 
@@ -808,7 +817,8 @@ void rdm_or_density(sbdg_ctx* c) {
     P.da = &c->Da;
     P.sb = &c->Sb;
     P.db = &c->Db;
-    P.ab = &c->ab64;
+    if (!c->abp.built) build_ab_pairs(c->Sb, L, c->abp, c->st);
+    P.ab = &c->abp;
     if (c->opt.doubles != 1) {  // the core tables exist (built for sigma, used or not)
       P.ca = &c->Ca;
       P.cb = &c->Cb;
@@ -818,9 +828,8 @@ void rdm_or_density(sbdg_ctx* c) {
     c->have_rdm = true;
   }
   c->d_dens.alloc(2 * L);
-  c->small.alloc(std::max<size_t>(c->small.n, (size_t)(na + nb + 16)));
   DBuf<double> part;
-  part.alloc(na + nb + 1);
+  part.alloc(std::max<int64_t>(density_part(na, nb), 1));
   density(c->W.p, c->d_a.p, na, c->d_b.p, nb, L, c->d_dens.p, part.p, c->st);
   SBDG_CHECK(hipStreamSynchronize(c->st));
   c->have_dens = true;
@@ -1076,7 +1085,7 @@ int sbdg_memory_plan(const sbdg_options* o, int norb, int64_t na, int64_t nb, co
   if (!o || !nnz || !mem || !dir || !out || norb < 1 || norb > 64 || na < 0 || nb < 0) return SBDG_ERR_ARG;
   out[0] = build_bytes(*o, norb, na, nb, nnz, mem, dir);
   out[1] = davidson_bytes(*o, na * nb);
-  out[2] = rdm_bytes(norb, nnz);
+  out[2] = rdm_bytes(norb, na, nb, nnz);
   return SBDG_OK;
 }
 

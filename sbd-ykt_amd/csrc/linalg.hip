@@ -510,34 +510,45 @@ __global__ void __launch_bounds__(RT) k_rowsq(const double* __restrict__ W, int6
   if (threadIdx.x == 0) rs[ia] = v;
 }
 
-__global__ void k_colsq(const double* __restrict__ W, int64_t na, int64_t nb, double* __restrict__ cs) {
-  const int64_t ib = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+// column sums of W^2 over one of COL_PARTS row ranges: part[range*nb + ib]
+constexpr int COL_PARTS = 64;
+__global__ void __launch_bounds__(RT) k_colsq(const double* __restrict__ W, int64_t na, int64_t nb,
+                                              double* __restrict__ part) {
+  const int64_t ib = (int64_t)blockIdx.x * RT + threadIdx.x;
   if (ib >= nb) return;
+  const int64_t per = (na + COL_PARTS - 1) / COL_PARTS, a0 = min(na, blockIdx.y * per), a1 = min(na, a0 + per);
   double v = 0.0;
-  for (int64_t ia = 0; ia < na; ++ia) {
+#pragma unroll 8
+  for (int64_t ia = a0; ia < a1; ++ia) {
     const double w = W[ia * nb + ib];
     v += w * w;
   }
+  part[blockIdx.y * nb + ib] = v;
+}
+
+__global__ void __launch_bounds__(RT) k_colsum(const double* __restrict__ part, int64_t nb, double* __restrict__ cs) {
+  const int64_t ib = (int64_t)blockIdx.x * RT + threadIdx.x;
+  if (ib >= nb) return;
+  double v = 0.0;
+#pragma unroll 8
+  for (int p = 0; p < COL_PARTS; ++p) v += part[p * nb + ib];
   cs[ib] = v;
 }
 
+// workgroup 2*o + s: density of orbital o, spin s
 __global__ void __launch_bounds__(RT) k_occ(const double* __restrict__ rs, const uint64_t* __restrict__ a, int64_t na,
                                             const double* __restrict__ cs, const uint64_t* __restrict__ b,
-                                            int64_t nb, int L, double* __restrict__ dens) {
+                                            int64_t nb, double* __restrict__ dens) {
   __shared__ double sh[RT / 64];
-  for (int o = 0; o < L; ++o) {
-    double va = 0.0, vb = 0.0;
-    for (int64_t i = threadIdx.x; i < na; i += RT)
-      if ((a[i] >> o) & 1ull) va += rs[i];
-    for (int64_t i = threadIdx.x; i < nb; i += RT)
-      if ((b[i] >> o) & 1ull) vb += cs[i];
-    va = block_sum(va, sh);
-    vb = block_sum(vb, sh);
-    if (threadIdx.x == 0) {
-      dens[2 * o] = va;
-      dens[2 * o + 1] = vb;
-    }
-  }
+  const int o = blockIdx.x >> 1;
+  const bool beta = blockIdx.x & 1;
+  const double* x = beta ? cs : rs;
+  const uint64_t* str = beta ? b : a;
+  const int64_t n = beta ? nb : na;
+  double v = 0.0;
+  for (int64_t i = threadIdx.x; i < n; i += RT) v += ((str[i] >> o) & 1ull) ? x[i] : 0.0;
+  v = block_sum(v, sh);
+  if (threadIdx.x == 0) dens[blockIdx.x] = v;
 }
 
 template <int MM, class F>
@@ -744,13 +755,20 @@ void row_sumsq(const double* W, int64_t na, int64_t nb, double* d_rs, hipStream_
   SBDG_CHECK(hipGetLastError());
 }
 
+int64_t density_part(int64_t na, int64_t nb) { return na + nb + COL_PARTS * nb; }
+
 void density(const double* W, const uint64_t* a, int64_t na, const uint64_t* b, int64_t nb, int L, double* d_dens,
              double* d_part, hipStream_t st) {
   double* rs = d_part;
   double* cs = d_part + na;
+  double* part = cs + nb;
   if (na > 0) hipLaunchKernelGGL(k_rowsq, dim3((unsigned)na), dim3(RT), 0, st, W, nb, rs);
-  if (nb > 0) hipLaunchKernelGGL(k_colsq, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st, W, na, nb, cs);
-  hipLaunchKernelGGL(k_occ, dim3(1), dim3(RT), 0, st, rs, a, na, cs, b, nb, L, d_dens);
+  if (nb > 0) {
+    const unsigned g = (unsigned)((nb + RT - 1) / RT);
+    hipLaunchKernelGGL(k_colsq, dim3(g, COL_PARTS), dim3(RT), 0, st, W, na, nb, part);
+    hipLaunchKernelGGL(k_colsum, dim3(g), dim3(RT), 0, st, part, nb, cs);
+  }
+  hipLaunchKernelGGL(k_occ, dim3(2 * L), dim3(RT), 0, st, rs, a, na, cs, b, nb, d_dens);
   SBDG_CHECK(hipGetLastError());
 }
 

@@ -80,6 +80,22 @@ struct DBuf {
   DBuf& operator=(const DBuf&) = delete;
 };
 
+// A table the kernel never writes, read at wave-uniform indices: through the constant address
+// space, so that the reads are scalar loads.  (As vector loads they share a counter with the
+// other loads in flight, and using one waits for all issued before it.)
+template <class I>
+__device__ inline I uniform_at(const I* p, int64_t i) {
+  return reinterpret_cast<const __attribute__((address_space(4))) I*>(reinterpret_cast<uintptr_t>(p))[i];
+}
+
+// The lanes of each half wave that one cycle of a 16-byte LDS read serves together: the first 16
+// entries are one such group, the others the second (lanes 32-63 alike).  Each group reads 16
+// slots of 16 bytes at once; different addresses in one slot (address / 16 mod 16) take a cycle
+// each, equal addresses none.  Measured with every lane on one address but two lanes on one
+// slot, for all pairs of lanes: 4.4 clocks per read, 5.5 where the two share a group.
+constexpr int LDS16_LANE[32] = {0, 1, 2, 3, 12, 13, 14, 15, 20, 21, 22, 23, 24, 25, 26, 27,
+                                4, 5, 6, 7, 8,  9,  10, 11, 16, 17, 18, 19, 28, 29, 30, 31};
+
 // Excitation table of one string set, CSR with ket indices ascending per bra row
 // (membership and order of chemistry/tpb/helper.h:132-197).
 //  exc word (singles): bits 0-5 ket-only orbital i, 6-11 bra-only orbital a,
@@ -111,14 +127,23 @@ struct SpmmTable {
   DBuf<int32_t> jai;
 };
 
-// Packed beta singles for the alpha-beta RDM kernel: bits 0-17 ket index jb, 18-29
-// orbital pair b*L+j, bit 30 sign.  cptr[ib*(nch+1)+k] is the first entry of row ib whose
-// ket lies in column chunk k (entries ascend in jb, so chunks are contiguous runs).
-struct AbTable {
-  int nch = 0;
-  int64_t chunk = 0;
-  DBuf<uint32_t> pack;
-  DBuf<int32_t> cptr;
+// Beta pairs (columns one excitation apart, each once) in tiles for the alpha-beta RDM kernel
+// (build_ab_pairs): entry = LDS vector of the column with the upper orbital | of the other one
+// << 15 | negative sign << 30, a tile's entries ordered for the LDS and padded to nt*u; rank is
+// their place when sorted by orbital pair.  runstart lists, per tile, the first place of each
+// orbital pair's run and then the tile's number of entries (runptr delimits the tiles' lists); pairptr/pairrun list each orbital
+// pair's runs.
+constexpr int64_t AB_PAIR_COLS = 80 * 1024 / 16 - 4;         // columns of one staged alpha pair: half a CU's LDS, a multiple of 4
+constexpr int64_t RDM_PART_BYTES = (int64_t)256 << 20;  // partial sums of one batch of orbital-pair keys
+struct AbPairs {
+  bool built = false;
+  int nt = 0, u = 0, sp = 1;  // threads, pairs per thread, alpha pairs staged at once
+  int64_t maxcols = 0, ntiles = 0, nruns = 0;
+  DBuf<int4> tile;       // first column and number of columns of the tile's two chunks
+  DBuf<int64_t> entoff;
+  DBuf<uint32_t> ent;
+  DBuf<uint16_t> rank;   // place of each entry in its tile's sorted list
+  DBuf<int32_t> runptr, runstart, pairptr, pairrun;
 };
 
 // Beta singles in an ELL layout for the alpha-beta sigma kernel.  Columns are cut into
@@ -217,7 +242,6 @@ void build_occ_table(const uint64_t* d_str, int64_t n, int L, const double* d_er
 void build_pair_integrals(const double* d_eri, int L, double* W, float* W32, hipStream_t st);
 // Vt[ab_pair(a,i)*npair + ab_pair(b,j)] = (ai|bj): one alpha single's slice is contiguous
 void build_pair_slices(const double* d_eri, int L, double* Vt, float* Vt32, hipStream_t st);
-void build_ab(const Table& sb, int L, int64_t chunk, AbTable& ab, hipStream_t st);
 // prec_bytes: 8 (FP64) or 4 (FP32) -- the launch geometry depends on the accumulator size
 void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t st);
 // Launch geometry of the alpha-beta kernel: threads, columns per thread, ket-row groups staged
@@ -286,12 +310,6 @@ __host__ __device__ inline uint32_t ab_pair(uint32_t b, uint32_t j) {
   const uint32_t h = b > j ? b : j, l = b > j ? j : b;
   return h * (h - 1) / 2 + l;
 }
-// Ket chunk of the RDM's alpha-beta kernel: the chunk's FP64 values and the L*L
-// accumulators of one orbital pair fill a CU's 160 KiB of LDS.
-inline int64_t rdm_chunk(int64_t nb, int L) {
-  const int64_t ch = std::max<int64_t>(256, (int64_t)(160 * 1024 / 8) - (int64_t)L * L - 8);
-  return std::min<int64_t>(std::max<int64_t>(nb, 1), ch);
-}
 inline int64_t ab_slice_span(int L) {
   return ab_pairs(L);
 }
@@ -337,6 +355,8 @@ void rotate_impl(T* X, int64_t ldx, int m, const double* U, int ld, int mk, int6
 // symmetric eigensolve of the m x m column-major d_H (ld) on the device: ascending
 // eigenvalues in d_E, eigenvectors in the columns of d_U (ld).
 void syev_device(const double* d_H, int m, int ld, double* d_E, double* d_U, hipStream_t st);
+// d_part: density_part(na, nb) doubles of scratch
+int64_t density_part(int64_t na, int64_t nb);
 void density(const double* W, const uint64_t* a, int64_t na, const uint64_t* b, int64_t nb, int L,
              double* d_dens, double* d_part, hipStream_t st);
 // d_rs[ia] = sum_ib W[ia,ib]^2 (fixed-order block sums)
@@ -352,10 +372,11 @@ struct RdmPlan {
   const Table* da = nullptr;
   const Table* sb = nullptr;
   const Table* db = nullptr;
-  const AbTable* ab = nullptr;
+  const AbPairs* ab = nullptr;
   const CoreTable* ca = nullptr;  // larger cores of the same-spin doubles (row-pair sums by block), or null
   const CoreTable* cb = nullptr;
 };
+void build_ab_pairs(const Table& sb, int L, AbPairs& ab, hipStream_t st);
 // one[2][L^2], two[4][L^4] in the reference layout (correlation.h:194-444) from the
 // separated-convention vector W; WT: scratch of na*nb doubles (W transposed).  Bitwise
 // reproducible: every sum is taken in a fixed order or as exact integer (fixed-point) adds.

@@ -406,14 +406,6 @@ __device__ inline void ab_batch(const uint32_t (&p)[B], uint32_t off, T (&s)[AbR
   }
 }
 
-// A table the kernel never writes, read at wave-uniform indices: through the constant address
-// space, so that the reads are scalar loads.  (As vector loads they share the counter of the
-// entry prefetch, and every group's start waited for the whole of it.)
-template <class I>
-__device__ inline I uniform_at(const I* p, int64_t i) {
-  return reinterpret_cast<const __attribute__((address_space(4))) I*>(reinterpret_cast<uintptr_t>(p))[i];
-}
-
 template <class T>
 struct AbArgs {
   int64_t nb, ntiles, chunk, kbase, groups;

@@ -229,33 +229,6 @@ __global__ void k_merge(int64_t n, int L, const int64_t* __restrict__ rps, const
   }
 }
 
-__global__ void k_abpack(int64_t nnz, int L, const int32_t* __restrict__ col,
-                         const uint32_t* __restrict__ exc, uint32_t* __restrict__ pack) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= nnz) return;
-  const uint32_t e = exc[q];
-  const uint32_t j = e & 63u, b = (e >> 6) & 63u, neg = (e >> 24) & 1u;
-  pack[q] = (uint32_t)col[q] | ((b * (uint32_t)L + j) << 18) | (neg << 30);
-}
-
-// cptr[r*(nch+1)+k] = first entry of row r with ket >= k*chunk (k = 0..nch)
-__global__ void k_abchunk(int64_t n, int nch, int64_t chunk, const int64_t* __restrict__ rp,
-                          const int32_t* __restrict__ col, int32_t* __restrict__ cptr) {
-  const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (t >= n * (nch + 1)) return;
-  const int64_t r = t / (nch + 1);
-  const int k = (int)(t % (nch + 1));
-  const int64_t lim = (int64_t)k * chunk;
-  int64_t lo = rp[r], hi = rp[r + 1];
-  while (lo < hi) {
-    int64_t mid = (lo + hi) >> 1;
-    if ((int64_t)col[mid] < lim) lo = mid + 1;
-    else hi = mid;
-  }
-  cptr[t] = (int32_t)lo;
-}
-
-
 // J[(p+1)*n + r] = sum_{o in occ(s[r])} eri[p*L^2 + o*L + o]; row 0 zero
 __global__ void k_occ_table(const uint64_t* __restrict__ s, int64_t n, int L, const double* __restrict__ eri,
                             double* __restrict__ J, float* __restrict__ J32) {
@@ -474,23 +447,6 @@ void build_spmm(const Table& s, const Table& d, SpmmTable& m, int L, hipStream_t
   } else {
     SBDG_CHECK(hipMemsetAsync(m.rowptr.p, 0, sizeof(int64_t), st));
   }
-}
-
-void build_ab(const Table& sb, int L, int64_t chunk, AbTable& ab, hipStream_t st) {
-  if (sb.n > (1 << 18)) throw Error(SBDG_ERR_LIMIT, "beta string set beyond 2^18 strings");
-  ab.chunk = chunk;
-  ab.nch = (int)((sb.n + chunk - 1) / chunk);
-  if (ab.nch < 1) ab.nch = 1;
-  ab.pack.alloc(std::max<int64_t>(sb.nnz, 1));
-  ab.cptr.alloc((size_t)sb.n * (ab.nch + 1) + 1);
-  if (sb.nnz > 0)
-    hipLaunchKernelGGL(k_abpack, dim3(blocks_for(sb.nnz, 256)), dim3(256), 0, st, sb.nnz, L, sb.col.p,
-                       sb.exc.p, ab.pack.p);
-  const int64_t nt = sb.n * (ab.nch + 1);
-  if (nt > 0)
-    hipLaunchKernelGGL(k_abchunk, dim3(blocks_for(nt, 256)), dim3(256), 0, st, sb.n, ab.nch, chunk,
-                       sb.rowptr.p, sb.col.p, ab.cptr.p);
-  SBDG_CHECK(hipGetLastError());
 }
 
 // Alpha-beta launch geometry for rows of nb columns: nt threads, m columns per thread, so that

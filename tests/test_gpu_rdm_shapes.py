@@ -1,0 +1,45 @@
+"""The RDM kernels at the edges of their shapes, through the C-ABI against the oracle on the same
+vector: one to three beta strings, odd row lengths, few beta pairs (one and four alpha pairs per
+step) and many, the last row length of one column chunk and the first of two and of three, alpha
+sets with a single string, and same-spin parts on rows of one column.
+
+Bars: 1e-11 on the RDMs, their partial traces and Hermiticity (sums of at most some ten thousand
+products of a unit vector's elements: a few hundred units of 1e-16), bit-identical on repetition
+(every sum has a fixed order)."""
+import numpy as np
+import pytest
+
+import oracle
+import sbdg
+from helpers import rdm_close, rdm_invariants, workload_small
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("norb,nel,na,nb", [
+    (12, 4, 40, 1), (12, 4, 1, 40), (12, 4, 30, 2), (12, 4, 30, 3), (16, 5, 65, 129), (16, 5, 30, 638),
+    (26, 5, 25, 641), (26, 5, 20, 2001), (18, 5, 20, 5116), (18, 5, 20, 5117), (22, 5, 9, 10241), (64, 3, 50, 70),
+])
+def test_rdm_at_shape_edges(norb, nel, na, nb):
+    c = workload_small(norb, nel, nel, na, nb, 61)
+    w = np.random.default_rng(5).normal(size=na * nb)
+    w /= np.linalg.norm(w)
+    p = oracle.Problem(c["norb"], c["core"], c["h1"], c["astr"], c["bstr"], eri=c["eri"])
+    one_o, two_o = p.rdm(w)
+    for doubles in (0, 1):
+        s = sbdg.Solver(c["norb"], c["core"], c["h1"], c["eri"], c["astr"], c["bstr"], doubles=doubles, max_it=1,
+                        max_nb=2, eps=1e10, init=2, do_rdm=1)
+        s.set_vector(w)
+        s.run()
+        one, two = s.rdm()
+        print(f"norb {norb}, {na} x {nb}, doubles {doubles}: one {np.abs(one - one_o).max():.1e}, "
+              f"two {np.abs(two[[0, 3]] - two_o[[0, 3]]).max():.1e} "
+              f"{np.abs(two[1] + two[2] - two_o[1] - two_o[2]).max():.1e}", flush=True)
+        rdm_close(one, two, one_o, two_o, 1e-11, mixed_sum=True)
+        rdm_invariants(one, two, nel, nel, norb, 1e-11)
+        one2, two2 = s.rdm(compute=True)
+        assert np.array_equal(one, one2) and np.array_equal(two, two2)
+        dens = s.density()
+        assert np.abs(dens[0::2] - one[0].reshape(norb, norb).diagonal()).max() < 1e-12
+        assert np.abs(dens[1::2] - one[1].reshape(norb, norb).diagonal()).max() < 1e-12
+        s.close()
