@@ -548,17 +548,18 @@ void build_segments(const Table& sa, int64_t nb, int64_t ntiles, AbSegments& g, 
   g.part.alloc(std::max<int64_t>((int64_t)np * nb, 1));
 }
 
-// Order of the entries of the lanes of one (group, chunk) block, step by step, so that the
-// lanes of each aligned pass group (P lanes) read distinct LDS slots (S slots of the
-// element size) in both the ket-row array and the integral array; equal addresses
-// broadcast and cost nothing.  Padding (the zero slot, pair 0) may be placed at any step
-// while a lane has slack.  Greedy: at each step the lanes with least slack choose first,
+// Order of the entries of the lanes of one (group, chunk) block, step by step, so that the 16
+// lanes that a 16-byte read serves together (LDS16_LANE) read distinct LDS slots of 16 in both
+// the ket-row array and the integral array; equal addresses broadcast and cost nothing.
+// (Against 32 contiguous lanes over the 16 slots: norb=36, 20,000^2 FP64 68.1 -> 64.4 ms, FP32
+// 37.1 -> 35.8, norb=26, 2,801 x 2,749 0.91 -> 0.81.)  Padding (the zero slot, pair 0) may be
+// placed at any step while a lane has slack.  Greedy: at each step the lanes with least slack choose first,
 // each taking the entry that adds the fewest new addresses to slots already in use.
 // lists[l] holds lane l's entries (ket byte address | pair << 18 | sign << 31); out gets
 // K*64.  Slots count 16-byte LDS vectors: the pair's slice vector is the pair index, the
 // ket's is its byte address / 16.
-static void schedule_block(std::vector<std::vector<uint32_t>>& lists, int K, int P, int S, uint32_t pad,
-                           uint32_t* out) {
+static void schedule_block(std::vector<std::vector<uint32_t>>& lists, int K, uint32_t pad, uint32_t* out) {
+  constexpr int P = 16, S = 16;
   struct Use {
     uint32_t addr[8];
     int n;
@@ -579,7 +580,7 @@ static void schedule_block(std::vector<std::vector<uint32_t>>& lists, int K, int
   for (int p0 = 0; p0 < 64; p0 += P) {
     for (int e = 0; e < K; ++e) {
       for (int x = 0; x < S; ++x) uc[x].n = uv[x].n = 0;
-      for (int i = 0; i < P; ++i) order[i] = p0 + i;
+      for (int i = 0; i < P; ++i) order[i] = (p0 & 32) + LDS16_LANE[(p0 & 31) + i];
       std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return rem[a] > rem[b]; });
       for (int l : order) {
         const int slack = (K - e) - rem[l];
@@ -712,10 +713,6 @@ void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t 
   const int64_t total = soff[nstream];
   const uint32_t pad = ((uint32_t)e.kbase + (uint32_t)chunk) << 4;  // zero slot, pair 0
   std::vector<uint32_t> ent((size_t)std::max<int64_t>(total, 1), pad);
-  // pass groups of the kernel's 16-byte LDS reads, as measured on gfx950 (the alpha-beta
-  // kernel at norb=36, 20,000^2 with four candidate models; this one was fastest): 32 lanes
-  // over 16 slots of 16 bytes (256 bytes of banks)
-  const int P = 32, S = 16;
   const uint32_t kbase = (uint32_t)e.kbase;  // ket vectors follow the slice vectors
   std::vector<std::vector<uint32_t>> lists(64);
   for (int64_t g = 0; g < e.groups; ++g)
@@ -734,7 +731,7 @@ void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t 
           lst.push_back(((kbase + (uint32_t)(col[q] - j0)) << 4) | (ab_pair(b, j) << 18) | (neg << 31));
         }
       }
-      schedule_block(lists, K[g * nch + k], P, S, pad, ent.data() + base);
+      schedule_block(lists, K[g * nch + k], pad, ent.data() + base);
     }
   e.colperm.alloc(perm.size());
   SBDG_CHECK(hipMemcpy(e.colperm.p, perm.data(), sizeof(int32_t) * perm.size(), hipMemcpyHostToDevice));
