@@ -96,6 +96,15 @@ __device__ inline I uniform_at(const I* p, int64_t i) {
 constexpr int LDS16_LANE[32] = {0, 1, 2, 3, 12, 13, 14, 15, 20, 21, 22, 23, 24, 25, 26, 27,
                                 4, 5, 6, 7, 8,  9,  10, 11, 16, 17, 18, 19, 28, 29, 30, 31};
 
+// The 16 x 16 x 4 FP64 matrix instruction.  Operands: lane l holds A[l % 16][l / 16] and
+// B[l / 16][l % 16]; of the product, element q of lane l is row(q, l), column l % 16.
+struct Mfma64 {
+  typedef double acc __attribute__((ext_vector_type(4)));
+  __device__ static inline acc mad(double a, double b, acc c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+  }
+  __device__ static inline int row(int q, int lane) { return 4 * q + lane / 16; }
+};
 // Excitation table of one string set, CSR with ket indices ascending per bra row
 // (membership and order of chemistry/tpb/helper.h:132-197).
 //  exc word (singles): bits 0-5 ket-only orbital i, 6-11 bra-only orbital a,
