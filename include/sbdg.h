@@ -83,10 +83,10 @@ typedef struct {
   double t_rdm;         /* seconds: RDMs or density */
   int64_t terms;        /* structurally connected (bra, ket) pairs per sigma, diagonal included */
   int64_t nnz[4];       /* alpha singles, alpha doubles, beta singles, beta doubles */
-  int64_t core_members[2]; /* alpha, beta: memberships of the core-grouped doubles (0: the
-                              excitation-table form is used for that spin) */
-  int64_t core_direct[2];  /* alpha, beta: double pairs of cores with fewer than ten members,
-                              read directly by the row product beside the core-grouped ones */
+  int64_t core_members[2]; /* alpha, beta: memberships of the cores with ten members or more
+                              (0: the excitation-table form is used for that spin); sigma takes
+                              the largest of them through its workspace */
+  int64_t core_direct[2];  /* alpha, beta: double pairs of cores with fewer than ten members */
   int64_t mem_now;      /* device bytes the library holds when the stats are read (all
                            contexts of the process) */
   int64_t mem_peak;     /* their high-water mark since the start of the last build or run */

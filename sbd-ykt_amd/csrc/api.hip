@@ -169,8 +169,8 @@ SigmaPlan plan(sbdg_ctx* c, bool fp32) {
   P.Ja32 = c->Ja32.p;
   P.Jb = c->Jb.p;
   P.Jb32 = c->Jb32.p;
-  P.ca = c->use_ca ? &c->Ca : nullptr;
-  P.cb = c->use_cb ? &c->Cb : nullptr;
+  P.ca = c->use_ca && c->Ca.zmem ? &c->Ca : nullptr;
+  P.cb = c->use_cb && c->Cb.zmem ? &c->Cb : nullptr;
   P.W = c->Wp.p;
   P.W32 = c->Wp32.p;
   P.npair = (int64_t)c->L * (c->L - 1) / 2;
@@ -211,8 +211,8 @@ void build(sbdg_ctx* c) {
     // workspace fits core_gib; otherwise the excitation-table form
     const size_t cap = (size_t)(c->opt.core_gib * 1073741824.0);
     auto fits = [&](const CoreTable& ct) { return (size_t)ct.nmem * CORE_COLS * sizeof(double) <= cap; };
-    c->use_ca = c->opt.doubles == 2 || (c->Da.nnz > 4 * c->Ca.nmem + c->Xa.nnz && fits(c->Ca));
-    c->use_cb = c->opt.doubles == 2 || (c->Db.nnz > 4 * c->Cb.nmem + c->Xb.nnz && fits(c->Cb));
+    c->use_ca = c->opt.doubles == 2 || (c->Da.nnz > 4 * c->Ca.nmem + c->Ca.small && fits(c->Ca));
+    c->use_cb = c->opt.doubles == 2 || (c->Db.nnz > 4 * c->Cb.nmem + c->Cb.small && fits(c->Cb));
   }
   // row products: the singles with the doubles of the excitation table, or with the direct
   // pairs of the small cores when the doubles go by core
@@ -233,7 +233,7 @@ void build(sbdg_ctx* c) {
     c->Wp32.alloc(std::max<int64_t>(npair * npair, 1));
     build_pair_integrals(c->d_eri.p, L, c->Wp.p, c->Wp32.p, c->st);
     auto need = [](const CoreTable& ct, int64_t ncols) {
-      return (size_t)ct.nmem * (size_t)((ncols + CORE_COLS - 1) / CORE_COLS * CORE_COLS) * sizeof(double);
+      return (size_t)ct.zmem * (size_t)((ncols + CORE_COLS - 1) / CORE_COLS * CORE_COLS) * sizeof(double);
     };
     auto least = [](const CoreTable& ct) { return (size_t)ct.nmem * CORE_COLS * sizeof(double); };
     size_t want = 0, low = 0;
@@ -275,8 +275,8 @@ void build(sbdg_ctx* c) {
   c->stats.nnz[3] = c->Db.nnz;
   c->stats.core_members[0] = c->use_ca ? c->Ca.nmem : 0;
   c->stats.core_members[1] = c->use_cb ? c->Cb.nmem : 0;
-  c->stats.core_direct[0] = c->use_ca ? c->Xa.nnz : 0;
-  c->stats.core_direct[1] = c->use_cb ? c->Xb.nnz : 0;
+  c->stats.core_direct[0] = c->use_ca ? c->Ca.small : 0;
+  c->stats.core_direct[1] = c->use_cb ? c->Cb.small : 0;
   c->stats.terms = N + (c->Sa.nnz + c->Da.nnz) * nb + (c->Sb.nnz + c->Db.nnz) * na + c->Sa.nnz * c->Sb.nnz;
 }
 
@@ -333,12 +333,14 @@ int64_t build_bytes(const sbdg_options& o, int L, int64_t na, int64_t nb, const 
   for (int sp = 0; sp < 2; ++sp) {
     const int64_t n = ns[sp], S = nnz[2 * sp], D = nnz[2 * sp + 1];
     const bool core = mem[sp] > 0;
+    // direct pairs: those of the smaller cores and of the cores below CORE_ZMIN members
+    const int64_t X = std::min(D, dir[sp] + (CORE_ZMIN - 1) * mem[sp]);
     b += 2 * 8 * (n + 1) + 20 * (S + D);                          // singles and doubles tables
-    b += 8 * (n + 1) + 20 * (S + (core ? dir[sp] : D));          // row-product table
+    b += 8 * (2 * n + 1) + 20 * (S + (core ? X : D));          // row-product table
     b += 12 * (L2 + 1) * n;                                        // occupation tables
     if (core) {
       any_core = true;
-      b += 4 * (n + 1) + 28 * mem[sp] + 8 * (n + 1) + 16 * dir[sp];  // members, blocks, slots; direct pairs
+      b += 4 * (n + 1) + 28 * mem[sp] + 8 * (n + 1) + 16 * X;  // members, blocks, slots; direct pairs
       zwant = std::max(zwant, mem[sp] * ((nc[sp] + CORE_COLS - 1) / CORE_COLS * CORE_COLS) * 8);
     }
   }

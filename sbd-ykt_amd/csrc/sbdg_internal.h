@@ -127,6 +127,7 @@ struct Table {
 struct SpmmTable {
   int64_t n = 0, nnz = 0;
   DBuf<int64_t> rowptr;
+  DBuf<int64_t> mid;  // n: where the row's doubles start
   DBuf<int32_t> col;
   DBuf<double> val;
   DBuf<float> val32;
@@ -207,20 +208,23 @@ struct AbSegments {
 // (x, y) shares exactly one core k = x & y (two electrons fewer than x), and its element
 // in the separated order is eps_x * eps_y * W[P_x][P_y], with P_x = (a < b) the pair added
 // to k to make x, eps_x = <x| c+_a c+_b |k> and W[(A,B)][(I,J)] = (AI|BJ) - (AJ|BI)
-// (zero when the pairs overlap).  Members are stored core by core (only cores with at
-// least CORE_KMIN members); row slots list, per string, the member entries it owns.  The
-// pairs of the smaller cores (two members and up) are cheaper read directly: they go to a
-// CSR table of their own that the row-streaming product merges with the singles.
+// (zero when the pairs overlap).  Members are stored core by core, the cores of CORE_ZMIN
+// members and more first: those go through the product and its workspace (row slots list, per
+// string, the member entries it owns there).  Cores down to CORE_KMIN members follow for the
+// RDMs' Gram products.  The pairs of all cores below CORE_ZMIN (two members and up) are cheaper
+// read directly: they go to a CSR table of their own that the row-streaming product merges with
+// the singles.
 struct CoreTable {
-  int64_t ncore = 0, nmem = 0, nblk = 0;
-  int maxm = 0;
+  int64_t ncore = 0, nmem = 0, nblk = 0;  // cores and members down to CORE_KMIN, product blocks
+  int64_t zmem = 0;                       // members of the cores that go through the workspace
+  int64_t small = 0;                      // direct pairs of the cores below CORE_KMIN
   DBuf<int32_t> start;    // ncore + 1
   DBuf<int32_t> row;      // nmem
   DBuf<int32_t> pair;     // nmem: P(a,b) = b(b-1)/2 + a, bit 31 set when eps is negative
   DBuf<int32_t> blk;      // nblk: core of each product block
   DBuf<int32_t> blk_x0;   // nblk: first member of the block
   DBuf<int32_t> slot_ptr; // n + 1
-  DBuf<int32_t> slot;     // nmem
+  DBuf<int32_t> slot;     // zmem
   int64_t ngrp = 0;
   DBuf<int32_t> grp;      // ngrp + 1: product blocks of each workgroup
 };
@@ -228,12 +232,16 @@ constexpr int CORE_XB = 16;     // output members per product block
 constexpr int CORE_COLS = 512;  // column granularity of the core-product passes
 constexpr int CORE_WORK = 256;  // member rows streamed per core-product workgroup (at most, when several blocks share one)
 constexpr int CORE_WGS = 4096;  // workgroups a core pass should have before blocks are grouped
-// Smallest core taken through the workspace: a core of k members costs about 3k row
-// transfers there (member rows in, Z out, Z gathered) and at most k(k-1) read directly,
-// fewer where members' pairs overlap, and the direct reads of one core's member rows hit
-// in cache.  FP64 sigma at norb=36, 20,000^2 strings with the cut at 2 (all through the
-// workspace) / 4 / 6 / 8 / 10 / 12 / 17 members: 204.2 / 198.9 / 194.8 / 189.9 / 190.5 /
-// 191.9 / 193.0 ms.
+// Smallest core taken through the workspace.  A core of k members costs 3k row transfers there
+// (member rows in, Z out, Z gathered), of which the 2k of Z go to memory and back; read directly
+// it costs at most k(k-1), fewer where members' pairs overlap, but of k rows that the next rows
+// of the same core find in cache.  FP64 sigma with the cut at
+// 10 / 13 / 20 / 28 / 40 members: norb=36, 20,000^2 strings 136.1 / 133.1 / 132.7 / 132.9 / 132.9
+// ms; norb=26, 4,000^2 4.59 / 4.57 / 4.43 / 4.39 / 4.40; norb=36, 5,001 x 4,999 5.24 / 5.09 / 4.96 / 4.68 /
+// 4.69; norb=58, 200 x 40,000 2.65 / 2.63 / 2.55 / 2.54 / 2.84.
+constexpr int CORE_ZMIN = 28;
+// Smallest core of the RDMs' Gram products (k_core_gram): one 16-row tile filled to more than
+// half; smaller cores' pairs one by one.
 constexpr int CORE_KMIN = 10;
 
 // kernels (tables.hip)

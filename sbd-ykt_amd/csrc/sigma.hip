@@ -13,6 +13,7 @@
 // one bra row per workgroup, stages the ket row c[ja,:] in LDS chunk by chunk together
 // with the (ai|..) slice, and gathers from LDS.  Every output element has one owner.
 #include <algorithm>
+#include <type_traits>
 
 #include "sbdg_internal.h"
 
@@ -38,28 +39,28 @@ constexpr int TS = 256;  // threads of the row-streaming product
 // norb=18, 239^2 strings 26 -> 9 us a product, norb=12, 495^2 19 -> 8; at norb=26, 1,400^2
 // (beyond) the plain form fills the chip.
 constexpr int64_t SPMM_KS_MAX = 1 << 20;
-constexpr int SPMM_U = 4;  // table entries gathered per step of the row product
-
-// rows per workgroup of the row product: FP64 one row of 512 columns, FP32 four rows (one
-// wave each) of 256 columns
-template <class T>
-constexpr int spmm_rows() {
-  return sizeof(T) == 8 ? 1 : 4;
-}
+constexpr int SPMM_ROWS = 4;  // rows per workgroup, one wave each (beyond SPMM_KS_MAX)
+constexpr int SPMM_US = 4, SPMM_UD = 4, SPMM_UZ = 8;  // singles, direct pairs, Z rows in flight
+constexpr int SPMM_DB = 16;  // direct pairs summed on their own: a short chain of roundings, as a
+// core's (norb=36, 3,600 x 3,500 strings in FP32: 3.2e-7 from the exact sigma in one chain, 1.8e-7 so)
 
 // Column range [cb, ce) of one row product:
 //   out[r, c] = (DIAG ? hii*X : 0)[r, c] + sum_q (val[q] + sgn_q J[p_q][c]) X[col[q], c]
 //             + (ZG ? sum_{s in slots(r)} Z[slot[s], c - cb] : 0)
 // jai[q] = +-(p_q) selects the row of the column strings' occupation table J that carries
-// the other-spin occupation part of a single (row 0: zero, for doubles).  Z holds the
-// core-grouped doubles of the same column range (k_core_prod).  A work item is one row of
-// one column tile; tiles are outer, rows inner.  Workgroups take spmm_rows consecutive
-// items, are dealt to the 8 XCDs in turn, and workgroup L takes items from
-// (L % 8) * per + L / 8 (per = ceil(workgroups / 8)): each XCD walks a contiguous run of
-// rows, whose strings share many excitation partners, so the rows of X they read meet in
-// that XCD's L2.  Measured on one GPU against one 1,024-column row per FP32 workgroup, four
-// rows of 256 columns take 3-4 % less time per pass; for FP64 four rows of 128 columns take
-// 4-11 % more than one row of 512, and 2 or 8 rows, or 8 entries per step, were slower.
+// the other-spin occupation part of a single; the doubles (entries from mid[r] on) have none
+// and are read without it.  Z holds the core-grouped doubles of the same column range
+// (k_core_prod).  A work item is one row of one tile of 64 lanes and belongs to one wave, so the
+// row's list is read through the scalar path; tiles are outer, rows inner.  Workgroups take
+// SPMM_ROWS consecutive items, are dealt to the 8 XCDs in turn, and workgroup L takes items from
+// (L % 8) * per + L / 8 (per = ceil(workgroups / 8)): each XCD walks a contiguous run of rows,
+// whose strings share many excitation partners, so the rows of X they read meet in that XCD's
+// L2.  Bound by the rate of those gathers (two 16-byte rows a lane and single, one a direct
+// pair) and by Z, which comes from memory.  With every entry reading a row of J and FP64 rows
+// of 512 columns over four waves a sigma at norb=36, 20,000^2 strings took 146.8 ms against 136.0
+// (FP32 76.1 / 71.6; the pairs of more cores read directly, CORE_ZMIN: 132.5 and 69.7).  Lanes split into groups that take
+// entries in turn over 8, 16 or 32 lanes' columns, so that a tile's whole piece of X stays in
+// one L2, were slower (174.4, 159.5, 153.8): the gathers, not the misses, set the time.
 //
 // A lane's VN columns are one 16-byte load at the element's own alignment (rows of an odd
 // length start anywhere); the lanes past the last whole vector take the row's last VN columns
@@ -71,33 +72,32 @@ constexpr int spmm_rows() {
 // row's columns together, a quarter of its list each, and their sums are added in order.
 template <class T, bool DIAG, bool VECTOR, bool ZG, bool KS>
 __global__ void __launch_bounds__(TS) k_spmm(int64_t nrows, int64_t ncols, int64_t cb, int64_t ce,
-                                             const int64_t* __restrict__ rowptr, const int32_t* __restrict__ col,
-                                             const T* __restrict__ val, const int32_t* __restrict__ jai,
-                                             const T* __restrict__ J, const T* __restrict__ X,
-                                             const T* __restrict__ hii, T* __restrict__ out,
+                                             const int64_t* __restrict__ rowptr, const int64_t* __restrict__ mid,
+                                             const int32_t* __restrict__ col, const T* __restrict__ val,
+                                             const int32_t* __restrict__ jai, const T* __restrict__ J,
+                                             const T* __restrict__ X, const T* __restrict__ hii, T* __restrict__ out,
                                              const int32_t* __restrict__ zptr, const int32_t* __restrict__ zslot,
                                              const T* __restrict__ Z, int64_t zcols) {
   constexpr int VN = V16<T>::n;
+  constexpr int RW = KS ? 1 : SPMM_ROWS;
   using VT = typename V16<T>::u;
-  constexpr int RW = KS ? 1 : spmm_rows<T>();
-  constexpr int RT = KS ? 64 : TS / RW;  // threads per row
-  const int64_t ntl = (ce - cb + RT * VN - 1) / (RT * VN);
+  const int64_t ntl = (ce - cb + 64 * VN - 1) / (64 * VN);
   const int64_t items = ntl * nrows;
   const int64_t per = ((items + RW - 1) / RW + 7) / 8;
   const int64_t bid = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;  // each XCD: a contiguous run of rows
-  const int64_t item = bid * RW + (RW == 1 ? 0 : threadIdx.x / RT);
-  if (item >= items) return;  // RW > 1: no barrier in this kernel, a row group may leave alone
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int64_t item = KS ? bid : bid * RW + wave;
+  if (item >= items) return;  // KS: the whole workgroup; otherwise there is no barrier
   const int64_t tile = item / nrows;
   const int64_t r = item - tile * nrows;
-  const int wave = KS ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
-  int64_t c0 = cb + tile * (int64_t)(RT * VN) + (int64_t)(RT == TS ? threadIdx.x : threadIdx.x % RT) * VN;
+  int64_t c0 = cb + (tile * 64 + lane) * VN;
   const bool active = c0 < ce;
   if (!KS && !active) return;
   if (VECTOR) c0 = min(c0, ce - VN);
   T acc[VN];
 #pragma unroll
   for (int k = 0; k < VN; ++k) acc[k] = T(0);
-  int64_t q = rowptr[r], q1 = rowptr[r + 1];
+  int64_t q = rowptr[r], q1 = rowptr[r + 1], qm = mid[r];
   int32_t z = 0, z1 = 0;
   if (ZG) {
     z = zptr[r];
@@ -107,64 +107,92 @@ __global__ void __launch_bounds__(TS) k_spmm(int64_t nrows, int64_t ncols, int64
     const int64_t nq = (q1 - q + 3) / 4;
     q = min(q1, q + wave * nq);
     q1 = min(q1, q + nq);
+    qm = max(q, min(q1, qm));
     const int32_t nz = (z1 - z + 3) / 4;
     z = min(z1, z + wave * nz);
     z1 = min(z1, z + nz);
   }
   if (VECTOR) {
-    if (DIAG && wave == 0) {
+    if (DIAG && (!KS || wave == 0)) {
       T hv[VN], xv[VN];
       *reinterpret_cast<VT*>(hv) = *reinterpret_cast<const VT*>(hii + r * ncols + c0);
       *reinterpret_cast<VT*>(xv) = *reinterpret_cast<const VT*>(X + r * ncols + c0);
 #pragma unroll
       for (int k = 0; k < VN; ++k) acc[k] = hv[k] * xv[k];
     }
-    for (; q + SPMM_U <= q1; q += SPMM_U) {
-      int32_t j[SPMM_U];
-      T v[SPMM_U], sg[SPMM_U], x[SPMM_U][VN], jv[SPMM_U][VN];
+    // the entries [e, e + U) of a list, the last step's clamped into it and left out of the sum
+    const T* Xc = X + c0;
+    const T* Jc = J + c0;
+    auto singles = [&](auto tail) {
+      constexpr bool TAIL = decltype(tail)::value;
+      constexpr int U = SPMM_US;
+      T v[U], sg[U], x[U][VN], jv[U][VN];
 #pragma unroll
-      for (int u = 0; u < SPMM_U; ++u) {
-        j[u] = col[q + u];
-        v[u] = val[q + u];
-        const int32_t p = jai[q + u];
+      for (int u = 0; u < U; ++u) {
+        const int64_t e = TAIL ? min(q + u, qm - 1) : q + u;
+        const int32_t p = jai[e];
+        v[u] = val[e];
         sg[u] = p < 0 ? T(-1) : T(1);
-        *reinterpret_cast<VT*>(x[u]) = *reinterpret_cast<const VT*>(X + (int64_t)j[u] * ncols + c0);
-        *reinterpret_cast<VT*>(jv[u]) = *reinterpret_cast<const VT*>(J + (int64_t)(p < 0 ? -p : p) * ncols + c0);
+        *reinterpret_cast<VT*>(x[u]) = *reinterpret_cast<const VT*>(Xc + (int64_t)col[e] * ncols);
+        *reinterpret_cast<VT*>(jv[u]) = *reinterpret_cast<const VT*>(Jc + (int64_t)(p < 0 ? -p : p) * ncols);
       }
 #pragma unroll
-      for (int u = 0; u < SPMM_U; ++u)
+      for (int u = 0; u < U; ++u)
 #pragma unroll
-        for (int k = 0; k < VN; ++k) acc[k] += (v[u] + sg[u] * jv[u][k]) * x[u][k];
-    }
-    for (; q < q1; ++q) {
-      const T v = val[q];
-      const int32_t p = jai[q];
-      const T sg = p < 0 ? T(-1) : T(1);
-      T x[VN], jv[VN];
-      *reinterpret_cast<VT*>(x) = *reinterpret_cast<const VT*>(X + (int64_t)col[q] * ncols + c0);
-      *reinterpret_cast<VT*>(jv) = *reinterpret_cast<const VT*>(J + (int64_t)(p < 0 ? -p : p) * ncols + c0);
+        for (int k = 0; k < VN; ++k) {
+          const T s = acc[k] + (v[u] + sg[u] * jv[u][k]) * x[u][k];
+          acc[k] = !TAIL || q + u < qm ? s : acc[k];
+        }
+    };
+    auto direct = [&](auto tail, T* sum) {
+      constexpr bool TAIL = decltype(tail)::value;
+      constexpr int U = SPMM_UD;
+      T v[U], x[U][VN];
 #pragma unroll
-      for (int k = 0; k < VN; ++k) acc[k] += (v + sg * jv[k]) * x[k];
+      for (int u = 0; u < U; ++u) {
+        const int64_t e = TAIL ? min(q + u, q1 - 1) : q + u;
+        v[u] = val[e];
+        *reinterpret_cast<VT*>(x[u]) = *reinterpret_cast<const VT*>(Xc + (int64_t)col[e] * ncols);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int k = 0; k < VN; ++k) {
+          const T s = sum[k] + v[u] * x[u][k];
+          sum[k] = !TAIL || q + u < q1 ? s : sum[k];
+        }
+    };
+    for (; q + SPMM_US <= qm; q += SPMM_US) singles(std::false_type{});
+    if (q < qm) singles(std::true_type{});
+    for (q = qm; q < q1;) {
+      const int64_t qb = min(q1, q + SPMM_DB);
+      T sum[VN];
+#pragma unroll
+      for (int k = 0; k < VN; ++k) sum[k] = T(0);
+      for (; q + SPMM_UD <= qb; q += SPMM_UD) direct(std::false_type{}, sum);
+      if (q < qb) {
+        direct(std::true_type{}, sum);
+        q = qb;
+      }
+#pragma unroll
+      for (int k = 0; k < VN; ++k) acc[k] += sum[k];
     }
     if (ZG) {
-      const int64_t zc = c0 - cb;
-      for (; z + 2 <= z1; z += 2) {
-        T za[VN], zb[VN];
-        *reinterpret_cast<VT*>(za) = *reinterpret_cast<const VT*>(Z + (int64_t)zslot[z] * zcols + zc);
-        *reinterpret_cast<VT*>(zb) = *reinterpret_cast<const VT*>(Z + (int64_t)zslot[z + 1] * zcols + zc);
+      constexpr int U = SPMM_UZ;
+      const T* Zc = Z + (c0 - cb);
+      for (; z < z1; z += U) {
+        T a[U][VN];
 #pragma unroll
-        for (int k = 0; k < VN; ++k) acc[k] += za[k] + zb[k];
-      }
-      if (z < z1) {
-        T za[VN];
-        *reinterpret_cast<VT*>(za) = *reinterpret_cast<const VT*>(Z + (int64_t)zslot[z] * zcols + zc);
+        for (int u = 0; u < U; ++u)
+          *reinterpret_cast<VT*>(a[u]) = *reinterpret_cast<const VT*>(Zc + (int64_t)zslot[min(z + u, z1 - 1)] * zcols);
 #pragma unroll
-        for (int k = 0; k < VN; ++k) acc[k] += za[k];
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+          for (int k = 0; k < VN; ++k) acc[k] = z + u < z1 ? acc[k] + a[u][k] : acc[k];
       }
     }
     if constexpr (KS) {
       __shared__ T part[3][64][VN];
-      const int lane = threadIdx.x & 63;
       if (wave > 0)
 #pragma unroll
         for (int k = 0; k < VN; ++k) part[wave - 1][lane][k] = acc[k];
@@ -656,8 +684,8 @@ void launch_spmm(bool diag, int64_t nrows, int64_t ncols, const SpmmTable& tb, c
   if (nrows == 0 || ce <= cb) return;
   constexpr int VN = V16<T>::n;
   const bool ks = nrows * (ce - cb) <= SPMM_KS_MAX && ce - cb >= VN;
-  const int RW = ks ? 1 : spmm_rows<T>(), RT = ks ? 64 : TS / RW;
-  const int64_t ntiles = (ce - cb + RT * VN - 1) / (RT * VN);
+  const int RW = ks ? 1 : SPMM_ROWS;
+  const int64_t ntiles = (ce - cb + 64 * VN - 1) / (64 * VN);
   const int64_t nblk = ((ntiles * nrows + RW - 1) / RW + 7) / 8 * 8;
   if (nblk > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
   const T* val = nullptr;
@@ -668,8 +696,8 @@ void launch_spmm(bool diag, int64_t nrows, int64_t ncols, const SpmmTable& tb, c
   const int32_t* zs = ct ? ct->slot.p : nullptr;
   dim3 g((unsigned)nblk), b(TS);
 #define SBDG_SPMM(D, V, ZG, KS)                                                                                   \
-  hipLaunchKernelGGL((k_spmm<T, D, V, ZG, KS>), g, b, 0, st, nrows, ncols, cb, ce, tb.rowptr.p, tb.col.p, val, \
-                     tb.jai.p, J, X, hii, out, zp, zs, Z, zcols)
+  hipLaunchKernelGGL((k_spmm<T, D, V, ZG, KS>), g, b, 0, st, nrows, ncols, cb, ce, tb.rowptr.p, tb.mid.p, \
+                     tb.col.p, val, tb.jai.p, J, X, hii, out, zp, zs, Z, zcols)
 #define SBDG_SPMM_V(D, ZG)                    \
   do {                                        \
     if (ks) SBDG_SPMM(D, true, ZG, true);     \
@@ -692,8 +720,8 @@ void launch_spmm(bool diag, int64_t nrows, int64_t ncols, const SpmmTable& tb, c
 template <class T>
 int64_t core_zcols(const SigmaPlan& P, const CoreTable& ct, int64_t ncols) {
   const int64_t whole = (ncols + CORE_COLS - 1) / CORE_COLS * CORE_COLS;
-  if (ct.nmem == 0) return whole;
-  const int64_t fit = (int64_t)(P.zbytes / (sizeof(T) * (size_t)ct.nmem)) / CORE_COLS * CORE_COLS;
+  if (ct.zmem == 0) return whole;
+  const int64_t fit = (int64_t)(P.zbytes / (sizeof(T) * (size_t)ct.zmem)) / CORE_COLS * CORE_COLS;
   if (fit < CORE_COLS) throw Error(SBDG_ERR_LIMIT, "core workspace too small");
   return std::min(fit, whole);
 }

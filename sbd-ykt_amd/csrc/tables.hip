@@ -205,13 +205,14 @@ __global__ void k_merge(int64_t n, int L, const int64_t* __restrict__ rps, const
                         const uint32_t* __restrict__ es,
                         const int64_t* __restrict__ rpd, const int32_t* __restrict__ cd,
                         const double* __restrict__ vd, const float* __restrict__ vd32,
-                        int64_t* __restrict__ rpm, int32_t* __restrict__ cm,
+                        int64_t* __restrict__ rpm, int64_t* __restrict__ mid, int32_t* __restrict__ cm,
                         double* __restrict__ vm, float* __restrict__ vm32, int32_t* __restrict__ jm) {
   const int64_t r = blockIdx.x;
   const int64_t b = rps[r] + rpd[r];
   const int64_t ns = rps[r + 1] - rps[r], nd = rpd[r + 1] - rpd[r];
   if (threadIdx.x == 0) {
     rpm[r] = b;
+    mid[r] = b + ns;
     if (r == n - 1) rpm[n] = rps[n] + rpd[n];
   }
   for (int64_t k = threadIdx.x; k < ns + nd; k += blockDim.x) {
@@ -417,11 +418,13 @@ void build_spmm(const Table& s, const Table& d, SpmmTable& m, int L, hipStream_t
     m.n = s.n;
     m.nnz = s.nnz;
     m.rowptr.alloc(m.n + 1);
+    m.mid.alloc(std::max<int64_t>(m.n, 1));
     m.col.alloc(std::max<int64_t>(m.nnz, 1));
     m.val.alloc(std::max<int64_t>(m.nnz, 1));
     m.val32.alloc(std::max<int64_t>(m.nnz, 1));
     m.jai.alloc(std::max<int64_t>(m.nnz, 1));
     SBDG_CHECK(hipMemcpyAsync(m.rowptr.p, s.rowptr.p, sizeof(int64_t) * (m.n + 1), hipMemcpyDeviceToDevice, st));
+    SBDG_CHECK(hipMemcpyAsync(m.mid.p, s.rowptr.p + 1, sizeof(int64_t) * m.n, hipMemcpyDeviceToDevice, st));
     if (m.nnz) {
       SBDG_CHECK(hipMemcpyAsync(m.col.p, s.col.p, sizeof(int32_t) * m.nnz, hipMemcpyDeviceToDevice, st));
       SBDG_CHECK(hipMemcpyAsync(m.val.p, s.val.p, sizeof(double) * m.nnz, hipMemcpyDeviceToDevice, st));
@@ -435,14 +438,15 @@ void build_spmm(const Table& s, const Table& d, SpmmTable& m, int L, hipStream_t
   m.n = s.n;
   m.nnz = s.nnz + d.nnz;
   m.rowptr.alloc(m.n + 1);
+  m.mid.alloc(std::max<int64_t>(m.n, 1));
   m.col.alloc(std::max<int64_t>(m.nnz, 1));
   m.val.alloc(std::max<int64_t>(m.nnz, 1));
   m.val32.alloc(std::max<int64_t>(m.nnz, 1));
   m.jai.alloc(std::max<int64_t>(m.nnz, 1));
   if (m.n > 0) {
     hipLaunchKernelGGL(k_merge, dim3((unsigned)m.n), dim3(TB), 0, st, m.n, L, s.rowptr.p, s.col.p, s.val.p,
-                       s.val32.p, s.exc.p, d.rowptr.p, d.col.p, d.val.p, d.val32.p, m.rowptr.p, m.col.p, m.val.p,
-                       m.val32.p, m.jai.p);
+                       s.val32.p, s.exc.p, d.rowptr.p, d.col.p, d.val.p, d.val32.p, m.rowptr.p, m.mid.p, m.col.p,
+                       m.val.p, m.val32.p, m.jai.p);
     SBDG_CHECK(hipGetLastError());
   } else {
     SBDG_CHECK(hipMemsetAsync(m.rowptr.p, 0, sizeof(int64_t), st));
@@ -745,8 +749,7 @@ void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t 
 
 void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* h_eri, int64_t ncols,
                  CoreTable& ct, Table& direct, hipStream_t st) {
-  ct.ncore = ct.nmem = ct.nblk = 0;
-  ct.maxm = 0;
+  ct.ncore = ct.nmem = ct.zmem = ct.small = ct.nblk = 0;
   const int64_t npp = (int64_t)nel * (nel - 1) / 2;
   const int64_t total = n * npp;
   std::vector<int32_t> start(1, 0), row, pair, blk, blk_x0, grp, slot_ptr(n + 1, 0), slot;
@@ -756,12 +759,15 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
     double v;
   };
   std::vector<Direct> dp;
-  auto unpair = [](int P, int& lo, int& hi) {
-    int b = 1;
-    while ((b + 1) * b / 2 <= P) ++b;
-    hi = b;
-    lo = P - b * (b - 1) / 2;
-  };
+  // orbitals of every pair index, and their bits
+  std::vector<int8_t> plo, phi;
+  std::vector<uint64_t> pbits;
+  for (int b = 1; b < L; ++b)
+    for (int a = 0; a < b; ++a) {
+      plo.push_back((int8_t)a);
+      phi.push_back((int8_t)b);
+      pbits.push_back((1ull << a) | (1ull << b));
+    }
   auto eri4h = [&](int p, int q, int r, int t) { return h_eri[(((int64_t)p * L + q) * L + r) * L + t]; };
   if (total > 0) {
     if (total >= (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "too many core memberships");
@@ -786,54 +792,73 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
     // keep, core by core, the members whose pair is disjoint from some other member's pair:
     // any other member is a single excitation away (or the same string), contributes
     // nothing and receives nothing.  Radix sort is stable: members ascend by string.
-    auto pair_mask = [](uint64_t v) {
-      const int P = (int)((v >> 32) & 0x7FFFFFFFull);
-      int b = 1;
-      while ((b + 1) * b / 2 <= P) ++b;
-      const int a = P - b * (b - 1) / 2;
-      return (1ull << a) | (1ull << b);
+    // Cores of CORE_ZMIN members and more come first: the product goes over those, the RDMs'
+    // over all that are kept.
+    struct Member {
+      uint64_t bits;
+      int32_t row, pair;  // pair as in CoreTable
     };
-    std::vector<uint64_t> masks;
-    std::vector<int64_t> keep;
+    std::vector<Member> all, keep, mids;
+    std::vector<int32_t> midsize;
+    auto push = [&](const Member* q, int64_t m) {
+      for (int64_t x = 0; x < m; ++x) {
+        row.push_back(q[x].row);
+        pair.push_back(q[x].pair);
+      }
+      start.push_back((int32_t)row.size());
+    };
     for (int64_t e = 0; e < total;) {
       int64_t f = e + 1;
       while (f < total && hk[f] == hk[e]) ++f;
-      masks.clear();
+      if (f - e < 2) {
+        e = f;
+        continue;
+      }
+      all.clear();
       keep.clear();
-      for (int64_t q = e; q < f; ++q) masks.push_back(pair_mask(hv[q]));
-      for (int64_t x = 0; x < f - e; ++x)
-        for (int64_t y = 0; y < f - e; ++y)
-          if ((masks[x] & masks[y]) == 0) {
-            keep.push_back(e + x);
+      for (int64_t q = e; q < f; ++q) {
+        const int32_t P = (int32_t)((hv[q] >> 32) & 0x7FFFFFFFull);
+        all.push_back({pbits[P], (int32_t)(hv[q] & 0xFFFFFFFFull), P | (int32_t)((hv[q] >> 63) << 31)});
+      }
+      for (const Member& x : all)
+        for (const Member& y : all)
+          if ((x.bits & y.bits) == 0) {
+            keep.push_back(x);
             break;
           }
       const int64_t m = (int64_t)keep.size();
-      if (m >= 2 && m < CORE_KMIN) {
-        for (int64_t x = 0; x < m; ++x)
-          for (int64_t y = 0; y < m; ++y) {
-            const uint64_t vx = hv[keep[x]], vy = hv[keep[y]];
-            if (x == y || (pair_mask(vx) & pair_mask(vy))) continue;  // W = 0
-            int A, B, I, J;
-            unpair((int)((vx >> 32) & 0x7FFFFFFFull), A, B);
-            unpair((int)((vy >> 32) & 0x7FFFFFFFull), I, J);
+      if (m >= 2 && m < CORE_ZMIN) {
+        const size_t before = dp.size();
+        for (const Member& x : keep)
+          for (const Member& y : keep) {
+            if (x.bits & y.bits) continue;  // W = 0 (and x == y)
+            const int Px = x.pair & 0x7FFFFFFF, Py = y.pair & 0x7FFFFFFF;
+            const int A = plo[Px], B = phi[Px], I = plo[Py], J = phi[Py];
             double v = eri4h(A, I, B, J) - eri4h(A, J, B, I);
-            if ((vx >> 63) != (vy >> 63)) v = -v;
-            dp.push_back({(int32_t)(vx & 0xFFFFFFFFull), (int32_t)(vy & 0xFFFFFFFFull), v});
+            if ((x.pair < 0) != (y.pair < 0)) v = -v;
+            dp.push_back({x.row, y.row, v});
           }
+        if (m < CORE_KMIN) {
+          ct.small += (int64_t)(dp.size() - before);
+        } else {
+          mids.insert(mids.end(), keep.begin(), keep.end());
+          midsize.push_back((int32_t)m);
+        }
       } else if (m >= 2) {
         const int32_t c = (int32_t)(start.size() - 1);
         for (int64_t x0 = 0; x0 < m; x0 += CORE_XB) {
           blk.push_back(c);
           blk_x0.push_back((int32_t)x0);
         }
-        for (int64_t q : keep) {
-          row.push_back((int32_t)(hv[q] & 0xFFFFFFFFull));
-          pair.push_back((int32_t)((hv[q] >> 32) & 0x7FFFFFFFull) | (int32_t)((hv[q] >> 63) << 31));
-        }
-        start.push_back((int32_t)row.size());
-        ct.maxm = std::max<int>(ct.maxm, (int)m);
+        push(keep.data(), m);
       }
       e = f;
+    }
+    ct.zmem = (int64_t)row.size();
+    const Member* next = mids.data();
+    for (int32_t m : midsize) {
+      push(next, m);
+      next += m;
     }
     // workgroups: consecutive product blocks until about CORE_WORK member rows, fewer where
     // the pass would then have less than CORE_WGS workgroups (a small problem's blocks one
@@ -851,11 +876,11 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
       }
     }
     // per-string slots (counting sort by row)
-    for (int32_t r : row) ++slot_ptr[r + 1];
+    for (int64_t q = 0; q < ct.zmem; ++q) ++slot_ptr[row[q] + 1];
     for (int64_t r = 0; r < n; ++r) slot_ptr[r + 1] += slot_ptr[r];
-    slot.resize(row.size());
+    slot.resize(ct.zmem);
     std::vector<int32_t> fillp(slot_ptr.begin(), slot_ptr.end() - 1);
-    for (size_t q = 0; q < row.size(); ++q) slot[fillp[row[q]]++] = (int32_t)q;
+    for (int64_t q = 0; q < ct.zmem; ++q) slot[fillp[row[q]]++] = (int32_t)q;
   }
   // the direct pairs as a CSR table (rows ascending; any order inside a row)
   {

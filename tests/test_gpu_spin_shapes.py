@@ -51,3 +51,15 @@ def test_core_pass_of_one_column():
     assert members > 0
     s = check(case, doubles=2, core_gib=(members * 512 * 8 + 4096) / 2**30)
     s.close()
+
+
+@pytest.mark.parametrize("norb,nb,capped", [(10, 129, False), (11, 203, False), (12, 65, False), (13, 1025, True)])
+def test_core_sizes_around_the_workspace_cut(norb, nb, capped):
+    """All alpha strings of five electrons: cores of 21, 28, 36 and 45 members, either side of
+    the size from which they go through the workspace (28), and a last pass of one column."""
+    case = workload_small(norb, 5, 5, 0, nb, 59)
+    s = check(case, doubles=2)
+    members = max(s.stats()["core_members"])
+    s.close()
+    if capped:
+        check(case, doubles=2, core_gib=(members * 512 * 8 + 4096) / 2**30).close()
