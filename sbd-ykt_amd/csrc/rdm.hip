@@ -863,15 +863,15 @@ __global__ void k_backward(int L, const double* __restrict__ one, const double* 
 inline unsigned nb_for(int64_t n, int t) { return (unsigned)std::max<int64_t>(1, (n + t - 1) / t); }
 
 // sort (key, index) pairs; returns sorted keys/indices in the out buffers
-void sort_pairs(int64_t n, DBuf<uint32_t>& keys, DBuf<int32_t>& idx, DBuf<uint32_t>& keys_out,
-                DBuf<int32_t>& idx_out, int end_bit, hipStream_t st) {
+void sort_pairs(int64_t n, WBuf<uint32_t>& keys, WBuf<int32_t>& idx, WBuf<uint32_t>& keys_out,
+                WBuf<int32_t>& idx_out, int end_bit, Arena& ar, hipStream_t st) {
   keys_out.alloc(std::max<int64_t>(n, 1));
   idx_out.alloc(std::max<int64_t>(n, 1));
   if (n == 0) return;
   size_t tmp = 0;
   SBDG_CHECK(hipcub::DeviceRadixSort::SortPairs(nullptr, tmp, keys.p, keys_out.p, idx.p, idx_out.p, (int)n, 0,
                                                 end_bit, st));
-  DBuf<unsigned char> t;
+  WBuf<unsigned char> t(ar);
   t.alloc(tmp + 1);
   SBDG_CHECK(hipcub::DeviceRadixSort::SortPairs(t.p, tmp, keys.p, keys_out.p, idx.p, idx_out.p, (int)n, 0, end_bit,
                                                 st));
@@ -887,17 +887,18 @@ int bits_for(uint64_t v) {
 // The singles of one spin sorted by key: pia/pja as k_alpha_pairs writes them, hk[key] the
 // first of key (host).  nkey keys (a, i) with a > i hold pairs.
 struct SortedSingles {
-  DBuf<int32_t> pia, pja;
+  explicit SortedSingles(Arena& ar) : pia(ar), pja(ar) {}
+  WBuf<int32_t> pia, pja;
   std::vector<int32_t> hk;
 };
 
-void sort_singles(const Table& t, int L, SortedSingles& ss, hipStream_t st) {
+void sort_singles(const Table& t, int L, SortedSingles& ss, Arena& ar, hipStream_t st) {
   const int L2 = L * L;
   ss.hk.assign(L2 + 1, 0);
   if (t.nnz == 0) return;
-  DBuf<int64_t> rowof;
-  DBuf<uint32_t> keys, ks;
-  DBuf<int32_t> idx, perm, kseg;
+  WBuf<int64_t> rowof(ar);
+  WBuf<uint32_t> keys(ar), ks(ar);
+  WBuf<int32_t> idx(ar), perm(ar), kseg(ar);
   rowof.alloc(t.nnz);
   keys.alloc(t.nnz);
   idx.alloc(t.nnz);
@@ -906,7 +907,7 @@ void sort_singles(const Table& t, int L, SortedSingles& ss, hipStream_t st) {
   kseg.alloc(L2 + 1);
   hipLaunchKernelGGL(k_rowof, dim3((unsigned)t.n), dim3(256), 0, st, t.n, t.rowptr.p, rowof.p);
   hipLaunchKernelGGL(k_single_keys, dim3(nb_for(t.nnz, 256)), dim3(256), 0, st, t.nnz, L, t.exc.p, keys.p, idx.p);
-  sort_pairs(t.nnz, keys, idx, ks, perm, bits_for((uint64_t)L2), st);
+  sort_pairs(t.nnz, keys, idx, ks, perm, bits_for((uint64_t)L2), ar, st);
   hipLaunchKernelGGL(k_alpha_pairs, dim3(nb_for(t.nnz, 256)), dim3(256), 0, st, t.nnz, perm.p, rowof.p, t.col.p,
                      t.exc.p, ss.pia.p, ss.pja.p);
   hipLaunchKernelGGL(k_keyseg, dim3(nb_for(L2 + 1, 256)), dim3(256), 0, st, t.nnz, L2, ks.p, kseg.p);
@@ -920,7 +921,8 @@ struct KeySegments {
   std::vector<int32_t> keys, krange, kseg, segs;
   std::vector<std::pair<size_t, size_t>> batch;
   int64_t widest = 0;  // segments of the largest batch
-  DBuf<int32_t> dkeys, dkrange, dkseg, dsegs;
+  WBuf<int32_t> dkeys, dkrange, dkseg, dsegs;
+  explicit KeySegments(Arena& ar) : dkeys(ar), dkrange(ar), dkseg(ar), dsegs(ar) {}
 };
 
 void key_segments(const std::vector<int32_t>& hk, int L, int64_t len, int64_t most, KeySegments& K, hipStream_t st) {
@@ -943,7 +945,7 @@ void key_segments(const std::vector<int32_t>& hk, int L, int64_t len, int64_t mo
     K.widest = std::max<int64_t>(K.widest, K.kseg[f] - K.kseg[k]);
     k = f;
   }
-  auto up = [&](DBuf<int32_t>& d, const std::vector<int32_t>& h) {
+  auto up = [&](WBuf<int32_t>& d, const std::vector<int32_t>& h) {
     d.alloc(std::max<size_t>(h.size(), 1));
     if (!h.empty())
       SBDG_CHECK(hipMemcpyAsync(d.p, h.data(), sizeof(int32_t) * h.size(), hipMemcpyHostToDevice, st));
@@ -956,14 +958,15 @@ void key_segments(const std::vector<int32_t>& hk, int L, int64_t len, int64_t mo
 
 // singles of one spin: pair sums by key segment, their occupation parts, then key owners
 void singles_part(const Table& t, const SortedSingles& ss, int L, int s, const double* X, int64_t ncols,
-                  const uint64_t* rstr, const uint64_t* cstr, double* one, double* two, hipStream_t st) {
+                  const uint64_t* rstr, const uint64_t* cstr, double* one, double* two, Arena& ar,
+                  hipStream_t st) {
   if (t.nnz == 0) return;
   const int NV = ncols >= 2 ? 2 : 1;
   const int64_t tw = (int64_t)RT * NV * PSU, ntiles = (ncols + tw - 1) / tw;
   const int64_t len = std::min<int64_t>(PSEG, std::max<int64_t>(16, t.nnz / 2 * ntiles / 4096));
-  KeySegments K;
+  KeySegments K(ar);
   key_segments(ss.hk, L, len, std::max<int64_t>(1, RDM_PART_BYTES / (8 * ncols)), K, st);
-  DBuf<double> D, gpart, occ;
+  WBuf<double> D(ar), gpart(ar), occ(ar);
   D.alloc((size_t)(K.widest * ncols));
   gpart.alloc((size_t)(ntiles * t.nnz));
   occ.alloc(K.segs.size() / 2 * 64);
@@ -989,8 +992,8 @@ void singles_part(const Table& t, const SortedSingles& ss, int L, int s, const d
 // cores, when sigma built them), by pair for the rest of the entries above the diagonal,
 // then mirrored to the entries below it.
 void doubles_gram(const Table& t, const CoreTable* ct, const uint64_t* strs, const double* X, int64_t ncols,
-                  double* g, hipStream_t st) {
-  DBuf<unsigned char> done;
+                  double* g, Arena& ar, hipStream_t st) {
+  WBuf<unsigned char> done(ar);
   done.alloc(t.nnz);
   SBDG_CHECK(hipMemsetAsync(done.p, 0, t.nnz, st));
   if (ct && ct->ncore > 0) {
@@ -1005,7 +1008,7 @@ void doubles_gram(const Table& t, const CoreTable* ct, const uint64_t* strs, con
       for (int bi = 0; bi < nbk; ++bi)
         for (int bj = bi; bj < nbk; ++bj) items[w].push_back(make_int4((int)k, bi, bj, 0));
     }
-    DBuf<int4> ditems[2];
+    WBuf<int4> ditems[2] = {WBuf<int4>(ar), WBuf<int4>(ar)};
     for (int w = 0; w < 2; ++w) {
       if (items[w].empty()) continue;
       ditems[w].alloc(items[w].size());
@@ -1022,8 +1025,8 @@ void doubles_gram(const Table& t, const CoreTable* ct, const uint64_t* strs, con
     SBDG_CHECK(hipGetLastError());
     SBDG_CHECK(hipStreamSynchronize(st));  // the item lists on the host stay alive until here
   }
-  DBuf<int32_t> flag, pos, qlist;
-  DBuf<int64_t> lptr;
+  WBuf<int32_t> flag(ar), pos(ar), qlist(ar);
+  WBuf<int64_t> lptr(ar);
   flag.alloc(t.nnz);
   pos.alloc(t.nnz);
   qlist.alloc(t.nnz);
@@ -1031,7 +1034,7 @@ void doubles_gram(const Table& t, const CoreTable* ct, const uint64_t* strs, con
   hipLaunchKernelGGL(k_pair_flags, dim3((unsigned)t.n), dim3(RT), 0, st, t.rowptr.p, t.col.p, done.p, flag.p);
   size_t tmp = 0;
   SBDG_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, flag.p, pos.p, (int)t.nnz, st));
-  DBuf<unsigned char> tb;
+  WBuf<unsigned char> tb(ar);
   tb.alloc(tmp + 1);
   SBDG_CHECK(hipcub::DeviceScan::ExclusiveSum(tb.p, tmp, flag.p, pos.p, (int)t.nnz, st));
   hipLaunchKernelGGL(k_pair_list, dim3(nb_for(t.nnz, 256)), dim3(256), 0, st, t.nnz, flag.p, pos.p, qlist.p);
@@ -1049,23 +1052,23 @@ void doubles_gram(const Table& t, const CoreTable* ct, const uint64_t* strs, con
 }
 
 void doubles_part(const Table& t, int L, int s, const double* X, int64_t ncols, const CoreTable* ct,
-                  const uint64_t* strs, double* two, hipStream_t st) {
+                  const uint64_t* strs, double* two, Arena& ar, hipStream_t st) {
   if (t.nnz == 0) return;
-  DBuf<double> g;
+  WBuf<double> g(ar);
   g.alloc(t.nnz);
-  doubles_gram(t, ct, strs, X, ncols, g.p, st);
-  DBuf<uint32_t> keys, ks;
-  DBuf<int32_t> idx, perm, flag, pos, seg;
+  doubles_gram(t, ct, strs, X, ncols, g.p, ar, st);
+  WBuf<uint32_t> keys(ar), ks(ar);
+  WBuf<int32_t> idx(ar), perm(ar), flag(ar), pos(ar), seg(ar);
   keys.alloc(t.nnz);
   idx.alloc(t.nnz);
   hipLaunchKernelGGL(k_double_keys, dim3(nb_for(t.nnz, 256)), dim3(256), 0, st, t.nnz, L, t.exc.p, keys.p, idx.p);
-  sort_pairs(t.nnz, keys, idx, ks, perm, bits_for((uint64_t)L * L * L * L), st);
+  sort_pairs(t.nnz, keys, idx, ks, perm, bits_for((uint64_t)L * L * L * L), ar, st);
   flag.alloc(t.nnz);
   pos.alloc(t.nnz);
   hipLaunchKernelGGL(k_flag, dim3(nb_for(t.nnz, 256)), dim3(256), 0, st, t.nnz, ks.p, flag.p);
   size_t tmp = 0;
   SBDG_CHECK(hipcub::DeviceScan::ExclusiveSum(nullptr, tmp, flag.p, pos.p, (int)t.nnz, st));
-  DBuf<unsigned char> tb;
+  WBuf<unsigned char> tb(ar);
   tb.alloc(tmp + 1);
   SBDG_CHECK(hipcub::DeviceScan::ExclusiveSum(tb.p, tmp, flag.p, pos.p, (int)t.nnz, st));
   int32_t lastpos = 0, lastflag = 0;
@@ -1240,7 +1243,8 @@ void build_ab_pairs(const Table& sb, int L, AbPairs& ab, hipStream_t st) {
   ab.built = true;
 }
 
-void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* one, double* two, hipStream_t st) {
+void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* one, double* two, Arena& ar,
+                 hipStream_t st) {
   const int L = P.L;
   const int64_t na = P.na, nb = P.nb, N = na * nb;
   const int64_t L2 = (int64_t)L * L, L4 = L2 * L2;
@@ -1251,7 +1255,7 @@ void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* one, dou
 
   // diagonal: density correlators
   {
-    DBuf<double> rsa, Pa, rsb, Daa, Dbb, Dab, dens, part;
+    WBuf<double> rsa(ar), Pa(ar), rsb(ar), Daa(ar), Dbb(ar), Dab(ar), dens(ar), part(ar);
     rsa.alloc(na);
     Pa.alloc(na * 64);
     rsb.alloc(nb);
@@ -1285,14 +1289,14 @@ void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* one, dou
     SBDG_CHECK(hipStreamSynchronize(st));
   }
   // alpha pairs (beta spectators from the beta strings of the columns)
-  SortedSingles ssa, ssb;
-  sort_singles(*P.sa, L, ssa, st);
-  sort_singles(*P.sb, L, ssb, st);
-  singles_part(*P.sa, ssa, L, 0, W, nb, P.a, P.b, one, two, st);
-  doubles_part(*P.da, L, 0, W, nb, P.ca, P.a, two, st);
+  SortedSingles ssa(ar), ssb(ar);
+  sort_singles(*P.sa, L, ssa, ar, st);
+  sort_singles(*P.sb, L, ssb, ar, st);
+  singles_part(*P.sa, ssa, L, 0, W, nb, P.a, P.b, one, two, ar, st);
+  doubles_part(*P.da, L, 0, W, nb, P.ca, P.a, two, ar, st);
   // beta pairs on the transposed vector (alpha spectators from the alpha strings)
-  singles_part(*P.sb, ssb, L, 1, WT, na, P.b, P.a, one, two, st);
-  doubles_part(*P.db, L, 1, WT, na, P.cb, P.b, two, st);
+  singles_part(*P.sb, ssb, L, 1, WT, na, P.b, P.a, one, two, ar, st);
+  doubles_part(*P.db, L, 1, WT, na, P.cb, P.b, two, ar, st);
 
   // alpha-beta
   const Table& sa = *P.sa;
@@ -1303,9 +1307,9 @@ void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* one, dou
     int64_t longest = 0;
     for (int key = 0; key < (int)L2; ++key) longest = std::max<int64_t>(longest, ssa.hk[key + 1] - ssa.hk[key]);
     while (plen < longest && (longest + plen - 1) / plen * ab.nruns * 16 > RDM_PART_BYTES) plen *= 2;
-    KeySegments K;
+    KeySegments K(ar);
     key_segments(ssa.hk, L, plen, std::max<int64_t>(1, RDM_PART_BYTES / (16 * std::max<int64_t>(1, ab.nruns))), K, st);
-    DBuf<double> part;
+    WBuf<double> part(ar);
     part.alloc((size_t)K.widest * ab.nruns * 2);
     const bool many = ab.nt == ABR_NT;
     const size_t lds = std::max<size_t>(16 * (size_t)(many ? 2 : ab.sp) * (size_t)(ab.maxcols + 1),

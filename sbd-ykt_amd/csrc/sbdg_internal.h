@@ -80,6 +80,81 @@ struct DBuf {
   DBuf& operator=(const DBuf&) = delete;
 };
 
+// Workspace carved out of device memory that lies idle (the RDMs' out of the Davidson vectors):
+// first fit over a list of pieces, everything on one stream, which orders a piece's next use
+// after its last.  Memory not found there is allocated.
+class Arena {
+ public:
+  void add(void* p, size_t bytes) {
+    const uintptr_t a = ((uintptr_t)p + 255) & ~(uintptr_t)255, e = ((uintptr_t)p + bytes) & ~(uintptr_t)255;
+    if (p && e > a) pieces_.push_back({a, e - a, false, true});
+  }
+  void* take(size_t bytes) {  // null: no piece is large enough
+    bytes = (bytes + 255) & ~(size_t)255;
+    for (size_t k = 0; k < pieces_.size(); ++k) {
+      if (pieces_[k].used || pieces_[k].bytes < bytes) continue;
+      const Piece rest{pieces_[k].at + bytes, pieces_[k].bytes - bytes, false, false};
+      pieces_[k].bytes = bytes;
+      pieces_[k].used = true;
+      const uintptr_t at = pieces_[k].at;
+      if (rest.bytes) pieces_.insert(pieces_.begin() + (int64_t)k + 1, rest);
+      return reinterpret_cast<void*>(at);
+    }
+    return nullptr;
+  }
+  void give(void* p) {
+    for (size_t k = 0; k < pieces_.size(); ++k) {
+      if (pieces_[k].at != (uintptr_t)p) continue;
+      pieces_[k].used = false;
+      if (k + 1 < pieces_.size() && !pieces_[k + 1].used && !pieces_[k + 1].first) join(k);
+      if (k > 0 && !pieces_[k - 1].used && !pieces_[k].first) join(k - 1);
+      return;
+    }
+  }
+
+ private:
+  struct Piece {
+    uintptr_t at;
+    size_t bytes;
+    bool used, first;  // first: start of a region
+  };
+  void join(size_t k) {
+    pieces_[k].bytes += pieces_[k + 1].bytes;
+    pieces_.erase(pieces_.begin() + (int64_t)k + 1);
+  }
+  std::vector<Piece> pieces_;
+};
+
+// A buffer from the arena, or of its own where the arena has no room.
+template <class T>
+struct WBuf {
+  T* p = nullptr;
+  explicit WBuf(Arena& a) : ar(a) {}
+  void alloc(size_t count) {
+    free();
+    if (!count) return;
+    p = static_cast<T*>(ar.take(sizeof(T) * count));
+    lent = p != nullptr;
+    if (lent) return;
+    own.alloc(count);
+    p = own.p;
+  }
+  void free() {
+    if (lent) ar.give(p);
+    own.free();
+    p = nullptr;
+    lent = false;
+  }
+  ~WBuf() { free(); }
+  WBuf(const WBuf&) = delete;
+  WBuf& operator=(const WBuf&) = delete;
+
+ private:
+  Arena& ar;
+  DBuf<T> own;
+  bool lent = false;
+};
+
 // A table the kernel never writes, read at wave-uniform indices: through the constant address
 // space, so that the reads are scalar loads.  (As vector loads they share a counter with the
 // other loads in flight, and using one waits for all issued before it.)
@@ -397,7 +472,9 @@ void build_ab_pairs(const Table& sb, int L, AbPairs& ab, hipStream_t st);
 // one[2][L^2], two[4][L^4] in the reference layout (correlation.h:194-444) from the
 // separated-convention vector W; WT: scratch of na*nb doubles (W transposed).  Bitwise
 // reproducible: every sum is taken in a fixed order or as exact integer (fixed-point) adds.
-void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* d_one, double* d_two, hipStream_t st);
+// Transient buffers come out of ar where they fit.
+void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* d_one, double* d_two, Arena& ar,
+                 hipStream_t st);
 // Hellmann-Feynman gradient: dh[p*L+q] = g*(one_a+one_b)[p+L*q];
 // deri[((p*L+q)*L+r)*L+s] = g/2 * sum_blk two[blk][p + L*r + L^2*q + L^3*s]
 void rdm_backward(const double* d_one, const double* d_two, int L, double g, double* d_dh,

@@ -369,7 +369,7 @@ def _torch_function():
         def forward(ctx, h1, eri, solver: Solver, core: float = 0.0):
             solver.set_integrals(core, h1.detach().cpu().double().numpy(), eri.detach().cpu().double().numpy())
             e = solver.run()
-            solver.rdm(compute=True)
+            solver._chk(lib().sbdg_compute_rdm(solver._c))  # they stay on the device
             dh, de = solver.rdm_backward(1.0)
             ctx.dh = torch.from_numpy(dh).to(h1.device)
             ctx.de = torch.from_numpy(de).to(h1.device)

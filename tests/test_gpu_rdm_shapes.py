@@ -43,3 +43,27 @@ def test_rdm_at_shape_edges(norb, nel, na, nb):
         assert np.abs(dens[0::2] - one[0].reshape(norb, norb).diagonal()).max() < 1e-12
         assert np.abs(dens[1::2] - one[1].reshape(norb, norb).diagonal()).max() < 1e-12
         s.close()
+
+
+@pytest.mark.parametrize("norb,nel,na,nb", [(12, 4, 40, 1), (16, 5, 65, 129), (18, 5, 900, 700)])
+def test_rdm_same_bits_whatever_memory_is_idle(norb, nel, na, nb):
+    """The transient buffers come out of the idle Davidson vectors and, where those have no room,
+    from allocations: the same RDMs and gradients with a basis of 2 and of 40 vectors, and the
+    solution intact afterwards."""
+    c = workload_small(norb, nel, nel, na, nb, 67)
+    w = np.random.default_rng(6).normal(size=na * nb)
+    w /= np.linalg.norm(w)
+    got = []
+    for max_nb, precision in ((2, 0), (40, 0), (40, 1)):
+        s = sbdg.Solver(c["norb"], c["core"], c["h1"], c["eri"], c["astr"], c["bstr"], max_it=1, max_nb=max_nb,
+                        eps=1e10, init=2, do_rdm=1)
+        s.set_vector(w)
+        s.run()
+        s.set_options(precision=precision)
+        before = s.vector()
+        one, two = s.rdm(compute=True)
+        got.append((one, two, *s.rdm_backward(2.0), s.density()))
+        assert np.array_equal(s.vector(), before)
+        s.close()
+    for other in got[1:]:
+        assert all(np.array_equal(x, y) for x, y in zip(got[0], other))
