@@ -428,17 +428,25 @@ __global__ void k_rotate(T* __restrict__ X, int64_t ldx, int m, const double* __
   }
 }
 
-// cyclic Jacobi on one wave; A, V in LDS (m <= 64)
+// Jacobi eigenvalues and vectors on one wave; A, V in LDS (m <= 64).  Bound by latency: a
+// rotation is a chain of a division, two roots and LDS round trips.  The rotations of a round
+// are disjoint (m / 2 pairs, in m - 1 rounds every pair once), so their angles are found side by
+// side, a lane each, and a lane takes a 2 x 2 block of the matrix through both its rotations at
+// once: one chain and two barriers a round, where one rotation after another took as much for
+// each of the m (m - 1) / 2.  A Davidson of 18 steps at norb=24, 275^2 strings (bases up to 10):
+// 15.4 -> 13.2 ms.
 __global__ void __launch_bounds__(64) k_jacobi(const double* __restrict__ H, int m, int ld,
                                                double* __restrict__ E, double* __restrict__ U) {
   __shared__ double A[64 * 64];
   __shared__ double Vv[64 * 64];
-  __shared__ int ord[64];
+  __shared__ double cs[32], sn[32];
+  __shared__ int pi[32], qi[32], ord[64];
   const int k = threadIdx.x;
-  for (int j = 0; j < m; ++j)
-    if (k < m) {
+  const int M = (m + 1) & ~1, P = M / 2;  // an odd m gets a row that stays zero
+  for (int j = 0; j < M; ++j)
+    if (k < M) {
       const int r = k <= j ? k : j, c = k <= j ? j : k;  // upper triangle is authoritative
-      A[k + 64 * j] = H[r + ld * c];
+      A[k + 64 * j] = c < m ? H[r + ld * c] : 0.0;
       Vv[k + 64 * j] = (k == j) ? 1.0 : 0.0;
     }
   __syncthreads();
@@ -453,42 +461,56 @@ __global__ void __launch_bounds__(64) k_jacobi(const double* __restrict__ H, int
     off = wave_sum(off);
     tot = wave_sum(tot);
     if (off <= 1e-30 * tot || off == 0.0) break;
-    for (int p = 0; p < m - 1; ++p)
-      for (int q = p + 1; q < m; ++q) {
+    for (int r = 0; r < M - 1; ++r) {
+      if (k < P) {  // pair k of round r: r and the last, or the places k either side of r on the ring
+        int x = r, y = M - 1;
+        if (k > 0) {
+          x = r + k >= M - 1 ? r + k - (M - 1) : r + k;
+          y = r - k < 0 ? r - k + (M - 1) : r - k;
+        }
+        const int p = min(x, y), q = max(x, y);
         const double apq = A[p + 64 * q];
-        if (fabs(apq) < 1e-300) continue;
-        const double app = A[p + 64 * p], aqq = A[q + 64 * q];
-        const double theta = (aqq - app) / (2.0 * apq);
-        const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
-        const double c = 1.0 / sqrt(t * t + 1.0), s = t * c;
-        __syncthreads();
-        if (k < m) {
-          const double akp = A[k + 64 * p], akq = A[k + 64 * q];
-          A[k + 64 * p] = c * akp - s * akq;
-          A[k + 64 * q] = s * akp + c * akq;
+        double c = 1.0, s = 0.0;
+        if (fabs(apq) >= 1e-300) {
+          const double theta = (A[q * 65] - A[p * 65]) / (2.0 * apq);
+          const double t = (theta >= 0 ? 1.0 : -1.0) / (fabs(theta) + sqrt(theta * theta + 1.0));
+          c = 1.0 / sqrt(t * t + 1.0);
+          s = t * c;
         }
-        __syncthreads();
-        if (k < m) {
-          const double apk = A[p + 64 * k], aqk = A[q + 64 * k];
-          A[p + 64 * k] = c * apk - s * aqk;
-          A[q + 64 * k] = s * apk + c * aqk;
-          const double vkp = Vv[k + 64 * p], vkq = Vv[k + 64 * q];
-          Vv[k + 64 * p] = c * vkp - s * vkq;
-          Vv[k + 64 * q] = s * vkp + c * vkq;
-        }
-        __syncthreads();
+        pi[k] = p;
+        qi[k] = q;
+        cs[k] = c;
+        sn[k] = s;
       }
-  }
-  if (k == 0) {
-    for (int i = 0; i < m; ++i) ord[i] = i;
-    for (int i = 0; i < m; ++i) {
-      int mi = i;
-      for (int j = i + 1; j < m; ++j)
-        if (A[ord[j] * 65] < A[ord[mi] * 65]) mi = j;
-      const int t = ord[i];
-      ord[i] = ord[mi];
-      ord[mi] = t;
+      __syncthreads();
+      // the 2 x 2 block of pairs (i, j): rows rotated by i, columns by j
+      for (int e = k; e < P * P; e += 64) {
+        const int i = e % P, j = e / P;
+        const int p = pi[i], q = qi[i], u = 64 * pi[j], v = 64 * qi[j];
+        const double ci = cs[i], si = sn[i], cj = cs[j], sj = sn[j];
+        const double pu = A[p + u], pv = A[p + v], qu = A[q + u], qv = A[q + v];
+        const double pu1 = cj * pu - sj * pv, pv1 = sj * pu + cj * pv;
+        const double qu1 = cj * qu - sj * qv, qv1 = sj * qu + cj * qv;
+        A[p + u] = ci * pu1 - si * qu1;
+        A[q + u] = si * pu1 + ci * qu1;
+        A[p + v] = ci * pv1 - si * qv1;
+        A[q + v] = si * pv1 + ci * qv1;
+      }
+      for (int e = k; e < m * P; e += 64) {
+        const int row = e % m, j = e / m;
+        const int u = row + 64 * pi[j], v = row + 64 * qi[j];
+        const double vu = Vv[u], vv = Vv[v];
+        Vv[u] = cs[j] * vu - sn[j] * vv;
+        Vv[v] = sn[j] * vu + cs[j] * vv;
+      }
+      __syncthreads();
     }
+  }
+  if (k < m) {  // ascending; equal values by index
+    const double e = A[k * 65];
+    int rank = 0;
+    for (int j = 0; j < m; ++j) rank += A[j * 65] < e || (A[j * 65] == e && j < k);
+    ord[rank] = k;
   }
   __syncthreads();
   for (int j = 0; j < m; ++j) {
