@@ -8,9 +8,9 @@
 //                                        + sum_{jb in S(ib)} sb (ai|bj) c[ja,jb] ]
 //                + sum_{jb in S(ib)} sb [ sum_{k in occ(ia)} (kk|bj) ] c[ia,jb]   (alpha-beta)
 // where va, vb are the string-pair values of the excitation tables.  The alpha product
-// streams whole rows c[ja,:] (coalesced, one workgroup per row tile, no atomics); the
+// streams whole rows c[ja,:] (coalesced, one wave per row tile, no atomics); the
 // beta product is the same kernel on the transposed vector; the alpha-beta kernel owns
-// one bra row per workgroup, stages the ket row c[ja,:] in LDS chunk by chunk together
+// a segment of one bra row per workgroup, stages the ket row c[ja,:] in LDS chunk by chunk together
 // with the (ai|..) slice, and gathers from LDS.  Every output element has one owner.
 #include <algorithm>
 #include <type_traits>
@@ -58,9 +58,9 @@ constexpr int SPMM_DB = 16;  // direct pairs summed on their own: a short chain 
 // L2.  Bound by the rate of those gathers (two 16-byte rows a lane and single, one a direct
 // pair) and by Z, which comes from memory.  With every entry reading a row of J and FP64 rows
 // of 512 columns over four waves a sigma at norb=36, 20,000^2 strings took 146.8 ms against 136.0
-// (FP32 76.1 / 71.6; the pairs of more cores read directly, CORE_ZMIN: 132.5 and 69.7).  Lanes split into groups that take
-// entries in turn over 8, 16 or 32 lanes' columns, so that a tile's whole piece of X stays in
-// one L2, were slower (174.4, 159.5, 153.8): the gathers, not the misses, set the time.
+// (FP32 76.1 / 71.6; the pairs of more cores read directly, CORE_ZMIN: 132.5 and 69.7).  Lanes
+// split into groups that take entries in turn over 8, 16 or 32 lanes' columns, so that a tile's
+// whole piece of X stays in one L2, were slower (174.4, 159.5, 153.8).
 //
 // A lane's VN columns are one 16-byte load at the element's own alignment (rows of an odd
 // length start anywhere); the lanes past the last whole vector take the row's last VN columns
@@ -226,7 +226,10 @@ __global__ void __launch_bounds__(TS) k_spmm(int64_t nrows, int64_t ncols, int64
 // every double pair of the string set is counted exactly once, in the core it shares.
 // The block's signed coefficients and member rows are staged in LDS, CORE_YC members at a
 // time (every lane reads the same entry: broadcast), and four member rows are loaded
-// before they are used.  Each lane owns VN columns.
+// before they are used.  Each lane owns VN columns.  Bound by the member rows' misses in L2 and
+// the Z writes: norb=36, 20,000^2 strings 16.2 ms a spin (FP32 8.3), norb=26, 4,000^2 0.41.  The
+// same products on the matrix instructions, 64 members by 256 columns a workgroup, were no faster
+// (16.8, 8.1 and 0.46 ms).
 // Workgroups are dealt to the 8 XCDs in turn; workgroup L takes work item
 // w = (L % 8) * per + L / 8 (per = ceil(items / 8)), so each XCD walks one contiguous range of
 // items, and item w is column tile w / ngroups, block group w % ngroups: the blocks of one
@@ -471,8 +474,8 @@ struct AbArgs {
 // and the wave-uniform tables are scalar loads: with each ket value loaded and waited for in
 // its own exec region (as a condition on the row and the column compiles) k_ab<double> took
 // 83.9 ms at norb=36, 20,000^2 strings (FP32 45.0) and staging alone 29.6 of them; issued
-// together 69.5 (37.6), with two columns per load 68.1 (37.1); norb=26, 2,801 x 2,749: 1.56 ->
-// 0.93 ms, norb=58, 40,000^2: 318 -> 256 ms.  Rows of few columns take S groups per barrier
+// together 69.5 (37.6), with two columns per load 68.1 (37.1), with the entries ordered over the
+// lanes one LDS cycle serves 61.2 (33.9); norb=26, 2,801 x 2,749: 1.56 -> 0.80 ms.  Rows of few columns take S groups per barrier
 // (239^2 at norb=18: 25 -> 21 us at S = 4).  Cutting rows into segments of their alpha
 // singles (build_segments) took norb=18, 239^2 from 132 to 26 us and norb=58, 200 x 40,000
 // from 6.7 to 1.0 ms: the Hartree-Fock row has ten times the singles of the average row.
