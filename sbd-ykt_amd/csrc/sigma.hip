@@ -235,9 +235,15 @@ __global__ void __launch_bounds__(TS) k_spmm(int64_t nrows, int64_t ncols, int64
 // items, and item w is column tile w / ngroups, block group w % ngroups: the blocks of one
 // core are neighbours in that range and find the core's member rows in their XCD's L2.
 constexpr int CORE_YC = 128;  // members staged per step
+// Ranges of up to 128 vectors take 128 threads where there are this many groups of product
+// blocks (four a CU): half of 256 threads would only wait at the barriers.  A sigma at norb=58,
+// 200 x 40,000 strings 2.53 -> 2.40 ms, FP32 1.64 -> 1.39, norb=26, 100 x 12,000 0.51 -> 0.49.
+// With fewer groups the staging of each block is the time, and more threads share it (norb=18,
+// 239^2: 62 us with 256 threads, 67 with 128).
+constexpr int64_t CORE_NARROW = 1024;
 
-template <class T, bool VECTOR>
-__global__ void __launch_bounds__(TS) k_core_prod(int64_t ncols, int64_t cb, int64_t ce,
+template <class T, bool VECTOR, int NT>
+__global__ void __launch_bounds__(NT) k_core_prod(int64_t ncols, int64_t cb, int64_t ce,
                                                   const int32_t* __restrict__ start,
                                                   const int32_t* __restrict__ row,
                                                   const int32_t* __restrict__ pair,
@@ -251,14 +257,14 @@ __global__ void __launch_bounds__(TS) k_core_prod(int64_t ncols, int64_t cb, int
   using VT = typename V16<T>::u;
   __shared__ __align__(16) T cf[CORE_YC][XB];  // signed coefficients of the staged members
   __shared__ int32_t rw[CORE_YC];              // their rows
-  const int64_t ntiles = (ce - cb + TS * VN - 1) / (TS * VN);
+  const int64_t ntiles = (ce - cb + NT * VN - 1) / (NT * VN);
   const int64_t ngrp = ngroups;
   const int64_t per = (ntiles * ngrp + 7) / 8;
   const int64_t w = (int64_t)(blockIdx.x % 8) * per + blockIdx.x / 8;
   if (w >= ntiles * ngrp) return;  // whole workgroup: no barrier is skipped by part of it
   const int64_t tile = w / ngrp;
   const int64_t g = w - tile * ngrp;
-  int64_t c0 = cb + tile * (TS * VN) + (int64_t)threadIdx.x * VN;
+  int64_t c0 = cb + tile * (NT * VN) + (int64_t)threadIdx.x * VN;
   const bool active = c0 < ce;  // inactive lanes still take part in the barriers
   if (VECTOR) c0 = min(c0, ce - VN);  // the last columns again rather than a part of a vector
   constexpr bool full = VECTOR;
@@ -277,7 +283,7 @@ __global__ void __launch_bounds__(TS) k_core_prod(int64_t ncols, int64_t cb, int
     for (int y0 = 0; y0 < m; y0 += CORE_YC) {
       const int ny = min(CORE_YC, m - y0);
       __syncthreads();  // previous step done with the staged entries
-      for (int e = threadIdx.x; e < ny * XB; e += TS) {
+      for (int e = threadIdx.x; e < ny * XB; e += NT) {
         const int yy = e / XB, xi = e - yy * XB;
         T v = T(0);
         if (xi < nx) {
@@ -745,17 +751,19 @@ void launch_spin(bool diag, int64_t nrows, int64_t ncols, const SpmmTable& tb, c
   for (int64_t cb = 0; cb < ncols; cb += zcols) {
     const int64_t ce = std::min(ncols, cb + zcols);
     if (ct->ngrp > 0) {
-      const int64_t ntiles = (ce - cb + TS * VN - 1) / (TS * VN);
-      const int64_t items = ntiles * ct->ngrp;
-      const int64_t nwg = (items + 7) / 8 * 8;
-      if (nwg > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
-      dim3 g((unsigned)nwg), b(TS);
-      if (ce - cb >= VN)
-        hipLaunchKernelGGL((k_core_prod<T, true>), g, b, 0, st, ncols, cb, ce, ct->start.p, ct->row.p, ct->pair.p,
-                           ct->blk.p, ct->blk_x0.p, ct->grp.p, ct->ngrp, W, npair, X, Z, zcols);
-      else
-        hipLaunchKernelGGL((k_core_prod<T, false>), g, b, 0, st, ncols, cb, ce, ct->start.p, ct->row.p,
-                           ct->pair.p, ct->blk.p, ct->blk_x0.p, ct->grp.p, ct->ngrp, W, npair, X, Z, zcols);
+      auto prod = [&](auto vec, auto threads) {
+        constexpr int NT = decltype(threads)::value;
+        const int64_t ntiles = (ce - cb + NT * VN - 1) / (NT * VN);
+        const int64_t items = ntiles * ct->ngrp;
+        const int64_t nwg = (items + 7) / 8 * 8;
+        if (nwg > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
+        hipLaunchKernelGGL((k_core_prod<T, decltype(vec)::value, NT>), dim3((unsigned)nwg), dim3(NT), 0, st, ncols, cb,
+                           ce, ct->start.p, ct->row.p, ct->pair.p, ct->blk.p, ct->blk_x0.p, ct->grp.p, ct->ngrp, W,
+                           npair, X, Z, zcols);
+      };
+      if (ce - cb < VN) prod(std::false_type{}, std::integral_constant<int, 64>{});
+      else if (ce - cb <= 128 * VN && ct->ngrp >= CORE_NARROW) prod(std::true_type{}, std::integral_constant<int, 128>{});
+      else prod(std::true_type{}, std::integral_constant<int, TS>{});
     }
     launch_spmm<T>(diag, nrows, ncols, tb, J, X, hii, out, st, cb, ce, ct, Z, zcols);
   }

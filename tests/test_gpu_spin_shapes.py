@@ -63,3 +63,10 @@ def test_core_sizes_around_the_workspace_cut(norb, nb, capped):
     s.close()
     if capped:
         check(case, doubles=2, core_gib=(members * 512 * 8 + 4096) / 2**30).close()
+
+
+@pytest.mark.parametrize("na", [3, 256, 257, 513])
+def test_core_pass_of_few_columns_and_many_blocks(na):
+    """Rows of up to 128 vectors (256 columns in FP64, 512 in FP32) over the 2,800 product blocks
+    of all strings of five electrons in 16 orbitals, and the first row length beyond."""
+    check(workload_small(16, 5, 5, na, 0, 73), doubles=2).close()
