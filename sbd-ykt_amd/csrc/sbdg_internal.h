@@ -402,6 +402,11 @@ __host__ __device__ inline uint32_t ab_pair(uint32_t b, uint32_t j) {
   const uint32_t h = b > j ? b : j, l = b > j ? j : b;
   return h * (h - 1) / 2 + l;
 }
+// A set of one beta string has no singles, so there are no alpha-beta terms.
+inline bool ab_any(int64_t nb) { return nb >= 2; }
+// First of the two neighbouring columns that place x of the alpha-beta kernel's staging loads of
+// a chunk of nj columns (nj >= 2: ab_any): the places past the last two take them again.
+__host__ __device__ inline int ab_stage_pair(int x, int nj) { return x < nj - 2 ? x : nj - 2; }
 inline int64_t ab_slice_span(int L) {
   return ab_pairs(L);
 }

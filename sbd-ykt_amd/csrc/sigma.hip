@@ -569,12 +569,7 @@ __global__ void __launch_bounds__(NT, NT == 768 ? 3 : 4) k_ab(const AbArgs<T> A)
         // of SR ket and SV slice vectors per thread.  Every global load of a round is issued,
         // at an index held inside the row, before its first use: a round costs one memory
         // latency (a load under a condition is waited for by itself).
-        const int xl = max(nj - 2, 0);   // the last pair of columns starts at xl
-        if (nj < 2 && xt == 0) {  // a single column
-#pragma unroll
-          for (int g = 0; g < G; ++g) cbv[0].v[g] = has[g] ? R::flip(crow[g][0], neg[g]) : T(0);
-        }
-        for (int x0 = nj < 2 ? 2 : 2 * xt, y0 = xt; x0 < nj || y0 < NPS; x0 += SR * NT, y0 += SV * NT) {
+        for (int x0 = 2 * xt, y0 = xt; x0 < nj || y0 < NPS; x0 += SR * NT, y0 += SV * NT) {
           RV sv[SV], kv[SR];
 #pragma unroll
           for (int u = 0; u < SV; ++u) {
@@ -584,7 +579,7 @@ __global__ void __launch_bounds__(NT, NT == 768 ? 3 : 4) k_ab(const AbArgs<T> A)
           }
 #pragma unroll
           for (int u = 0; u < SR; u += 2) {
-            const int x = min(x0 + u * NT, xl);
+            const int x = ab_stage_pair(x0 + u * NT, nj);
 #pragma unroll
             for (int g = 0; g < G; ++g) {
               const typename R::P2 w = __builtin_nontemporal_load(reinterpret_cast<const typename R::P2*>(crow[g] + x));
@@ -604,7 +599,7 @@ __global__ void __launch_bounds__(NT, NT == 768 ? 3 : 4) k_ab(const AbArgs<T> A)
               kv[u].v[g] = has[g] ? R::flip(kv[u].v[g], neg[g]) : T(0);
               kv[u + 1].v[g] = has[g] ? R::flip(kv[u + 1].v[g], neg[g]) : T(0);
             }
-            const int xx = x0 + u * NT, x = min(xx, xl);
+            const int xx = x0 + u * NT, x = ab_stage_pair(xx, nj);
             if (xx < nj) {
               cbv[x] = kv[u];
               cbv[x + 1] = kv[u + 1];
@@ -819,6 +814,7 @@ void launch_ab(const SigmaPlan& P, const T* eri, const T* c, T* sigma, hipStream
   if (P.na == 0 || P.nb == 0) return;
   const EllTable& E = *P.ell;
   if ((int64_t)E.nt * E.m * E.ntiles != E.groups * 64) throw Error(SBDG_ERR_STATE, "alpha-beta table geometry");
+  if (P.nb - (int64_t)(E.nch - 1) * E.chunk < 2) throw Error(SBDG_ERR_STATE, "alpha-beta chunk of less than two columns");
   const size_t lds = ab_lds_bytes(E.kbase, E.chunk) * E.s;
   bool done = false;  // the shapes ab_geometry picks
 #define SBDG_AB(NT, M, S)                                        \
@@ -890,7 +886,7 @@ void sigma_apply(const SigmaPlan& P, const T* c, T* sigma, const SigmaScratch<T>
   // determinants the fork and join cost more than the overlap gains (239^2 strings: 86 us
   // with it, 69 in sequence; 275^2: 95 and 89; 500 x 321: 125 and 152).
   T* sab = scr.sab;
-  const bool beside = P.st2 && P.na * P.nb >= 100000;
+  const bool ab = ab_any(P.nb), beside = P.st2 && ab && P.na * P.nb >= 100000;
   if (beside) {
     SBDG_CHECK(hipEventRecord(P.fork, st));
     SBDG_CHECK(hipStreamWaitEvent(P.st2, P.fork, 0));
@@ -923,7 +919,7 @@ void sigma_apply(const SigmaPlan& P, const T* c, T* sigma, const SigmaScratch<T>
   } else {
     launch_transpose<T, 1>(P.nb, P.na, sT, sigma, st);
     if (ev) SBDG_CHECK(hipEventRecord(ev[4], st));
-    launch_ab<T>(P, eri, c, sigma, st, 0);
+    if (ab) launch_ab<T>(P, eri, c, sigma, st, 0);
     if (ev) SBDG_CHECK(hipEventRecord(ev[5], st));
   }
   SBDG_CHECK(hipGetLastError());
