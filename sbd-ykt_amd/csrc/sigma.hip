@@ -667,16 +667,18 @@ __global__ void __launch_bounds__(NT, NT == 768 ? 3 : 4) k_ab(const AbArgs<T> A)
   }
 }
 
-// out[row, :] += the partial rows of the row's further segments, in order
+// out[row, :] += the partial rows of the row's further segments, in order.  Rows and column
+// tiles are one grid dimension: the rows with partial rows are as many as the alpha strings, and
+// a second dimension ends at 65,535.
 template <class T>
-__global__ void __launch_bounds__(256) k_ab_join(int64_t nb, const int32_t* __restrict__ jrow,
+__global__ void __launch_bounds__(256) k_ab_join(int64_t nb, int64_t ntiles, const int32_t* __restrict__ jrow,
                                                  const int32_t* __restrict__ jptr, const T* __restrict__ part,
                                                  T* __restrict__ out) {
-  const int64_t c = (int64_t)blockIdx.x * 256 + threadIdx.x;
+  const int64_t j = blockIdx.x / ntiles, c = (blockIdx.x % ntiles) * 256 + threadIdx.x;
   if (c >= nb) return;
-  const int64_t r = jrow[blockIdx.y];
+  const int64_t r = jrow[j];
   T v = out[r * nb + c];
-  for (int e = jptr[blockIdx.y]; e < jptr[blockIdx.y + 1]; ++e) v += part[(int64_t)e * nb + c];
+  for (int e = jptr[j]; e < jptr[j + 1]; ++e) v += part[(int64_t)e * nb + c];
   out[r * nb + c] = v;
 }
 
@@ -850,9 +852,12 @@ void launch_ab(const SigmaPlan& P, const T* eri, const T* c, T* sigma, hipStream
 #undef SBDG_AB
   if (!done) throw Error(SBDG_ERR_STATE, "alpha-beta columns per thread");
   const AbSegments& G = *P.seg;
-  if (G.njoin > 0)
-    hipLaunchKernelGGL(k_ab_join<T>, dim3((unsigned)((P.nb + 255) / 256), (unsigned)G.njoin), dim3(256), 0, st, P.nb,
-                       G.jrow.p, G.jptr.p, reinterpret_cast<const T*>(G.part.p), sigma);
+  if (G.njoin > 0) {
+    const int64_t tiles = (P.nb + 255) / 256, nblk = tiles * G.njoin;
+    if (nblk > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
+    hipLaunchKernelGGL(k_ab_join<T>, dim3((unsigned)nblk), dim3(256), 0, st, P.nb, tiles, G.jrow.p, G.jptr.p,
+                       reinterpret_cast<const T*>(G.part.p), sigma);
+  }
 }
 
 }  // namespace

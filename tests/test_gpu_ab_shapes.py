@@ -36,3 +36,30 @@ def test_sigma_at_launch_shape_edges(norb, nel, na, nb):
     s.set_options(overlap=0)
     assert np.abs(s.sigma(x) - want).max() <= 1e-12 * top
     s.close()
+
+
+def test_sigma_with_more_joined_rows_than_a_grid_dimension():
+    """All strings of 8 electrons in 19 orbitals: 75,582 alpha rows of 88 singles, each cut after
+    64, so that more than 65,535 rows are joined.  Rows at both ends and around that count against
+    the oracle, every row on one stream against two."""
+    c = workload_small(19, 8, 3, 0, 5, 79)
+    s = sbdg.Solver(c["norb"], c["core"], c["h1"], c["eri"], c["astr"], c["bstr"])
+    p = oracle.Problem(c["norb"], c["core"], c["h1"], c["astr"], c["bstr"], eri=c["eri"])
+    assert s.na > 65535 and int(np.diff(s.table(0)[0]).min()) > 64
+    x = np.random.default_rng(8).normal(size=s.ndet)
+    hii = p.hii()
+    got = {}
+    for overlap in (0, 1):
+        s.set_options(overlap=overlap)
+        for precision in (0, 1):
+            got[overlap, precision] = s.sigma(x, precision=precision).reshape(s.na, s.nb)
+    top = np.abs(got[0, 0]).max()
+    for r0 in (0, 40000, 65520, s.na - 30):
+        want = p.sigma_rows(x, hii, r0, r0 + 30).reshape(s.na, s.nb)[r0:r0 + 30]
+        for (overlap, precision), y in got.items():
+            err = np.abs(y[r0:r0 + 30] - want).max() / top
+            print(f"rows {r0}+30, overlap {overlap}, precision {precision}: {err:.1e}", flush=True)
+            assert err <= (2e-5 if precision else 1e-12)
+    for precision, bar in ((0, 1e-12), (1, 2e-5)):
+        assert np.abs(got[0, precision] - got[1, precision]).max() <= bar * top
+    s.close()
