@@ -506,10 +506,9 @@ __global__ void __launch_bounds__(64) k_jacobi(const double* __restrict__ H, int
       __syncthreads();
     }
   }
-  if (k < m) {  // ascending; equal values by index
-    const double e = A[k * 65];
+  if (k < m) {
     int rank = 0;
-    for (int j = 0; j < m; ++j) rank += A[j * 65] < e || (A[j * 65] == e && j < k);
+    for (int j = 0; j < m; ++j) rank += eigen_before(A[j * 65], j, A[k * 65], k);
     ord[rank] = k;
   }
   __syncthreads();

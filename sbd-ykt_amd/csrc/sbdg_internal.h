@@ -449,6 +449,12 @@ void gs_impl(const double* V, int64_t ldv, int m, const double* s, double* t, in
 // in place: X_j = sum_k U[k + ld*j] X_k for j < mk (thick-restart rotation)
 template <class T>
 void rotate_impl(T* X, int64_t ldx, int m, const double* U, int ld, int mk, int64_t n, hipStream_t st);
+// Order of eigenvalues x at place i and y at place j: ascending, NaN last, equal ones by place.  A
+// strict order whatever the values, so that counting the places before each gives every rank once.
+__host__ __device__ inline bool eigen_before(double x, int i, double y, int j) {
+  if (x != x || y != y) return (x != x) == (y != y) ? i < j : y != y;
+  return x < y || (x == y && i < j);
+}
 // symmetric eigensolve of the m x m column-major d_H (ld) on the device: ascending
 // eigenvalues in d_E, eigenvectors in the columns of d_U (ld).
 void syev_device(const double* d_H, int m, int ld, double* d_E, double* d_U, hipStream_t st);

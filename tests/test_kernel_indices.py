@@ -65,3 +65,39 @@ int main() {
   return seen > 50 ? 0 : 1;
 }
 """)
+
+
+def test_eigenvalue_ranks_are_a_permutation_whatever_the_values(tmp_path):
+    """k_jacobi ranks the diagonal by counting the places before each and writes each place to its
+    rank: with NaN and infinities too every rank has to occur once (one left out would be an unset
+    place, then an index into LDS), and ordinary values come out ascending."""
+    run_replay(tmp_path, r"""
+int main() {
+  const double nan = __builtin_nan(""), inf = __builtin_inf();
+  const double pool[] = {nan, -inf, -1.0, -0.0, 0.0, 0.0, 2.5, inf, nan, -1.0};
+  unsigned long long r = 12345;
+  for (int t = 0; t < 20000; ++t) {
+    const int m = 1 + t % 48;
+    std::vector<double> a(m);
+    for (double& x : a) {
+      r = r * 6364136223846793005ull + 1442695040888963407ull;
+      x = t % 3 ? pool[(r >> 33) % 10] : (double)(long long)(r >> 20);
+    }
+    std::vector<int> ord(m, -1);
+    for (int k = 0; k < m; ++k) {
+      int rank = 0;
+      for (int j = 0; j < m; ++j) rank += eigen_before(a[j], j, a[k], k);
+      if (rank >= m || ord[rank] >= 0) {
+        printf("rank %d of %d twice\n", rank, m);
+        return 1;
+      }
+      ord[rank] = k;
+    }
+    for (int k = 1; k < m; ++k) {
+      const double x = a[ord[k - 1]], y = a[ord[k]];
+      if (x > y || (x != x && y == y) || (x == y && ord[k - 1] > ord[k])) return 1;
+    }
+  }
+  return 0;
+}
+""")
