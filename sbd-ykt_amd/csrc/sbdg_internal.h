@@ -404,6 +404,11 @@ __host__ __device__ inline uint32_t ab_pair(uint32_t b, uint32_t j) {
 }
 // A set of one beta string has no singles, so there are no alpha-beta terms.
 inline bool ab_any(int64_t nb) { return nb >= 2; }
+// Vectors that a thread of the alpha-beta kernel stages per round.  Ket vectors: what its m columns
+// need, up to eight, four where the FP64 accumulators take the registers; more would only load the
+// row's last pair again.  Slice vectors: 512 of a workgroup of up to 256 threads.
+constexpr int ab_ket_round(int elem, int m) { return m <= 2 ? 2 : m <= 4 || elem * m > 160 ? 4 : 8; }
+constexpr int ab_slice_round(int nt) { return nt <= 256 ? 512 / nt : 2; }
 // First of the two neighbouring columns that place x of the alpha-beta kernel's staging loads of
 // a chunk of nj columns (nj >= 2: ab_any): the places past the last two take them again.
 __host__ __device__ inline int ab_stage_pair(int x, int nj) { return x < nj - 2 ? x : nj - 2; }

@@ -496,8 +496,7 @@ __global__ void __launch_bounds__(NT, NT == 768 ? 3 : 4) k_ab(const AbArgs<T> A)
   constexpr int B = AB_BATCH;
   // 16-byte vectors per thread per staging round: SR ket vectors (4*SR VGPRs beside the
   // accumulators) and SV slice vectors
-  constexpr int SR = (int)sizeof(T) * M <= 160 ? 8 : 4;
-  constexpr int SV = 2;
+  constexpr int SR = ab_ket_round((int)sizeof(T), M), SV = ab_slice_round(NT);
   extern __shared__ __align__(16) unsigned char smem[];
   const int64_t nb = A.nb, chunk = A.chunk, kbase = A.kbase;
   const int L = A.L;
@@ -824,6 +823,10 @@ void launch_ab(const SigmaPlan& P, const T* eri, const T* c, T* sigma, hipStream
     launch_ab_m<T, M, NT, S>(P, lds, eri, c, sigma, st, assign); \
     done = true;                                                 \
   }
+  SBDG_AB(64, 1, 2)
+  SBDG_AB(64, 2, 2)
+  SBDG_AB(128, 1, 2)
+  SBDG_AB(256, 1, 1)
   SBDG_AB(256, 1, 4)
   SBDG_AB(256, 1, 2)
   SBDG_AB(256, 2, 4)

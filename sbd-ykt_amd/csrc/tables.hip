@@ -457,6 +457,12 @@ void build_spmm(const Table& s, const Table& d, SpmmTable& m, int L, hipStream_t
 // one workgroup covers a whole row where it can (a second column tile stages every ket row
 // again: norb=36, 4,000 x 24,000 9.2 ms with one tile, 11.7 with two), s groups of ket rows
 // staged per barrier, and the ket columns cut into equal chunks that fill the LDS share.
+//  * up to 128 columns the slices are most of what is staged: 64 threads for up to 400 slice
+//    vectors, 128 up to 1,000, 256 beyond, and many workgroups on a CU (256 threads of four groups
+//    against one workgroup of 64 threads per whole row and these: norb=26, 20,000 x 64 FP64 1,054 /
+//    654 / 420 us, FP32 769 / 355 / 252, 20,000 x 4 800 / 537 / 274 and 611 / 290 / 161; norb=16,
+//    4,368 x 20 193 / 101 / 93; norb=36, 5,000 x 64 164 / 772 / 102; norb=58, 3,000 x 20
+//    170 / 700 / 133);
 //  * up to 1,024 columns: 256 threads and several groups per barrier while a few workgroups
 //    still fit a CU (norb=26, 2,000 x 1,000: 259 us with one group, 214 with two; norb=58,
 //    600 x 400: 115 / 104 / 249 us with one, two and four);
@@ -475,7 +481,10 @@ AbGeometry ab_geometry(int64_t nb, int L, int elem) {
   const bool half = nb <= 6000;
   g.nt = nb <= 1024 ? 256 : half ? 512 : 1024;
   g.s = 1;
-  if (nb <= 1024) {
+  if (nb <= 128) {
+    g.nt = kb <= 400 ? 64 : kb <= 1000 ? 128 : 256;
+    g.s = kb <= 1000 ? 2 : 1;
+  } else if (nb <= 1024) {
     const int64_t grp = 16 * (kb + nb + 1);
     g.s = nb <= 512 && 4 * grp <= 48 * 1024 ? 4 : 2 * grp <= 80 * 1024 ? 2 : 1;
   }
@@ -483,9 +492,11 @@ AbGeometry ab_geometry(int64_t nb, int L, int elem) {
   const int64_t maxchunk = (half ? 80 : 160) * 1024 / 16 / g.s - kb - 1;
   const int64_t nch = std::max<int64_t>(1, (nb + maxchunk - 1) / maxchunk);
   g.chunk = std::max<int64_t>(1, (nb + nch - 1) / nch);
-  static const int m256[] = {1, 2, 4, 0}, m512[] = {4, 6, 8, 10, 12, 0}, m1024d[] = {8, 12, 16, 20, 24, 0},
-                   m1024f[] = {8, 12, 16, 20, 24, 40, 48, 0}, m768[] = {32, 40, 48, 53, 0};
-  const int* ms = g.nt == 256 ? m256 : g.nt == 512 ? m512 : g.nt == 768 ? m768 : elem == 4 ? m1024f : m1024d;
+  static const int m64[] = {1, 2, 0}, m128[] = {1, 0}, m256[] = {1, 2, 4, 0}, m512[] = {4, 6, 8, 10, 12, 0},
+                   m1024d[] = {8, 12, 16, 20, 24, 0}, m1024f[] = {8, 12, 16, 20, 24, 40, 48, 0},
+                   m768[] = {32, 40, 48, 53, 0};
+  const int* ms = g.nt == 64 ? m64 : g.nt == 128 ? m128 : g.nt == 256 ? m256 : g.nt == 512 ? m512 : g.nt == 768 ? m768
+                  : elem == 4 ? m1024f : m1024d;
   g.m = 0;
   for (int i = 0; ms[i]; ++i) {
     g.m = ms[i];

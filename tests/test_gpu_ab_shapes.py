@@ -63,3 +63,13 @@ def test_sigma_with_more_joined_rows_than_a_grid_dimension():
     for precision, bar in ((0, 1e-12), (1, 2e-5)):
         assert np.abs(got[0, precision] - got[1, precision]).max() <= bar * top
     s.close()
+
+
+@pytest.mark.parametrize("norb,nel,na,nb", [
+    (12, 4, 200, 2), (18, 5, 90, 63), (18, 5, 90, 64), (18, 5, 90, 65), (18, 5, 90, 128), (18, 5, 90, 129),
+    (29, 5, 80, 128), (30, 5, 80, 33), (45, 5, 80, 128), (46, 5, 80, 3), (58, 6, 80, 128),
+])
+def test_sigma_at_narrow_row_shapes(norb, nel, na, nb):
+    """Rows of up to 128 columns: workgroups of 64, 128 and 256 threads by the number of slice
+    vectors (406 at norb=29, 990 at 45, 1,035 at 46), and the first row length beyond."""
+    test_sigma_at_launch_shape_edges(norb, nel, na, nb)

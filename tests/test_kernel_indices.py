@@ -34,12 +34,12 @@ def test_alpha_beta_staging_stays_inside_the_ket_row(tmp_path):
     run_replay(tmp_path, r"""
 int main() {
   long seen = 0;
-  for (int L : {2, 18, 64})
+  for (int L : {2, 18, 36, 64})
     for (int elem : {4, 8})
-      for (int64_t nb : {1, 2, 3, 5, 256, 257, 512, 513, 1024, 1025, 2047, 6000, 6001, 8193, 24576, 24577, 40705}) {
+      for (int64_t nb : {1, 2, 3, 5, 64, 65, 128, 129, 256, 257, 512, 513, 1024, 1025, 2047, 6000, 6001, 8193, 24576, 24577, 40705}) {
         if (!ab_any(nb)) continue;  // not launched
         const AbGeometry g = ab_geometry(nb, L, elem);
-        const int SR = elem * g.m <= 160 ? 8 : 4, SV = 2, NPS = (int)ab_pairs(L);
+        const int SR = ab_ket_round(elem, g.m), SV = ab_slice_round(g.nt), NPS = (int)ab_pairs(L);
         for (int64_t j0 = 0; j0 < nb; j0 += g.chunk) {
           const int nj = (int)(std::min(nb, j0 + g.chunk) - j0);
           std::vector<char> stored(nj, 0);
