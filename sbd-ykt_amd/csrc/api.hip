@@ -105,7 +105,7 @@ struct sbdg_ctx {
   DBuf<double> Wp;        // antisymmetrised pair integrals
   DBuf<float> Wp32;
   DBuf<double> Zbuf;      // core-product workspace
-  AbPairs abp;      // beta pairs (RDMs; built by the first RDM of a string set)
+  AbPairs abp;      // beta pairs (RDMs; built by the first RDM of a string set, kept while the beta strings and norb are)
   EllTable ell;      // beta singles, ELL (alpha-beta sigma, FP64; FP32 too when the geometries agree)
   EllTable ell32;    // the FP32 ELL when its launch geometry differs (wide rows)
   bool own_ell32 = false;
@@ -264,7 +264,6 @@ void build(sbdg_ctx* c) {
   compute_hii(c->d_a.p, na, c->d_b.p, nb, L, c->core, c->d_h1.p, c->d_eri.p, c->d_hii.p, c->st);
   cast_d2f(c->d_hii.p, c->d_hii32.p, N, c->st);
   SBDG_CHECK(hipStreamSynchronize(c->st));
-  c->abp.built = false;
   c->built = true;
   c->solved = c->have_rdm = c->have_dens = false;
   c->stats = sbdg_stats{};
@@ -964,6 +963,7 @@ int sbdg_set_integrals(sbdg_ctx* c, int norb, double core, const double* h1, con
     if (!h1 || !eri) return fail(c, SBDG_ERR_ARG, "null integral pointer");
     const int L = norb;
     const int64_t L4 = (int64_t)L * L * L * L;
+    if (c->L != L) c->abp.built = false;
     c->L = L;
     c->core = core;
     c->h1.assign(h1, h1 + L * L);
@@ -1035,6 +1035,7 @@ int sbdg_set_strings(sbdg_ctx* c, const uint64_t* a, int64_t na, const uint64_t*
     if (!m.empty()) return fail(c, SBDG_ERR_ARG, m);
     if (nb > (1 << 18)) return fail(c, SBDG_ERR_LIMIT, "beta string set beyond 262144 strings");
     if (na > (int64_t)INT32_MAX) return fail(c, SBDG_ERR_LIMIT, "alpha string set beyond 2^31 strings");
+    if ((int64_t)c->b.size() != nb || !std::equal(b, b + nb, c->b.begin())) c->abp.built = false;
     c->a.assign(a, a + na);
     c->b.assign(b, b + nb);
     c->have_strs = true;

@@ -67,3 +67,30 @@ def test_rdm_same_bits_whatever_memory_is_idle(norb, nel, na, nb):
         s.close()
     for other in got[1:]:
         assert all(np.array_equal(x, y) for x, y in zip(got[0], other))
+
+
+def test_rdm_after_new_integrals_and_new_strings():
+    """The beta-pair tables belong to the beta strings and norb: one context taken through new
+    integrals on its strings, other alpha strings, other beta strings of the same number, and
+    another norb gives the bits of a context made for each."""
+    first = workload_small(14, 4, 4, 60, 300, 83)
+    steps = [first, dict(workload_small(14, 4, 4, 60, 300, 84), astr=first["astr"], bstr=first["bstr"])]
+    steps.append(dict(steps[1], astr=workload_small(14, 4, 4, 55, 300, 85)["astr"]))
+    steps.append(dict(steps[2], bstr=workload_small(14, 4, 4, 55, 300, 86)["bstr"]))
+    steps.append(dict(workload_small(16, 4, 4, 55, 300, 87), astr=steps[3]["astr"], bstr=steps[3]["bstr"]))
+    options = dict(max_it=1, max_nb=2, eps=1e10, init=1, seed=9, do_rdm=1)
+    s = None
+    for c in steps:
+        fresh = sbdg.Solver(c["norb"], c["core"], c["h1"], c["eri"], c["astr"], c["bstr"], **options)
+        if s is None:
+            s = sbdg.Solver(c["norb"], c["core"], c["h1"], c["eri"], c["astr"], c["bstr"], **options)
+        else:
+            s.norb, s.astr, s.bstr, s.na, s.nb = c["norb"], c["astr"], c["bstr"], len(c["astr"]), len(c["bstr"])
+            s.set_integrals(c["core"], c["h1"], c["eri"])
+        for x in (s, fresh):
+            x.run()
+        got, want = (*s.rdm(), s.density()), (*fresh.rdm(), fresh.density())
+        assert all(np.array_equal(x, y) for x, y in zip(got, want))
+        assert abs(got[0][1].reshape(c["norb"], -1).trace() - 4) < 1e-11
+        fresh.close()
+    s.close()
