@@ -1091,42 +1091,53 @@ void doubles_part(const Table& t, int L, int s, const double* X, int64_t ncols, 
 // together (LDS16_LANE).  Per set and slot of the first column, the largest class of
 // pairs (by their two slots) whose second slot is still free in the set; a slot left without
 // one takes the largest class of any.  out and rank: the pairs in order and their places in
-// the sorted list.
+// the sorted list.  The sixteen classes of a first slot are compared as one vector of 16-bit
+// counts (all strings of 7 electrons in 20 orbitals, 3.5M pairs: 171 -> 85 ms on the host).
 static void order_pairs(const uint32_t* in, int n, uint32_t* out, uint16_t* rank) {
+  typedef int16_t v16 __attribute__((vector_size(32)));
+  alignas(32) int16_t left[256] = {0};  // pairs left per class (n is at most a tile's: 12,288)
   std::vector<int> next(256, 0), cls(n);
-  std::vector<int> cnt(257, 0);
   auto slots = [](uint32_t w) { return (int)((w & 15u) * 16 + ((w >> 15) & 15u)); };
-  for (int e = 0; e < n; ++e) ++cnt[slots(in[e]) + 1];
-  for (int k = 0; k < 256; ++k) cnt[k + 1] += cnt[k];
-  for (int k = 0; k < 256; ++k) next[k] = cnt[k];
-  for (int e = 0; e < n; ++e) cls[next[slots(in[e])]++] = e;
-  for (int k = 0; k < 256; ++k) next[k] = cnt[k];
+  for (int e = 0; e < n; ++e) ++left[slots(in[e])];
+  for (int k = 1; k < 256; ++k) next[k] = next[k - 1] + left[k - 1];
+  {
+    std::vector<int> at(next);
+    for (int e = 0; e < n; ++e) cls[at[slots(in[e])]++] = e;
+  }
   int pos = 0;
   auto take = [&](int k) {
     const int e = cls[next[k]++];
+    --left[k];
     const int at = pos - (pos & 31) + LDS16_LANE[pos & 31];
     out[at] = in[e];
     rank[at] = (uint16_t)e;
     ++pos;
   };
+  auto largest = [](v16 m) {  // of 16 numbers, by halves
+    auto fold = [&](v16 o) { m = m > o ? m : o; };
+    fold(__builtin_shufflevector(m, m, 8, 9, 10, 11, 12, 13, 14, 15, 0, 1, 2, 3, 4, 5, 6, 7));
+    fold(__builtin_shufflevector(m, m, 4, 5, 6, 7, 0, 1, 2, 3, 12, 13, 14, 15, 8, 9, 10, 11));
+    fold(__builtin_shufflevector(m, m, 2, 3, 0, 1, 6, 7, 4, 5, 10, 11, 8, 9, 14, 15, 12, 13));
+    fold(__builtin_shufflevector(m, m, 1, 0, 3, 2, 5, 4, 7, 6, 9, 8, 11, 10, 13, 12, 15, 14));
+    return (int)m[0];
+  };
   while (pos < n) {
-    unsigned used = 0;
+    v16 open = v16{} - 1;  // second slots still free in the set
     for (int t = 0; t < 16 && pos < n; ++t) {
       const int i = (t + pos / 16) & 15;  // no slot always chooses last
-      int best = -1;
-      for (int j = 0; j < 16; ++j) {
-        const int k = i * 16 + j, left = cnt[k + 1] - next[k];
-        if (left > 0 && !((used >> j) & 1u) && (best < 0 || left > cnt[best + 1] - next[best])) best = k;
-      }
-      if (best < 0) continue;
-      used |= 1u << (best & 15);
-      take(best);
+      const v16 c = *reinterpret_cast<const v16*>(left + 16 * i) & open;
+      const int most = largest(c);
+      if (most == 0) continue;
+      int j = 0;
+      while (c[j] != most) ++j;
+      open[j] = 0;
+      take(16 * i + j);
     }
     // fill the set to a multiple of 16 with what is left over
     while (pos < n && (pos & 15)) {
-      int best = -1;
-      for (int k = 0; k < 256; ++k)
-        if (cnt[k + 1] > next[k] && (best < 0 || cnt[k + 1] - next[k] > cnt[best + 1] - next[best])) best = k;
+      int best = 0;
+      for (int k = 1; k < 256; ++k)
+        if (left[k] > left[best]) best = k;
       take(best);
     }
   }
@@ -1141,17 +1152,16 @@ static void order_pairs(const uint32_t* in, int n, uint32_t* out, uint16_t* rank
 void build_ab_pairs(const Table& sb, int L, AbPairs& ab, hipStream_t st) {
   const int64_t nb = sb.n;
   if (nb > (1 << 18)) throw Error(SBDG_ERR_LIMIT, "beta string set beyond 2^18 strings");
+  const int64_t nnz = sb.nnz;
   std::vector<int64_t> rp(nb + 1, 0);
-  SBDG_CHECK(hipMemcpyAsync(rp.data(), sb.rowptr.p, sizeof(int64_t) * (nb + 1), hipMemcpyDeviceToHost, st));
-  SBDG_CHECK(hipStreamSynchronize(st));
-  const int64_t nnz = rp[nb];
   std::vector<int32_t> col(nnz);
   std::vector<uint32_t> exc(nnz);
+  SBDG_CHECK(hipMemcpyAsync(rp.data(), sb.rowptr.p, sizeof(int64_t) * (nb + 1), hipMemcpyDeviceToHost, st));
   if (nnz) {
     SBDG_CHECK(hipMemcpyAsync(col.data(), sb.col.p, sizeof(int32_t) * nnz, hipMemcpyDeviceToHost, st));
     SBDG_CHECK(hipMemcpyAsync(exc.data(), sb.exc.p, sizeof(uint32_t) * nnz, hipMemcpyDeviceToHost, st));
-    SBDG_CHECK(hipStreamSynchronize(st));
   }
+  SBDG_CHECK(hipStreamSynchronize(st));
   const int64_t NP = std::max<int64_t>(1, (int64_t)L * (L - 1) / 2);
   const bool small = nnz / 2 < 32768;
   ab.nt = small ? ABR_NT_S : ABR_NT;
@@ -1228,18 +1238,8 @@ void build_ab_pairs(const Table& sb, int L, AbPairs& ab, hipStream_t st) {
   }
   ab.ntiles = (int64_t)tile.size();
   ab.nruns = (int64_t)runstart.size();
-  auto up = [&](auto& d, const auto& h) {
-    d.alloc(std::max<size_t>(h.size(), 1));
-    if (!h.empty()) SBDG_CHECK(hipMemcpy(d.p, h.data(), sizeof(h[0]) * h.size(), hipMemcpyHostToDevice));
-  };
-  up(ab.tile, tile);
-  up(ab.entoff, entoff);
-  up(ab.ent, ent);
-  up(ab.rank, rank);
-  up(ab.runptr, runptr);
-  up(ab.runstart, runstart);
-  up(ab.pairptr, pairptr);
-  up(ab.pairrun, pairrun);
+  ab.mem.put({{&ab.tile, tile}, {&ab.entoff, entoff}, {&ab.ent, ent}, {&ab.rank, rank}, {&ab.runptr, runptr},
+              {&ab.runstart, runstart}, {&ab.pairptr, pairptr}, {&ab.pairrun, pairrun}});
   ab.built = true;
 }
 
@@ -1314,7 +1314,7 @@ void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* one, dou
     const bool many = ab.nt == ABR_NT;
     const size_t lds = std::max<size_t>(16 * (size_t)(many ? 2 : ab.sp) * (size_t)(ab.maxcols + 1),
                                         8 * (size_t)ab.nt * ab.u);
-    AbRdmArgs A{nb, ab.nruns, ab.ntiles, 0, ab.tile.p, ab.entoff.p, ab.ent.p, ab.rank.p, ab.runptr.p, ab.runstart.p,
+    AbRdmArgs A{nb, ab.nruns, ab.ntiles, 0, ab.tile, ab.entoff, ab.ent, ab.rank, ab.runptr, ab.runstart,
                 nullptr, ssa.pia.p, ssa.pja.p, W, part.p};
     for (const auto& bt : K.batch) {
       const int64_t s0 = K.kseg[bt.first], ns = K.kseg[bt.second] - s0;
@@ -1327,7 +1327,7 @@ void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* one, dou
       else if (ab.sp > 1) hipLaunchKernelGGL(k_ab_rdm_small<4>, g, t, lds, st, A);
       else hipLaunchKernelGGL(k_ab_rdm_small<1>, g, t, lds, st, A);
       hipLaunchKernelGGL(k_ab_slots, dim3((unsigned)(bt.second - bt.first)), dim3(256), 0, st, L,
-                         K.dkeys.p + bt.first, K.dkseg.p + bt.first, s0, ab.nruns, ab.pairptr.p, ab.pairrun.p, part.p, two);
+                         K.dkeys.p + bt.first, K.dkseg.p + bt.first, s0, ab.nruns, ab.pairptr, ab.pairrun, part.p, two);
     }
     SBDG_CHECK(hipGetLastError());
     SBDG_CHECK(hipStreamSynchronize(st));

@@ -16,6 +16,8 @@
 
 #include <algorithm>
 #include <atomic>
+#include <cstring>
+#include <initializer_list>
 #include <string>
 #include <vector>
 
@@ -78,6 +80,41 @@ struct DBuf {
   DBuf() = default;
   DBuf(const DBuf&) = delete;
   DBuf& operator=(const DBuf&) = delete;
+};
+
+// Tables made on the host, together in one device buffer: one allocation, and one copy where they
+// are small (each takes some 10 us, which a set of a few strings feels).
+class TableMem {
+ public:
+  struct Part {
+    void* at;  // const T*: set to the table's place
+    void (*set)(void*, const void*);
+    const void* src;
+    size_t bytes;
+    template <class T>
+    Part(const T** a, const std::vector<T>& h)
+        : at(a), set([](void* d, const void* p) { *static_cast<const T**>(d) = static_cast<const T*>(p); }),
+          src(h.data()), bytes(sizeof(T) * h.size()) {}
+  };
+  void put(std::initializer_list<Part> parts) {
+    size_t total = 0;
+    for (const Part& x : parts) total += room(x);
+    mem_.alloc(total);
+    std::vector<unsigned char> host(total <= SMALL ? total : 0);
+    size_t o = 0;
+    for (const Part& x : parts) {
+      x.set(x.at, mem_.p + o);
+      if (x.bytes && !host.empty()) std::memcpy(host.data() + o, x.src, x.bytes);
+      else if (x.bytes) SBDG_CHECK(hipMemcpy(mem_.p + o, x.src, x.bytes, hipMemcpyHostToDevice));
+      o += room(x);
+    }
+    if (!host.empty()) SBDG_CHECK(hipMemcpy(mem_.p, host.data(), total, hipMemcpyHostToDevice));
+  }
+
+ private:
+  static constexpr size_t SMALL = 1 << 20;
+  static size_t room(const Part& x) { return (x.bytes + 255) / 256 * 256 + (x.bytes ? 0 : 256); }
+  DBuf<unsigned char> mem_;
 };
 
 // Workspace carved out of device memory that lies idle (the RDMs' out of the Davidson vectors):
@@ -224,11 +261,12 @@ struct AbPairs {
   bool built = false;
   int nt = 0, u = 0, sp = 1;  // threads, pairs per thread, alpha pairs staged at once
   int64_t maxcols = 0, ntiles = 0, nruns = 0;
-  DBuf<int4> tile;       // first column and number of columns of the tile's two chunks
-  DBuf<int64_t> entoff;
-  DBuf<uint32_t> ent;
-  DBuf<uint16_t> rank;   // place of each entry in its tile's sorted list
-  DBuf<int32_t> runptr, runstart, pairptr, pairrun;
+  TableMem mem;
+  const int4* tile;      // first column and number of columns of the tile's two chunks
+  const int64_t* entoff;
+  const uint32_t* ent;
+  const uint16_t* rank;  // place of each entry in its tile's sorted list
+  const int32_t *runptr, *runstart, *pairptr, *pairrun;
 };
 
 // Beta singles in an ELL layout for the alpha-beta sigma kernel.  Columns are cut into
