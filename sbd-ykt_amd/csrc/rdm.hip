@@ -1092,7 +1092,8 @@ void doubles_part(const Table& t, int L, int s, const double* X, int64_t ncols, 
 // pairs (by their two slots) whose second slot is still free in the set; a slot left without
 // one takes the largest class of any.  out and rank: the pairs in order and their places in
 // the sorted list.  The sixteen classes of a first slot are compared as one vector of 16-bit
-// counts (all strings of 7 electrons in 20 orbitals, 3.5M pairs: 171 -> 85 ms on the host).
+// counts (3.5M pairs, all strings of 7 electrons in 20 orbitals: 180 -> 70 ms on the host; 2.9M of
+// 200,000 sampled strings at norb=36, whose 1,543 tiles leave more to the fills: 210 -> 64).
 static void order_pairs(const uint32_t* in, int n, uint32_t* out, uint16_t* rank) {
   typedef int16_t v16 __attribute__((vector_size(32)));
   alignas(32) int16_t left[256] = {0};  // pairs left per class (n is at most a tile's: 12,288)
@@ -1113,20 +1114,13 @@ static void order_pairs(const uint32_t* in, int n, uint32_t* out, uint16_t* rank
     rank[at] = (uint16_t)e;
     ++pos;
   };
-  auto largest = [](v16 m) {  // of 16 numbers, by halves
-    auto fold = [&](v16 o) { m = m > o ? m : o; };
-    fold(__builtin_shufflevector(m, m, 8, 9, 10, 11, 12, 13, 14, 15, 0, 1, 2, 3, 4, 5, 6, 7));
-    fold(__builtin_shufflevector(m, m, 4, 5, 6, 7, 0, 1, 2, 3, 12, 13, 14, 15, 8, 9, 10, 11));
-    fold(__builtin_shufflevector(m, m, 2, 3, 0, 1, 6, 7, 4, 5, 10, 11, 8, 9, 14, 15, 12, 13));
-    fold(__builtin_shufflevector(m, m, 1, 0, 3, 2, 5, 4, 7, 6, 9, 8, 11, 10, 13, 12, 15, 14));
-    return (int)m[0];
-  };
+  const v16* rows = reinterpret_cast<const v16*>(left);
   while (pos < n) {
     v16 open = v16{} - 1;  // second slots still free in the set
     for (int t = 0; t < 16 && pos < n; ++t) {
       const int i = (t + pos / 16) & 15;  // no slot always chooses last
-      const v16 c = *reinterpret_cast<const v16*>(left + 16 * i) & open;
-      const int most = largest(c);
+      const v16 c = rows[i] & open;
+      const int16_t most = __builtin_reduce_max(c);
       if (most == 0) continue;
       int j = 0;
       while (c[j] != most) ++j;
@@ -1135,10 +1129,13 @@ static void order_pairs(const uint32_t* in, int n, uint32_t* out, uint16_t* rank
     }
     // fill the set to a multiple of 16 with what is left over
     while (pos < n && (pos & 15)) {
-      int best = 0;
-      for (int k = 1; k < 256; ++k)
-        if (left[k] > left[best]) best = k;
-      take(best);
+      v16 m = rows[0];
+      for (int i = 1; i < 16; ++i) m = __builtin_elementwise_max(m, rows[i]);
+      const int16_t most = __builtin_reduce_max(m);
+      int i = 0, j = 0;
+      while (!__builtin_reduce_or(rows[i] == most)) ++i;
+      while (rows[i][j] != most) ++j;
+      take(16 * i + j);
     }
   }
 }
