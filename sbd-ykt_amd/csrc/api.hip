@@ -204,8 +204,8 @@ void build(sbdg_ctx* c) {
   const int nel_a = na ? __builtin_popcountll(c->a[0]) : 0, nel_b = nb ? __builtin_popcountll(c->b[0]) : 0;
   c->use_ca = c->use_cb = false;
   if (c->opt.doubles != 1) {
-    build_cores(c->d_a.p, na, L, nel_a, c->eri.data(), nb, c->Ca, c->Xa, c->st);
-    build_cores(c->d_b.p, nb, L, nel_b, c->eri.data(), na, c->Cb, c->Xb, c->st);
+    build_cores(c->d_a.p, na, L, nel_a, c->d_eri.p, nb, c->Ca, c->Xa, c->st);
+    build_cores(c->d_b.p, nb, L, nel_b, c->d_eri.p, na, c->Cb, c->Xb, c->st);
     // auto: the core form (its workspace for the larger cores, the pairs of the smaller
     // ones read directly) where it moves fewer rows and one 512-column pass of its
     // workspace fits core_gib; otherwise the excitation-table form

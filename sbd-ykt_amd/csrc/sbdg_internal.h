@@ -309,12 +309,13 @@ struct EllTable {
 constexpr int64_t AB_PART_BYTES = (int64_t)256 << 20;  // at most this much in partial rows
 struct AbSegments {
   int64_t nseg = 0, npart = 0, njoin = 0;
-  DBuf<int32_t> row;   // nseg
-  DBuf<int64_t> q;     // 2*nseg: first and past-the-end alpha single
-  DBuf<int32_t> dst;   // nseg: -1 or the row of part
-  DBuf<int32_t> jrow;  // njoin rows with partial rows
-  DBuf<int32_t> jptr;  // njoin + 1
-  DBuf<double> part;   // npart rows of nb
+  TableMem mem;
+  const int32_t* row;   // nseg
+  const int64_t* q;     // 2*nseg: first and past-the-end alpha single
+  const int32_t* dst;   // nseg: -1 or the row of part
+  const int32_t* jrow;  // njoin rows with partial rows
+  const int32_t* jptr;  // njoin + 1
+  DBuf<double> part;    // npart rows of nb
 };
 
 // Double excitations of one spin grouped by their (n-2)-electron core: a double pair
@@ -361,8 +362,8 @@ constexpr int CORE_KMIN = 10;
 void build_table(const uint64_t* d_str, int64_t n, int L, const double* d_h1, const double* d_eri,
                  Table& t_single, Table& t_double, hipStream_t st);
 void build_spmm(const Table& s, const Table& d, SpmmTable& m, int L, hipStream_t st, bool with_doubles = true);
-// h_eri: the integrals on the host (full L^4), for the values of the direct pairs
-void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* h_eri, int64_t ncols,
+// d_eri: the integrals (full L^4), for the values of the direct pairs
+void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* d_eri, int64_t ncols,
                  CoreTable& ct, Table& direct, hipStream_t st);
 // J[(p+1)*n + r] = sum_{o in occ(s[r])} eri[p*L^2 + o*L + o] for p < L^2 (row 0 zero):
 // the occupation part of the other spin's singles, (ai|oo) summed over the string's orbitals

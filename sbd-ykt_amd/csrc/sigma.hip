@@ -794,9 +794,9 @@ void launch_ab_m(const SigmaPlan& P, size_t lds, const T* eri, const T* c, T* si
   A.nch = E.nch;
   A.nseg = (int)G.nseg;
   A.assign = assign;
-  A.segrow = G.row.p;
-  A.segq = G.q.p;
-  A.segdst = G.dst.p;
+  A.segrow = G.row;
+  A.segq = G.q;
+  A.segdst = G.dst;
   A.colSa = P.sa->col.p;
   A.excSa = P.sa->exc.p;
   A.soff = E.soff.p;
@@ -858,7 +858,7 @@ void launch_ab(const SigmaPlan& P, const T* eri, const T* c, T* sigma, hipStream
   if (G.njoin > 0) {
     const int64_t tiles = (P.nb + 255) / 256, nblk = tiles * G.njoin;
     if (nblk > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
-    hipLaunchKernelGGL(k_ab_join<T>, dim3((unsigned)nblk), dim3(256), 0, st, P.nb, tiles, G.jrow.p, G.jptr.p,
+    hipLaunchKernelGGL(k_ab_join<T>, dim3((unsigned)nblk), dim3(256), 0, st, P.nb, tiles, G.jrow, G.jptr,
                        reinterpret_cast<const T*>(G.part.p), sigma);
   }
 }

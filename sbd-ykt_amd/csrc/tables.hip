@@ -298,6 +298,20 @@ __global__ void k_pair_int(const double* __restrict__ eri, int L, int64_t npair,
   W32[t] = (float)v;
 }
 
+// value of a direct pair: orbitals A, B of the bra's pair, I, J of the ket's, six bits each, and
+// the product of the two signs in bit 31
+__global__ void k_direct_values(const uint32_t* __restrict__ word, int64_t n, int L, const double* __restrict__ eri,
+                                double* __restrict__ val, float* __restrict__ val32) {
+  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (q >= n) return;
+  const uint32_t w = word[q];
+  const int A = w & 63, B = (w >> 6) & 63, I = (w >> 12) & 63, J = (w >> 18) & 63;
+  double v = eri4(eri, L, A, I, B, J) - eri4(eri, L, A, J, B, I);
+  if (w >> 31) v = -v;
+  val[q] = v;
+  val32[q] = (float)v;
+}
+
 __global__ void k_pair_slices(const double* __restrict__ eri, int L, int64_t npair, double* __restrict__ Vt,
                               float* __restrict__ Vt32) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -551,15 +565,7 @@ void build_segments(const Table& sa, int64_t nb, int64_t ntiles, AbSegments& g, 
   g.nseg = (int64_t)segs.size();
   g.npart = np;
   g.njoin = (int64_t)jrow.size();
-  auto up = [&](auto& d, const auto& h) {
-    d.alloc(std::max<size_t>(h.size(), 1));
-    if (!h.empty()) SBDG_CHECK(hipMemcpy(d.p, h.data(), sizeof(h[0]) * h.size(), hipMemcpyHostToDevice));
-  };
-  up(g.row, row);
-  up(g.dst, dst);
-  up(g.q, q);
-  up(g.jrow, jrow);
-  up(g.jptr, jptr);
+  g.mem.put({{&g.row, row}, {&g.dst, dst}, {&g.q, q}, {&g.jrow, jrow}, {&g.jptr, jptr}});
   g.part.alloc(std::max<int64_t>((int64_t)np * nb, 1));
 }
 
@@ -758,28 +764,28 @@ void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t 
   SBDG_CHECK(hipMemcpy(e.ent.p, ent.data(), sizeof(uint32_t) * ent.size(), hipMemcpyHostToDevice));
 }
 
-void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* h_eri, int64_t ncols,
+void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* d_eri, int64_t ncols,
                  CoreTable& ct, Table& direct, hipStream_t st) {
   ct.ncore = ct.nmem = ct.zmem = ct.small = ct.nblk = 0;
   const int64_t npp = (int64_t)nel * (nel - 1) / 2;
   const int64_t total = n * npp;
   std::vector<int32_t> start(1, 0), row, pair, blk, blk_x0, grp, slot_ptr(n + 1, 0), slot;
-  // direct pairs of the small cores: (row, column, value), value eps_x eps_y W[P_x][P_y]
+  // direct pairs of the small cores: (row, column, word of k_direct_values), value
+  // eps_x eps_y W[P_x][P_y].  The values are formed on the device: two reads of the integrals a
+  // pair were most of this function's host time (norb=26, 5,000 strings 4.0 ms).
   struct Direct {
     int32_t r, c;
-    double v;
+    uint32_t w;
   };
   std::vector<Direct> dp;
-  // orbitals of every pair index, and their bits
-  std::vector<int8_t> plo, phi;
+  // orbitals of every pair index (six bits each), and their bits
+  std::vector<uint32_t> porb;
   std::vector<uint64_t> pbits;
-  for (int b = 1; b < L; ++b)
-    for (int a = 0; a < b; ++a) {
-      plo.push_back((int8_t)a);
-      phi.push_back((int8_t)b);
+  for (uint32_t b = 1; b < (uint32_t)L; ++b)
+    for (uint32_t a = 0; a < b; ++a) {
+      porb.push_back(a | (b << 6));
       pbits.push_back((1ull << a) | (1ull << b));
     }
-  auto eri4h = [&](int p, int q, int r, int t) { return h_eri[(((int64_t)p * L + q) * L + r) * L + t]; };
   if (total > 0) {
     if (total >= (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "too many core memberships");
     DBuf<uint64_t> key, val, key2, val2;
@@ -843,11 +849,9 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
         for (const Member& x : keep)
           for (const Member& y : keep) {
             if (x.bits & y.bits) continue;  // W = 0 (and x == y)
-            const int Px = x.pair & 0x7FFFFFFF, Py = y.pair & 0x7FFFFFFF;
-            const int A = plo[Px], B = phi[Px], I = plo[Py], J = phi[Py];
-            double v = eri4h(A, I, B, J) - eri4h(A, J, B, I);
-            if ((x.pair < 0) != (y.pair < 0)) v = -v;
-            dp.push_back({x.row, y.row, v});
+            dp.push_back({x.row, y.row,
+                          porb[x.pair & 0x7FFFFFFF] | (porb[y.pair & 0x7FFFFFFF] << 12) |
+                              ((uint32_t)(x.pair ^ y.pair) & 0x80000000u)});
           }
         if (m < CORE_KMIN) {
           ct.small += (int64_t)(dp.size() - before);
@@ -899,14 +903,12 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
     for (const Direct& d : dp) ++rp[d.r + 1];
     for (int64_t r = 0; r < n; ++r) rp[r + 1] += rp[r];
     std::vector<int32_t> dc(dp.size());
-    std::vector<double> dv(dp.size());
-    std::vector<float> dv32(dp.size());
+    std::vector<uint32_t> dw(dp.size());
     std::vector<int64_t> fill(rp.begin(), rp.end() - 1);
     for (const Direct& d : dp) {
       const int64_t q = fill[d.r]++;
       dc[q] = d.c;
-      dv[q] = d.v;
-      dv32[q] = (float)d.v;
+      dw[q] = d.w;
     }
     direct.n = n;
     direct.nnz = (int64_t)dp.size();
@@ -918,8 +920,13 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
     SBDG_CHECK(hipMemcpy(direct.rowptr.p, rp.data(), sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice));
     if (!dp.empty()) {
       SBDG_CHECK(hipMemcpy(direct.col.p, dc.data(), sizeof(int32_t) * dp.size(), hipMemcpyHostToDevice));
-      SBDG_CHECK(hipMemcpy(direct.val.p, dv.data(), sizeof(double) * dp.size(), hipMemcpyHostToDevice));
-      SBDG_CHECK(hipMemcpy(direct.val32.p, dv32.data(), sizeof(float) * dp.size(), hipMemcpyHostToDevice));
+      DBuf<uint32_t> word;
+      word.alloc(dp.size());
+      SBDG_CHECK(hipMemcpy(word.p, dw.data(), sizeof(uint32_t) * dp.size(), hipMemcpyHostToDevice));
+      hipLaunchKernelGGL(k_direct_values, dim3(blocks_for(direct.nnz, 256)), dim3(256), 0, st, word.p, direct.nnz, L,
+                         d_eri, direct.val.p, direct.val32.p);
+      SBDG_CHECK(hipGetLastError());
+      SBDG_CHECK(hipStreamSynchronize(st));
     }
   }
   ct.ncore = (int64_t)start.size() - 1;
