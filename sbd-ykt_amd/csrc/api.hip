@@ -341,6 +341,8 @@ int64_t build_bytes(const sbdg_options& o, int L, int64_t na, int64_t nb, const 
       any_core = true;
       b += 4 * (n + 1) + 28 * mem[sp] + 8 * (n + 1) + 16 * X;  // members, blocks, slots; direct pairs
       zwant = std::max(zwant, mem[sp] * ((nc[sp] + CORE_COLS - 1) / CORE_COLS * CORE_COLS) * 8);
+    } else if (o.doubles != 1) {
+      b += 12 * (n + 1) + 44 * D;  // made for the choice of form and the RDMs: each member has a partner
     }
   }
   if (any_core) b += 12 * npair * npair + std::min<int64_t>(zwant, (int64_t)(o.core_gib * 1073741824.0));
@@ -355,8 +357,10 @@ int64_t build_bytes(const sbdg_options& o, int L, int64_t na, int64_t nb, const 
     b += 4 * (64 * Sb + 64 * AB_BATCH * groups * nch) + 4 * nch * groups * 64 + 16 * groups * nch;
     if (!two) break;  // one table for both precisions
   }
-  // bra-row segments: at most every single its own, and their partial rows
-  b += 16 * (na + nnz[0]) + std::min<int64_t>(AB_PART_BYTES, 8 * nnz[0] * nb);
+  // bra-row segments: one a row and the further ones of eight singles or more, which make joined
+  // rows, and their partial rows
+  const int64_t more = nnz[0] / 8;
+  b += 24 * (na + more) + 8 * std::min(na, more) + std::min<int64_t>(AB_PART_BYTES, 8 * more * nb) + 2048;
   return b;
 }
 
@@ -380,7 +384,7 @@ int64_t rdm_bytes(int L, int64_t na, int64_t nb, const int64_t* nnz) {
   // sums of one batch of keys (runs: at most one per beta pair and tile)
   const int64_t Sa = nnz[0], pairs = nnz[2] / 2, nch = (nb + AB_PAIR_COLS / 2 - 1) / (AB_PAIR_COLS / 2);
   const int64_t tiles = nch * (nch + 1) / 2 + pairs / 1024 + 1, runs = pairs + tiles;
-  const int64_t table = 32 * tiles + 6 * (pairs + 12288 * tiles) + 8 * runs + 4 * (L2 + runs);
+  const int64_t table = 32 * tiles + 6 * (pairs + 12288 * tiles) + 8 * runs + 4 * (L2 + runs) + 4096;
   const int64_t part = std::min(std::max(RDM_PART_BYTES, 16 * runs), 16 * runs * (Sa / 32 + L2));
   peak = std::max(peak, part) + table + sorted;
   return peak + 8 * (2 * L2 + 4 * L4);

@@ -302,3 +302,29 @@ def test_sigma_repeated_calls_several_ket_chunks():
     em = s.run()
     assert s.stats()["sigma_fp32"] > 0 and abs(em - e64) < 1e-6, (em, e64)
     s.close()
+
+
+@pytest.mark.parametrize("norb,nel,na,nb,options", [
+    (40, 20, 60000, 40, dict(doubles=1)), (40, 20, 3000, 40, {}), (26, 5, 5000, 130, {}), (58, 12, 600, 400, {}),
+    (12, 4, 60, 60, {}),
+])
+def test_built_tables_within_plan(norb, nel, na, nb, options):
+    """What a build holds stays within its plan, for sets without a single excitation among them
+    (random strings: one row segment each, nothing else that grows with the strings) too."""
+    rng = np.random.default_rng(37)
+    case = workload_small(norb, 4, 4, 2, 2, 37)
+    if nel == 20:
+        draw = lambda n: np.unique(np.array([np.bitwise_or.reduce(np.uint64(1) << rng.permutation(norb)[:nel].astype(np.uint64))
+                                             for _ in range(n)], dtype=np.uint64))
+        case["astr"], case["bstr"] = draw(na), draw(nb)
+    else:
+        case["astr"], case["bstr"] = syn.sample_strings(norb, nel, na, rng), syn.sample_strings(norb, nel, nb, rng)
+    s = solver(case, **options)
+    before = s.stats()["mem_now"]
+    s.build()
+    st = s.stats()
+    plan = sbdg.memory_plan(norb, s.na, s.nb, st["nnz"], st["core_members"], st["core_direct"], **options)
+    held = st["mem_now"] - before
+    print(f"norb {norb}, {s.na} x {s.nb}: nnz {st['nnz']}, held {held}, planned {plan['build']}", flush=True)
+    assert held <= plan["build"]
+    s.close()
