@@ -94,3 +94,31 @@ def test_rdm_after_new_integrals_and_new_strings():
         assert abs(got[0][1].reshape(c["norb"], -1).trace() - 4) < 1e-11
         fresh.close()
     s.close()
+
+
+@pytest.mark.parametrize("refresh_k", [3, 0])
+@pytest.mark.parametrize("norb,nel,na,nb", [(16, 5, 65, 129), (18, 5, 300, 251)])
+def test_rdm_out_of_a_mixed_solves_vectors(norb, nel, na, nb, refresh_k):
+    """A mixed solve leaves its basis and the FP32 sigma vectors idle (no FP64 ones): the RDMs'
+    buffers come out of those, the vector stays, repeats give the same bits, and the RDMs and
+    gradients are those of an FP64 context that holds the vector (its norm is formed again there:
+    a unit in the last place of every element, so 1e-12 instead of the same bits)."""
+    c = workload_small(norb, nel, nel, na, nb, 97)
+    args = c["norb"], c["core"], c["h1"], c["eri"], c["astr"], c["bstr"]
+    s = sbdg.Solver(*args, max_it=20, max_nb=6, eps=1e-5, precision=1, refresh_k=refresh_k, do_rdm=1)
+    s.run()
+    assert s.stats()["sigma_fp32"] > 0
+    w = s.vector()
+    one, two = s.rdm()
+    grad = s.rdm_backward(1.0)
+    again = (*s.rdm(compute=True), *s.rdm_backward(1.0))
+    assert all(np.array_equal(x, y) for x, y in zip((one, two, *grad), again))
+    assert np.array_equal(s.vector(), w)
+    r = sbdg.Solver(*args, max_it=1, max_nb=2, eps=1e10, init=2, do_rdm=1)
+    r.set_vector(w)
+    r.run()
+    for x, y in zip((one, two, *grad, s.density()), (*r.rdm(), *r.rdm_backward(1.0), r.density())):
+        assert np.abs(x - y).max() < 1e-12
+    rdm_invariants(one, two, nel, nel, norb, 1e-11)
+    s.close()
+    r.close()

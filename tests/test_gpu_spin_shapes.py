@@ -11,7 +11,7 @@ import pytest
 
 import oracle
 import sbdg
-from helpers import workload_small
+from helpers import core_split, workload_small
 
 pytestmark = pytest.mark.gpu
 
@@ -70,3 +70,21 @@ def test_core_pass_of_few_columns_and_many_blocks(na):
     """Rows of up to 128 vectors (256 columns in FP64, 512 in FP32) over the 2,800 product blocks
     of all strings of five electrons in 16 orbitals, and the first row length beyond."""
     check(workload_small(16, 5, 5, na, 0, 73), doubles=2).close()
+
+
+def test_core_passes_end_with_one_column():
+    """1,025 of the 1,287 strings of five electrons in 13 orbitals on either side, most of whose
+    cores go through the workspace, with the workspace capped at one 512-column pass of the cores
+    of ten members and more: both precisions take several passes, the last of a single column."""
+    case = workload_small(13, 5, 5, 1025, 1025, 89)
+    s = check(case, doubles=2)
+    members = s.stats()["core_members"]
+    s.close()
+    cap = max(members) * 512 * 8
+    for strs, kept in zip((case["astr"], case["bstr"]), members):
+        assert core_split(strs)[0] == kept
+        through = core_split(strs, 28)[0]
+        for size in (8, 4):
+            columns = cap // (size * through) // 512 * 512
+            assert 512 <= columns < 1025 and 1025 % columns == 1
+    check(case, doubles=2, core_gib=(cap + 64) / 2**30).close()
