@@ -921,8 +921,10 @@ struct KeySegments {
   std::vector<int32_t> keys, krange, kseg, segs;
   std::vector<std::pair<size_t, size_t>> batch;
   int64_t widest = 0;  // segments of the largest batch
-  WBuf<int32_t> dkeys, dkrange, dkseg, dsegs;
-  explicit KeySegments(Arena& ar) : dkeys(ar), dkrange(ar), dkseg(ar), dsegs(ar) {}
+  const int32_t *dkeys = nullptr, *dkrange = nullptr, *dkseg = nullptr, *dsegs = nullptr;
+  std::vector<int32_t> lists;  // the four, copied at once
+  WBuf<int32_t> dlists;
+  explicit KeySegments(Arena& ar) : dlists(ar) {}
 };
 
 void key_segments(const std::vector<int32_t>& hk, int L, int64_t len, int64_t most, KeySegments& K, hipStream_t st) {
@@ -945,15 +947,14 @@ void key_segments(const std::vector<int32_t>& hk, int L, int64_t len, int64_t mo
     K.widest = std::max<int64_t>(K.widest, K.kseg[f] - K.kseg[k]);
     k = f;
   }
-  auto up = [&](WBuf<int32_t>& d, const std::vector<int32_t>& h) {
-    d.alloc(std::max<size_t>(h.size(), 1));
-    if (!h.empty())
-      SBDG_CHECK(hipMemcpyAsync(d.p, h.data(), sizeof(int32_t) * h.size(), hipMemcpyHostToDevice, st));
-  };
-  up(K.dkeys, K.keys);
-  up(K.dkrange, K.krange);
-  up(K.dkseg, K.kseg);
-  up(K.dsegs, K.segs);
+  const std::vector<int32_t>* all[] = {&K.keys, &K.krange, &K.kseg, &K.segs};
+  for (const auto* h : all) K.lists.insert(K.lists.end(), h->begin(), h->end());
+  K.dlists.alloc(K.lists.size());
+  SBDG_CHECK(hipMemcpyAsync(K.dlists.p, K.lists.data(), sizeof(int32_t) * K.lists.size(), hipMemcpyHostToDevice, st));
+  K.dkeys = K.dlists.p;
+  K.dkrange = K.dkeys + K.keys.size();
+  K.dkseg = K.dkrange + K.krange.size();
+  K.dsegs = K.dkseg + K.kseg.size();
 }
 
 // singles of one spin: pair sums by key segment, their occupation parts, then key owners
@@ -975,15 +976,15 @@ void singles_part(const Table& t, const SortedSingles& ss, int L, int s, const d
     if (ns * ntiles > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
     if (NV == 2)
       hipLaunchKernelGGL(k_pair_sums<2>, dim3((unsigned)(ns * ntiles)), dim3(RT), 0, st, ncols, ntiles, ns,
-                         K.dsegs.p + 2 * s0, ss.pia.p, ss.pja.p, t.nnz, X, D.p, gpart.p);
+                         K.dsegs + 2 * s0, ss.pia.p, ss.pja.p, t.nnz, X, D.p, gpart.p);
     else
       hipLaunchKernelGGL(k_pair_sums<1>, dim3((unsigned)(ns * ntiles)), dim3(RT), 0, st, ncols, ntiles, ns,
-                         K.dsegs.p + 2 * s0, ss.pia.p, ss.pja.p, t.nnz, X, D.p, gpart.p);
+                         K.dsegs + 2 * s0, ss.pia.p, ss.pja.p, t.nnz, X, D.p, gpart.p);
     hipLaunchKernelGGL(k_occ_contract<false>, dim3((unsigned)ns), dim3(RT), 0, st, ncols, D.p, cstr, occ.p + s0 * 64,
                        nullptr);
   }
-  hipLaunchKernelGGL(k_single_slots, dim3((unsigned)K.keys.size()), dim3(RT), 0, st, L, s, K.dkeys.p, K.dkrange.p,
-                     K.dkseg.p, ss.pia.p, ss.pja.p, rstr, t.nnz, ntiles, gpart.p, occ.p, one, two);
+  hipLaunchKernelGGL(k_single_slots, dim3((unsigned)K.keys.size()), dim3(RT), 0, st, L, s, K.dkeys, K.dkrange,
+                     K.dkseg, ss.pia.p, ss.pja.p, rstr, t.nnz, ntiles, gpart.p, occ.p, one, two);
   SBDG_CHECK(hipGetLastError());
   SBDG_CHECK(hipStreamSynchronize(st));
 }
@@ -1318,13 +1319,13 @@ void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* one, dou
       const int64_t nblk = (ns + 7) / 8 * 8 * ab.ntiles;
       if (nblk > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
       A.nseg = ns;
-      A.segptr = K.dsegs.p + 2 * s0;
+      A.segptr = K.dsegs + 2 * s0;
       const dim3 g((unsigned)nblk), t(ab.nt);
       if (many) hipLaunchKernelGGL(k_ab_rdm, g, t, lds, st, A);
       else if (ab.sp > 1) hipLaunchKernelGGL(k_ab_rdm_small<4>, g, t, lds, st, A);
       else hipLaunchKernelGGL(k_ab_rdm_small<1>, g, t, lds, st, A);
       hipLaunchKernelGGL(k_ab_slots, dim3((unsigned)(bt.second - bt.first)), dim3(256), 0, st, L,
-                         K.dkeys.p + bt.first, K.dkseg.p + bt.first, s0, ab.nruns, ab.pairptr, ab.pairrun, part.p, two);
+                         K.dkeys + bt.first, K.dkseg + bt.first, s0, ab.nruns, ab.pairptr, ab.pairrun, part.p, two);
     }
     SBDG_CHECK(hipGetLastError());
     SBDG_CHECK(hipStreamSynchronize(st));

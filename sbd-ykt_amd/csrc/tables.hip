@@ -298,18 +298,28 @@ __global__ void k_pair_int(const double* __restrict__ eri, int L, int64_t npair,
   W32[t] = (float)v;
 }
 
-// value of a direct pair: orbitals A, B of the bra's pair, I, J of the ket's, six bits each, and
-// the product of the two signs in bit 31
-__global__ void k_direct_values(const uint32_t* __restrict__ word, int64_t n, int L, const double* __restrict__ eri,
-                                double* __restrict__ val, float* __restrict__ val32) {
-  const int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (q >= n) return;
-  const uint32_t w = word[q];
-  const int A = w & 63, B = (w >> 6) & 63, I = (w >> 12) & 63, J = (w >> 18) & 63;
-  double v = eri4(eri, L, A, I, B, J) - eri4(eri, L, A, J, B, I);
-  if (w >> 31) v = -v;
-  val[q] = v;
-  val32[q] = (float)v;
+// The direct pairs of member z of a small core, from its place in the table on: every member of the
+// core, in order, whose pair shares no orbital with z's; value eps_x eps_y W[P_x][P_y].  mem: row,
+// orbitals of the pair (six bits each, bit 31 the sign), first member of the core and their number.
+__global__ void k_direct_fill(const int4* __restrict__ mem, const int64_t* __restrict__ at, int64_t n, int L,
+                              const double* __restrict__ eri, int32_t* __restrict__ col, double* __restrict__ val,
+                              float* __restrict__ val32) {
+  const int64_t z = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (z >= n) return;
+  const int4 x = mem[z];
+  const int A = x.y & 63, B = (x.y >> 6) & 63;
+  int64_t q = at[z];
+  for (int k = 0; k < x.w; ++k) {
+    const int4 y = mem[x.z + k];
+    const int I = y.y & 63, J = (y.y >> 6) & 63;
+    if (A == I || A == J || B == I || B == J) continue;
+    double v = eri4(eri, L, A, I, B, J) - eri4(eri, L, A, J, B, I);
+    if ((x.y ^ y.y) < 0) v = -v;
+    col[q] = y.x;
+    val[q] = v;
+    val32[q] = (float)v;
+    ++q;
+  }
 }
 
 __global__ void k_pair_slices(const double* __restrict__ eri, int L, int64_t npair, double* __restrict__ Vt,
@@ -770,14 +780,11 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
   const int64_t npp = (int64_t)nel * (nel - 1) / 2;
   const int64_t total = n * npp;
   std::vector<int32_t> start(1, 0), row, pair, blk, blk_x0, grp, slot_ptr(n + 1, 0), slot;
-  // direct pairs of the small cores: (row, column, word of k_direct_values), value
-  // eps_x eps_y W[P_x][P_y].  The values are formed on the device: two reads of the integrals a
-  // pair were most of this function's host time (norb=26, 5,000 strings 4.0 ms).
-  struct Direct {
-    int32_t r, c;
-    uint32_t w;
-  };
-  std::vector<Direct> dp;
+  // members of the small cores as k_direct_fill takes them, and the pairs of each.  Only counted
+  // here: pairs listed and valued on the host were most of this function's time (norb=16, 2,703
+  // strings, half a million pairs: 2 of 2.4 ms).
+  std::vector<int4> dmem;
+  std::vector<int32_t> dcnt;
   // orbitals of every pair index (six bits each), and their bits
   std::vector<uint32_t> porb;
   std::vector<uint64_t> pbits;
@@ -845,16 +852,17 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
           }
       const int64_t m = (int64_t)keep.size();
       if (m >= 2 && m < CORE_ZMIN) {
-        const size_t before = dp.size();
-        for (const Member& x : keep)
-          for (const Member& y : keep) {
-            if (x.bits & y.bits) continue;  // W = 0 (and x == y)
-            dp.push_back({x.row, y.row,
-                          porb[x.pair & 0x7FFFFFFF] | (porb[y.pair & 0x7FFFFFFF] << 12) |
-                              ((uint32_t)(x.pair ^ y.pair) & 0x80000000u)});
-          }
+        const int32_t base = (int32_t)dmem.size();
+        int64_t pairs = 0;
+        for (const Member& x : keep) {
+          int32_t with = 0;
+          for (const Member& y : keep) with += (x.bits & y.bits) == 0;  // else W = 0 (and x == y)
+          dmem.push_back(make_int4(x.row, (int)(porb[x.pair & 0x7FFFFFFF] | ((uint32_t)x.pair & 0x80000000u)), base, (int)m));
+          dcnt.push_back(with);
+          pairs += with;
+        }
         if (m < CORE_KMIN) {
-          ct.small += (int64_t)(dp.size() - before);
+          ct.small += pairs;
         } else {
           mids.insert(mids.end(), keep.begin(), keep.end());
           midsize.push_back((int32_t)m);
@@ -897,34 +905,32 @@ void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double*
     std::vector<int32_t> fillp(slot_ptr.begin(), slot_ptr.end() - 1);
     for (int64_t q = 0; q < ct.zmem; ++q) slot[fillp[row[q]]++] = (int32_t)q;
   }
-  // the direct pairs as a CSR table (rows ascending; any order inside a row)
+  // the direct pairs as a CSR table (rows ascending, a row's by core)
   {
-    std::vector<int64_t> rp(n + 1, 0);
-    for (const Direct& d : dp) ++rp[d.r + 1];
+    std::vector<int64_t> rp(n + 1, 0), at(dmem.size());
+    for (size_t z = 0; z < dmem.size(); ++z) rp[dmem[z].x + 1] += dcnt[z];
     for (int64_t r = 0; r < n; ++r) rp[r + 1] += rp[r];
-    std::vector<int32_t> dc(dp.size());
-    std::vector<uint32_t> dw(dp.size());
     std::vector<int64_t> fill(rp.begin(), rp.end() - 1);
-    for (const Direct& d : dp) {
-      const int64_t q = fill[d.r]++;
-      dc[q] = d.c;
-      dw[q] = d.w;
+    for (size_t z = 0; z < dmem.size(); ++z) {
+      at[z] = fill[dmem[z].x];
+      fill[dmem[z].x] += dcnt[z];
     }
     direct.n = n;
-    direct.nnz = (int64_t)dp.size();
+    direct.nnz = rp[n];
+    const size_t nnz = (size_t)std::max<int64_t>(rp[n], 1);
     direct.rowptr.alloc(n + 1);
-    direct.col.alloc(std::max<size_t>(dp.size(), 1));
+    direct.col.alloc(nnz);
     direct.exc.alloc(1);
-    direct.val.alloc(std::max<size_t>(dp.size(), 1));
-    direct.val32.alloc(std::max<size_t>(dp.size(), 1));
+    direct.val.alloc(nnz);
+    direct.val32.alloc(nnz);
     SBDG_CHECK(hipMemcpy(direct.rowptr.p, rp.data(), sizeof(int64_t) * (n + 1), hipMemcpyHostToDevice));
-    if (!dp.empty()) {
-      SBDG_CHECK(hipMemcpy(direct.col.p, dc.data(), sizeof(int32_t) * dp.size(), hipMemcpyHostToDevice));
-      DBuf<uint32_t> word;
-      word.alloc(dp.size());
-      SBDG_CHECK(hipMemcpy(word.p, dw.data(), sizeof(uint32_t) * dp.size(), hipMemcpyHostToDevice));
-      hipLaunchKernelGGL(k_direct_values, dim3(blocks_for(direct.nnz, 256)), dim3(256), 0, st, word.p, direct.nnz, L,
-                         d_eri, direct.val.p, direct.val32.p);
+    if (direct.nnz > 0) {
+      TableMem t;
+      const int4* mem;
+      const int64_t* place;
+      t.put({{&mem, dmem}, {&place, at}});
+      hipLaunchKernelGGL(k_direct_fill, dim3(blocks_for((int64_t)dmem.size(), 256)), dim3(256), 0, st, mem, place,
+                         (int64_t)dmem.size(), L, d_eri, direct.col.p, direct.val.p, direct.val32.p);
       SBDG_CHECK(hipGetLastError());
       SBDG_CHECK(hipStreamSynchronize(st));
     }
