@@ -895,9 +895,11 @@ void sigma_apply(const SigmaPlan& P, const T* c, T* sigma, const SigmaScratch<T>
   // the alpha-beta terms (LDS-bound) into their own buffer on the second stream, while the
   // spin phases (HBM-bound) run on this one; the transpose-add joins them.  Below 100,000
   // determinants the fork and join cost more than the overlap gains (239^2 strings: 86 us
-  // with it, 69 in sequence; 275^2: 95 and 89; 500 x 321: 125 and 152).
+  // with it, 69 in sequence; 275^2: 95 and 89; 500 x 321: 125 and 152), unless rows are so wide
+  // that both sides are long for a few determinants (2 x 13,922: 442 and 490; 4 x 20,000: 445 and
+  // 557; 3 x 8,000: 188 and 176).
   T* sab = scr.sab;
-  const bool ab = ab_any(P.nb), beside = P.st2 && ab && P.na * P.nb >= 100000;
+  const bool ab = ab_any(P.nb), beside = P.st2 && ab && (P.na * P.nb >= 100000 || P.nb >= 10000);
   if (beside) {
     SBDG_CHECK(hipEventRecord(P.fork, st));
     SBDG_CHECK(hipStreamWaitEvent(P.st2, P.fork, 0));
