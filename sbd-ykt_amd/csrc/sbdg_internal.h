@@ -110,6 +110,7 @@ class TableMem {
     }
     if (!host.empty()) SBDG_CHECK(hipMemcpy(mem_.p, host.data(), total, hipMemcpyHostToDevice));
   }
+  void free() { mem_.free(); }
 
  private:
   static constexpr size_t SMALL = 1 << 20;
@@ -290,15 +291,13 @@ struct EllTable {
   int nt = 0, m = 0, s = 1;  // alpha-beta launch: threads per workgroup, columns per thread, groups staged at once
   int64_t chunk = 0, groups = 0, ntiles = 0;
   int64_t kbase = 0;        // first ket vector (16-byte units): after the slice vectors
-  DBuf<int64_t> soff;       // ntiles*(nt/64)*nch + 1: start of each wave's entry stream per chunk
-  DBuf<int32_t> nq;         // ntiles*(nt/64)*nch*m: four-row batches of each group of the stream
-  DBuf<uint32_t> ent;
-  DBuf<int32_t> colperm;    // nch * groups*64: column of each lane position in each chunk (-1: none)
+  TableMem mem;
+  const int64_t* soff;      // ntiles*(nt/64)*nch + 1: start of each wave's entry stream per chunk
+  const int32_t* nq;        // ntiles*(nt/64)*nch*m: four-row batches of each group of the stream
+  const uint32_t* ent;
+  const int32_t* colperm;   // nch * groups*64: column of each lane position in each chunk (-1: none)
   void release() {
-    soff.free();
-    nq.free();
-    ent.free();
-    colperm.free();
+    mem.free();
     nch = nt = m = 0;
   }
 };

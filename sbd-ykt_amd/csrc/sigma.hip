@@ -802,10 +802,10 @@ void launch_ab_m(const SigmaPlan& P, size_t lds, const T* eri, const T* c, T* si
   A.segdst = G.dst;
   A.colSa = P.sa->col.p;
   A.excSa = P.sa->exc.p;
-  A.soff = E.soff.p;
-  A.nq = E.nq.p;
-  A.ent = E.ent.p;
-  A.colperm = E.colperm.p;
+  A.soff = E.soff;
+  A.nq = E.nq;
+  A.ent = E.ent;
+  A.colperm = E.colperm;
   A.Vt = eri;
   A.c = c;
   A.sigma = sigma;

@@ -547,35 +547,51 @@ void build_segments(const Table& sa, int64_t nb, int64_t ntiles, AbSegments& g, 
     return e;
   };
   while (extra(len) * nb * (int64_t)sizeof(double) > AB_PART_BYTES) len *= 2;
-  struct Seg {
-    int32_t row, dst;
-    int64_t q0, q1;
-  };
-  std::vector<Seg> segs;
-  std::vector<int32_t> jrow, jptr(1, 0);
-  int32_t np = 0;
-  for (int64_t r = 0; r < na; ++r) {
-    segs.push_back({(int32_t)r, -1, rp[r], std::min(rp[r + 1], rp[r] + len)});
-    if (rp[r] + len < rp[r + 1]) {
-      for (int64_t q = rp[r] + len; q < rp[r + 1]; q += len)
-        segs.push_back({(int32_t)r, np++, q, std::min(rp[r + 1], q + len)});
-      jrow.push_back((int32_t)r);
-      jptr.push_back(np);
+  // every row's segments of l singles, the last one shorter: the row's first writes sigma (dst -1)
+  auto each = [&](auto&& f) {
+    int32_t np = 0;
+    for (int64_t r = 0; r < na; ++r) {
+      int64_t q = rp[r];
+      do {
+        const int64_t end = std::min(rp[r + 1], q + len);
+        f(r, q, end, q == rp[r] ? -1 : np++);
+        q = end;
+      } while (q < rp[r + 1]);
     }
+  };
+  std::vector<int64_t> at(std::min<int64_t>(len, rp[na]) + 2, 0);  // by decreasing length
+  auto place = [&](int64_t l) -> int64_t& { return at[at.size() - 1 - l]; };
+  int32_t np = 0;
+  std::vector<int32_t> jrow, jptr(1, 0);
+  each([&](int64_t r, int64_t q, int64_t end, int32_t dst) {
+    ++place(end - q);
+    if (dst < 0) return;
+    np = dst + 1;
+    if (jrow.empty() || jrow.back() != r) {
+      jrow.push_back((int32_t)r);
+      jptr.push_back(0);
+    }
+    jptr.back() = np;
+  });
+  int64_t nseg = 0;
+  for (int64_t& x : at) {
+    const int64_t k = x;
+    x = nseg;
+    nseg += k;
   }
-  std::stable_sort(segs.begin(), segs.end(), [](const Seg& x, const Seg& y) { return x.q1 - x.q0 > y.q1 - y.q0; });
-  std::vector<int32_t> row, dst;
-  std::vector<int64_t> q;
-  for (const Seg& x : segs) {
-    row.push_back(x.row);
-    dst.push_back(x.dst);
-    q.push_back(x.q0);
-    q.push_back(x.q1);
-  }
-  g.nseg = (int64_t)segs.size();
+  std::vector<int32_t> row(nseg), to(nseg);
+  std::vector<int64_t> q(2 * nseg);
+  each([&](int64_t r, int64_t q0, int64_t q1, int32_t dst) {
+    const int64_t k = place(q1 - q0)++;
+    row[k] = (int32_t)r;
+    to[k] = dst;
+    q[2 * k] = q0;
+    q[2 * k + 1] = q1;
+  });
+  g.nseg = nseg;
   g.npart = np;
   g.njoin = (int64_t)jrow.size();
-  g.mem.put({{&g.row, row}, {&g.dst, dst}, {&g.q, q}, {&g.jrow, jrow}, {&g.jptr, jptr}});
+  g.mem.put({{&g.row, row}, {&g.dst, to}, {&g.q, q}, {&g.jrow, jrow}, {&g.jptr, jptr}});
   g.part.alloc(std::max<int64_t>((int64_t)np * nb, 1));
 }
 
@@ -667,16 +683,16 @@ void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t 
   const int nch = e.nch;
   const int64_t ng = e.groups * nch;
   // host copies of the beta singles
-  SBDG_CHECK(hipStreamSynchronize(st));
-  std::vector<int64_t> rp(nb + 1);
-  SBDG_CHECK(hipMemcpy(rp.data(), sb.rowptr.p, sizeof(int64_t) * (nb + 1), hipMemcpyDeviceToHost));
-  const int64_t nnz = rp[nb];
+  const int64_t nnz = sb.nnz;
+  std::vector<int64_t> rp(nb + 1, 0);
   std::vector<int32_t> col(nnz);
   std::vector<uint32_t> exc(nnz);
+  SBDG_CHECK(hipMemcpyAsync(rp.data(), sb.rowptr.p, sizeof(int64_t) * (nb + 1), hipMemcpyDeviceToHost, st));
   if (nnz) {
-    SBDG_CHECK(hipMemcpy(col.data(), sb.col.p, sizeof(int32_t) * nnz, hipMemcpyDeviceToHost));
-    SBDG_CHECK(hipMemcpy(exc.data(), sb.exc.p, sizeof(uint32_t) * nnz, hipMemcpyDeviceToHost));
+    SBDG_CHECK(hipMemcpyAsync(col.data(), sb.col.p, sizeof(int32_t) * nnz, hipMemcpyDeviceToHost, st));
+    SBDG_CHECK(hipMemcpyAsync(exc.data(), sb.exc.p, sizeof(uint32_t) * nnz, hipMemcpyDeviceToHost, st));
   }
+  SBDG_CHECK(hipStreamSynchronize(st));
   // entries of column ib in chunk k: its singles with ket in the chunk
   std::vector<int32_t> cnt((size_t)nb * nch, 0);
   for (int64_t ib = 0; ib < nb; ++ib)
@@ -764,14 +780,7 @@ void build_ell(const Table& sb, int L, int prec_bytes, EllTable& e, hipStream_t 
       }
       schedule_block(lists, K[g * nch + k], pad, ent.data() + base);
     }
-  e.colperm.alloc(perm.size());
-  SBDG_CHECK(hipMemcpy(e.colperm.p, perm.data(), sizeof(int32_t) * perm.size(), hipMemcpyHostToDevice));
-  e.nq.alloc(nq.size());
-  SBDG_CHECK(hipMemcpy(e.nq.p, nq.data(), sizeof(int32_t) * nq.size(), hipMemcpyHostToDevice));
-  e.soff.alloc(soff.size());
-  SBDG_CHECK(hipMemcpy(e.soff.p, soff.data(), sizeof(int64_t) * soff.size(), hipMemcpyHostToDevice));
-  e.ent.alloc(ent.size());
-  SBDG_CHECK(hipMemcpy(e.ent.p, ent.data(), sizeof(uint32_t) * ent.size(), hipMemcpyHostToDevice));
+  e.mem.put({{&e.soff, soff}, {&e.nq, nq}, {&e.ent, ent}, {&e.colperm, perm}});
 }
 
 void build_cores(const uint64_t* d_str, int64_t n, int L, int nel, const double* d_eri, int64_t ncols,
