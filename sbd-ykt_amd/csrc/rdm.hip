@@ -885,7 +885,7 @@ int bits_for(uint64_t v) {
 }
 
 // The singles of one spin sorted by key: pia/pja as k_alpha_pairs writes them, hk[key] the
-// first of key (host).  nkey keys (a, i) with a > i hold pairs.
+// first of key (host; L^2 + 1 of them).
 struct SortedSingles {
   explicit SortedSingles(Arena& ar) : pia(ar), pja(ar) {}
   WBuf<int32_t> pia, pja;

@@ -525,7 +525,7 @@ struct RdmPlan {
 void build_ab_pairs(const Table& sb, int L, AbPairs& ab, hipStream_t st);
 // one[2][L^2], two[4][L^4] in the reference layout (correlation.h:194-444) from the
 // separated-convention vector W; WT: scratch of na*nb doubles (W transposed).  Bitwise
-// reproducible: every sum is taken in a fixed order or as exact integer (fixed-point) adds.
+// reproducible: every sum is taken in a fixed order.
 // Transient buffers come out of ar where they fit.
 void rdm_compute(const RdmPlan& P, const double* W, double* WT, double* d_one, double* d_two, Arena& ar,
                  hipStream_t st);

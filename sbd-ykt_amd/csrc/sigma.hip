@@ -847,7 +847,6 @@ void launch_ab(const SigmaPlan& P, const T* eri, const T* c, T* sigma, hipStream
   SBDG_AB(1024, 20, 1)
   SBDG_AB(1024, 24, 1)
   if constexpr (sizeof(T) == 8) {
-    SBDG_AB(768, 32, 1)
     SBDG_AB(768, 40, 1)
     SBDG_AB(768, 48, 1)
     SBDG_AB(768, 53, 1)

@@ -518,7 +518,7 @@ AbGeometry ab_geometry(int64_t nb, int L, int elem) {
   g.chunk = std::max<int64_t>(1, (nb + nch - 1) / nch);
   static const int m64[] = {1, 2, 0}, m128[] = {1, 0}, m256[] = {1, 2, 4, 0}, m512[] = {4, 6, 8, 10, 12, 0},
                    m1024d[] = {8, 12, 16, 20, 24, 0}, m1024f[] = {8, 12, 16, 20, 24, 40, 48, 0},
-                   m768[] = {32, 40, 48, 53, 0};
+                   m768[] = {40, 48, 53, 0};
   const int* ms = g.nt == 64 ? m64 : g.nt == 128 ? m128 : g.nt == 256 ? m256 : g.nt == 512 ? m512 : g.nt == 768 ? m768
                   : elem == 4 ? m1024f : m1024d;
   g.m = 0;
