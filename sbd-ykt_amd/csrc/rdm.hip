@@ -572,11 +572,11 @@ __global__ void k_keyseg(int64_t n, int nkeys, const uint32_t* __restrict__ keys
 // and two FMAs, and no table is read.  At the end the sums go through LDS and each run of pairs
 // with one (b, j) is summed in a fixed order by one wave: no atomics, the same bits every time.
 //
-// Bound: the 16-byte LDS gathers (with the pairs ordered by order_pairs a read takes 4.6 clocks
-// and 0.4 of bank conflicts, unordered 4.1 of conflicts) and the latency of the next rows, about
-// evenly.  Before, every product was a fixed-point 64-bit LDS atomic into the L^2 sums of one
-// key, with the pairs re-read from their table for each alpha pair: norb=16 full space 108 ms,
-// norb=36 4,000 x 20,000 strings 57; now 11.5 and 8.9.  On the way, the same two sets: two
+// Bound: the 16-byte LDS gathers (ordered by order_pairs they spend 0.38 bank-conflict cycles an
+// LDS instruction at norb=16, full space, and 0.62 at norb=36, 4,000 x 20,000 strings) and the
+// latency of the next rows, about evenly.  Before, every product was a fixed-point 64-bit LDS
+// atomic into the L^2 sums of one key, with the pairs re-read from their table for each alpha
+// pair: those two sets 108 ms and 57; now 11.0 and 8.6.  On the way, the same two sets: two
 // workgroups of 512 threads and 8,192 pairs on a CU 14.4 and 9.1 ms, of 6,144 pairs 19.8 and 9.1
 // (an alpha pair costs its staging latency, not its pairs); one of 1,024 threads with the next
 // rows in registers 14.3 and 10.4; ordered pairs, empty rounds skipped, one column per load

@@ -484,10 +484,10 @@ struct AbArgs {
 // its own exec region (as a condition on the row and the column compiles) k_ab<double> took
 // 83.9 ms at norb=36, 20,000^2 strings (FP32 45.0) and staging alone 29.6 of them; issued
 // together 69.5 (37.6), with two columns per load 68.1 (37.1), with the entries ordered over the
-// lanes one LDS cycle serves 61.2 (33.9); norb=26, 2,801 x 2,749: 1.56 -> 0.80 ms.  Rows of few columns take S groups per barrier
+// lanes one LDS cycle serves 60.7 (33.9); norb=26, 2,801 x 2,749: 1.56 -> 0.80 ms.  Rows of few columns take S groups per barrier
 // (239^2 at norb=18: 25 -> 21 us at S = 4).  Cutting rows into segments of their alpha
-// singles (build_segments) took norb=18, 239^2 from 132 to 26 us and norb=58, 200 x 40,000
-// from 6.7 to 1.0 ms: the Hartree-Fock row has ten times the singles of the average row.
+// singles (build_segments) took norb=18, 239^2 from 132 to 21 us and norb=58, 200 x 40,000
+// from 6.7 to 0.78 ms: the Hartree-Fock row has ten times the singles of the average row.
 // Measured and not kept: batches of two rows (the shorter padding is no gain: the
 // padding reads one broadcast address), two batches in flight, two column tiles per row with
 // two workgroups on a CU at norb=36, 20,000^2 (91.8 ms: the ket rows are staged twice).
@@ -673,10 +673,11 @@ __global__ void __launch_bounds__(NT, NT == 768 ? 3 : 4) k_ab(const AbArgs<T> A)
 // tiles are one grid dimension: the rows with partial rows are as many as the alpha strings, and
 // a second dimension ends at 65,535.
 template <class T>
-__global__ void __launch_bounds__(256) k_ab_join(int64_t nb, int64_t ntiles, const int32_t* __restrict__ jrow,
+__global__ void __launch_bounds__(256) k_ab_join(int64_t nb, unsigned ntiles, const int32_t* __restrict__ jrow,
                                                  const int32_t* __restrict__ jptr, const T* __restrict__ part,
                                                  T* __restrict__ out) {
-  const int64_t j = blockIdx.x / ntiles, c = (blockIdx.x % ntiles) * 256 + threadIdx.x;
+  const unsigned j = blockIdx.x / ntiles;
+  const int64_t c = (int64_t)(blockIdx.x - j * ntiles) * 256 + threadIdx.x;
   if (c >= nb) return;
   const int64_t r = jrow[j];
   T v = out[r * nb + c];
@@ -860,7 +861,7 @@ void launch_ab(const SigmaPlan& P, const T* eri, const T* c, T* sigma, hipStream
   if (G.njoin > 0) {
     const int64_t tiles = (P.nb + 255) / 256, nblk = tiles * G.njoin;
     if (nblk > (int64_t)INT32_MAX) throw Error(SBDG_ERR_LIMIT, "grid too large");
-    hipLaunchKernelGGL(k_ab_join<T>, dim3((unsigned)nblk), dim3(256), 0, st, P.nb, tiles, G.jrow, G.jptr,
+    hipLaunchKernelGGL(k_ab_join<T>, dim3((unsigned)nblk), dim3(256), 0, st, P.nb, (unsigned)tiles, G.jrow, G.jptr,
                        reinterpret_cast<const T*>(G.part.p), sigma);
   }
 }
