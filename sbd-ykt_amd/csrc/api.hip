@@ -98,6 +98,7 @@ struct sbdg_ctx {
   CoreTable Ca, Cb;       // same-spin doubles by core (used when use_ca / use_cb)
   Table Xa, Xb;           // the pairs of the small cores, read directly (with Ca / Cb)
   bool use_ca = false, use_cb = false;
+  bool have_cores = false;  // Ca and Cb were made by the last build (its doubles option was not 1)
   DBuf<double> Ja, Jb;    // occupation tables of the alpha / beta strings
   DBuf<float> Ja32, Jb32;
   DBuf<double> Vt;        // alpha-beta integral slices by orbital pair
@@ -203,7 +204,8 @@ void build(sbdg_ctx* c) {
   // when the table would stream more than four times the member rows a core pass moves.
   const int nel_a = na ? __builtin_popcountll(c->a[0]) : 0, nel_b = nb ? __builtin_popcountll(c->b[0]) : 0;
   c->use_ca = c->use_cb = false;
-  if (c->opt.doubles != 1) {
+  c->have_cores = c->opt.doubles != 1;
+  if (c->have_cores) {
     build_cores(c->d_a.p, na, L, nel_a, c->d_eri.p, nb, c->Ca, c->Xa, c->st);
     build_cores(c->d_b.p, nb, L, nel_b, c->d_eri.p, na, c->Cb, c->Xb, c->st);
     // auto: the core form (its workspace for the larger cores, the pairs of the smaller
@@ -837,7 +839,7 @@ void rdm_or_density(sbdg_ctx* c) {
     P.db = &c->Db;
     if (!c->abp.built) build_ab_pairs(c->Sb, L, c->abp, c->st);
     P.ab = &c->abp;
-    if (c->opt.doubles != 1) {  // the core tables exist (built for sigma, used or not)
+    if (c->have_cores) {  // made for sigma, used there or not; the option may have changed since
       P.ca = &c->Ca;
       P.cb = &c->Cb;
     }

@@ -122,3 +122,27 @@ def test_rdm_out_of_a_mixed_solves_vectors(norb, nel, na, nb, refresh_k):
     rdm_invariants(one, two, nel, nel, norb, 1e-11)
     s.close()
     r.close()
+
+
+def test_rdm_after_the_doubles_option_changed():
+    """Core tables of an earlier string set must not serve a later one that was built without:
+    a context with cores of 1,287 strings, then 200 strings by excitation table, then the option
+    set back before the RDMs of that solution are asked for."""
+    big = workload_small(13, 5, 5, 0, 60, 101)
+    small = workload_small(13, 5, 5, 200, 60, 102)
+    options = dict(max_it=1, max_nb=2, eps=1e10, init=1, seed=9)
+    s = sbdg.Solver(13, big["core"], big["h1"], big["eri"], big["astr"], big["bstr"], doubles=2, **options)
+    s.run()
+    s.astr, s.na = small["astr"], len(small["astr"])
+    s.bstr, s.nb = small["bstr"], len(small["bstr"])
+    s.set_options(doubles=1, **options)
+    s.set_integrals(small["core"], small["h1"], small["eri"])
+    s.run()
+    s.set_options(doubles=0, **options)
+    got = s.rdm(compute=True)
+    fresh = sbdg.Solver(13, small["core"], small["h1"], small["eri"], small["astr"], small["bstr"], doubles=1, **options)
+    fresh.run()
+    want = fresh.rdm(compute=True)
+    assert all(np.array_equal(x, y) for x, y in zip(got, want))
+    s.close()
+    fresh.close()
