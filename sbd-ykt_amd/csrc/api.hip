@@ -969,14 +969,46 @@ int sbdg_set_integrals(sbdg_ctx* c, int norb, double core, const double* h1, con
     if (!h1 || !eri) return fail(c, SBDG_ERR_ARG, "null integral pointer");
     const int L = norb;
     const int64_t L4 = (int64_t)L * L * L * L;
-    if (c->L != L) c->abp.built = false;
+    if (layout != 0 && layout != 1) return fail(c, SBDG_ERR_ARG, "eri_layout must be 0 or 1");
+    // checked as they come: a refused call leaves the context as it was
+    const int64_t np = (int64_t)L * (L + 1) / 2, given = layout == 0 ? L4 : np * (np + 1) / 2;
+    for (int64_t k = 0; k < (int64_t)L * L; ++k)
+      if (!std::isfinite(h1[k])) return fail(c, SBDG_ERR_ARG, "non-finite one-electron integral");
+    for (int64_t k = 0; k < given; ++k)
+      if (!std::isfinite(eri[k])) return fail(c, SBDG_ERR_ARG, "non-finite two-electron integral");
+    if (layout == 0) {
+      // the kernels read (pq|rs) through its images ((ai|bj) for b < j from (ai|jb) in the
+      // alpha-beta kernel): the tensor must carry the 8-fold symmetry of real orbitals
+      double mx = 0.0;
+      for (int64_t k = 0; k < L4; ++k) mx = std::max(mx, std::fabs(eri[k]));
+      const double tol = 1e-10 * mx;
+      auto at = [&](int64_t p, int64_t q, int64_t r, int64_t s_) { return eri[((p * L + q) * L + r) * L + s_]; };
+      for (int64_t p = 0; p < L; ++p)
+        for (int64_t q = 0; q < L; ++q)
+          for (int64_t r = 0; r < L; ++r)
+            for (int64_t s_ = 0; s_ < L; ++s_) {
+              const double x = at(p, q, r, s_);
+              if (std::fabs(x - at(q, p, r, s_)) > tol || std::fabs(x - at(p, q, s_, r)) > tol ||
+                  std::fabs(x - at(r, s_, p, q)) > tol)
+                return fail(c, SBDG_ERR_ARG, "two-electron integrals lack the 8-fold symmetry (pq|rs) = (qp|rs) = (pq|sr) = (rs|pq)");
+            }
+    }
+    c->built = c->solved = c->have_rdm = c->have_dens = false;
+    if (c->L != L) {
+      c->abp.built = false;
+      auto beyond = [&](const std::vector<uint64_t>& v) {
+        return L < 64 && std::any_of(v.begin(), v.end(), [&](uint64_t x) { return (x >> L) != 0; });
+      };
+      if (beyond(c->a) || beyond(c->b)) c->have_strs = false;  // strings of more orbitals: to be set again
+    }
     c->L = L;
     c->core = core;
+    c->have_ints = false;
     c->h1.assign(h1, h1 + L * L);
-    c->eri.assign(L4, 0.0);
+    c->eri.resize(L4);
     if (layout == 0) {
       std::memcpy(c->eri.data(), eri, sizeof(double) * L4);
-    } else if (layout == 1) {
+    } else {
       // twoInt::store (integrals.h:24-67): slot of (ij|kl) = a(a+1)/2+b, a=max(ij,kl),
       // b=min(ij,kl), ij = max(i,j)(max(i,j)+1)/2 + min(i,j)
       auto pr = [](int64_t i, int64_t j) { return i > j ? i * (i + 1) / 2 + j : j * (j + 1) / 2 + i; };
@@ -988,33 +1020,8 @@ int sbdg_set_integrals(sbdg_ctx* c, int norb, double core, const double* h1, con
               const int64_t aa = std::max(ij, kl), bb = std::min(ij, kl);
               c->eri[(((int64_t)p * L + q) * L + r) * L + s_] = eri[aa * (aa + 1) / 2 + bb];
             }
-    } else {
-      return fail(c, SBDG_ERR_ARG, "eri_layout must be 0 or 1");
-    }
-    for (double x : c->h1)
-      if (!std::isfinite(x)) return fail(c, SBDG_ERR_ARG, "non-finite one-electron integral");
-    for (double x : c->eri)
-      if (!std::isfinite(x)) return fail(c, SBDG_ERR_ARG, "non-finite two-electron integral");
-    if (layout == 0) {
-      // the kernels read (pq|rs) through its images ((ai|bj) for b < j from (ai|jb) in the
-      // alpha-beta kernel): the tensor must carry the 8-fold symmetry of real orbitals
-      double mx = 0.0;
-      for (double x : c->eri) mx = std::max(mx, std::fabs(x));
-      const double tol = 1e-10 * mx;
-      const double* e = c->eri.data();
-      auto at = [&](int64_t p, int64_t q, int64_t r, int64_t s_) { return e[((p * L + q) * L + r) * L + s_]; };
-      for (int64_t p = 0; p < L; ++p)
-        for (int64_t q = 0; q < L; ++q)
-          for (int64_t r = 0; r < L; ++r)
-            for (int64_t s_ = 0; s_ < L; ++s_) {
-              const double x = at(p, q, r, s_);
-              if (std::fabs(x - at(q, p, r, s_)) > tol || std::fabs(x - at(p, q, s_, r)) > tol ||
-                  std::fabs(x - at(r, s_, p, q)) > tol)
-                return fail(c, SBDG_ERR_ARG, "two-electron integrals lack the 8-fold symmetry (pq|rs) = (qp|rs) = (pq|sr) = (rs|pq)");
-            }
     }
     c->have_ints = true;
-    c->built = c->solved = c->have_rdm = c->have_dens = false;
     return SBDG_OK;
   });
 }

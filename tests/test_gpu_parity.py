@@ -638,3 +638,33 @@ def test_errors_from_the_host():
     s = solver(case, max_it=50, max_nb=8, eps=1e-12, max_time=1e-9)
     s.run()
     assert s.stats()["iterations"] == 1 and s.stats()["converged"] == 0
+
+
+def test_refused_integrals_leave_the_context_and_smaller_norb_drops_the_strings():
+    """set_integrals checks before it changes anything: after a refused call with another norb the
+    context computes as before.  Integrals of fewer orbitals than the strings use are taken, and
+    then the strings have to be set again."""
+    case = workload_small(12, 4, 4, 50, 40, 103)
+    s = solver(case)
+    x = np.random.default_rng(3).normal(size=s.ndet)
+    want = s.sigma(x)
+    for norb, bad in ((8, "nan"), (8, "symmetry"), (64, "inf")):
+        h1, eri = syn.synthetic_integrals(norb, np.random.default_rng(4))
+        if bad == "symmetry":
+            eri[0, 1, 2, 3] += 1.0
+        else:
+            (h1 if bad == "inf" else eri)[(1,) * (2 if bad == "inf" else 4)] = float(bad)
+        rc = sbdg.lib().sbdg_set_integrals(s._c, norb, 0.0, sbdg._d(h1), sbdg._d(eri), 0)
+        assert rc == sbdg.ERR_ARG
+        assert np.array_equal(s.sigma(x), want)
+        s.set_options(doubles=2)  # the tables are made again, of the integrals that were taken
+        assert np.abs(s.sigma(x) - want).max() <= 1e-12 * np.abs(want).max()
+        s.set_options(doubles=0)
+    h1, eri = syn.synthetic_integrals(6, np.random.default_rng(5))
+    assert sbdg.lib().sbdg_set_integrals(s._c, 6, 0.0, sbdg._d(h1), sbdg._d(eri), 0) == sbdg.OK
+    with pytest.raises(sbdg.SbdgError) as ei:
+        s.build()
+    assert ei.value.code == sbdg.ERR_STATE
+    s.set_integrals(case["core"], case["h1"], case["eri"])
+    assert np.array_equal(s.sigma(x), want)
+    s.close()
