@@ -104,7 +104,8 @@ int sbdg_default_options(sbdg_options *opt);
  * h1: L*L row-major; eri_layout 0: full (pq|rs) row-major L^4, 8-fold symmetric
  * ((pq|rs) = (qp|rs) = (pq|sr) = (rs|pq) within 1e-10 of the largest element, else
  * SBDG_ERR_ARG); eri_layout 1: the reference's packed store twoInt::store
- * (integrals.h:24-67), symmetric by construction. */
+ * (integrals.h:24-67), symmetric by construction.  A refused call leaves the context as it
+ * was.  Strings stay set, unless they use orbitals beyond a smaller norb. */
 int sbdg_set_integrals(sbdg_ctx *ctx, int norb, double core, const double *h1, const double *eri,
                        int eri_layout);
 
